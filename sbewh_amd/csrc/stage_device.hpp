@@ -118,12 +118,12 @@ __device__ __forceinline__ void wsync() { __syncthreads(); }
 
 // coalesced copy of the wave's KPW matrices (n x n at src + k*stride + off,
 // complex) into LDS natural layout [kk][N][N], zero padded.
-template <int N, int LR, class Lay = SwLay<N>>
+template <int N, int LR, class Lay = SwLay<N>, int CHUNK = Lay::CHUNK>
 __device__ __forceinline__ void load_mats(cd *lds, const double *src, long stride, long off, int n, long nk, long blk)
 {
     using G = Geo<N, LR>;
     constexpr int IT = G::KPW * G::NN / 64;  // entries per lane
-    constexpr int CH = N >= 16 ? 4 : (Lay::CHUNK < IT ? Lay::CHUNK : IT);     // entries whose loads are in flight together
+    constexpr int CH = N >= 16 ? 4 : (CHUNK < IT ? CHUNK : IT);     // entries whose loads are in flight together
     const double2 *s2 = reinterpret_cast<const double2 *>(src);
     // unconditional loads (masked entries read entry `off` of k-point 0)
     for_chunks<IT, CH>([&](auto i0c) {
@@ -148,14 +148,151 @@ __device__ __forceinline__ void load_mats(cd *lds, const double *src, long strid
     });
 }
 
+// loads through the constant address space: with a wave-uniform address they
+// are scalar loads.  Only for memory that no kernel of the same launch writes.
+typedef double sd2 __attribute__((ext_vector_type(2)));
+typedef int si2 __attribute__((ext_vector_type(2)));
+template <class V>
+__device__ __forceinline__ V load_const(const void *p, unsigned i)
+{
+    typedef const __attribute__((address_space(4))) char *cptr;
+    typedef const __attribute__((address_space(4))) V *vptr;
+    return *(vptr)((cptr)(unsigned long long)p + (unsigned)(i * sizeof(V)));
+}
+
+// H(k) of operator op for layouts whose matrices fill whole wavefronts, into
+// registers: acc[kk N^2 / 64 + u] is entry threadIdx.x + 64 u (row-major, N x N) of k-point kk
+// (N >= 8: register u of a lane belongs to k-point kk = 64 u / N^2 for all 64
+// lanes): everything that depends on the k-point alone is wave-uniform, so the
+// phase map and the twiddles come through scalar loads, and a phase-sum row is
+// loaded once for all k-points of the wavefront that share it, QG cells in one
+// memory trip.  Consecutive k-points share rest(k) along a Fourier block's last
+// axis, so a wavefront has one or two distinct rows; each gets a pass.
+// false, with nothing done, for an R box wider than 16 cells along the last
+// axis.  Sums in the order of phase_mats.
+// Why: one wave-uniform branch and one memory trip per cell and pair of entries
+// (104 in series for 8 bands and 13 cells) kept the 8-band kernel waiting; four
+// right-hand sides on 150 x 150 k, 8 bands: 362 -> 316 us, an integration there
+// 64.3 -> 54.3 ms; 48^3 k, 16 bands: 6.86 -> 6.66 ms.
+template <int N, int LR>
+__device__ __forceinline__ bool phase_rows(cd *acc, const StageArgs &a, int op, long blk)
+{
+    using G = Geo<N, LR>;
+    static_assert(G::NN % 64 == 0, "a k-point's matrix fills whole wavefronts");
+    constexpr int EK = G::NN / 64;                 // entries per lane and k-point
+    constexpr int KPW = G::KPW, KT = KPW < 4 ? KPW : 4;
+    constexpr int QG = EK == 1 ? 4 : 2;            // cells per memory trip
+    const int n = a.n, nn = n * n, M = 2 * nn, WL = a.ph.WL;
+    if (WL > 16) return false;
+    const int blkl = __builtin_amdgcn_readfirstlane((int)blk);
+    const double2 *Yb = reinterpret_cast<const double2 *>(a.ph.Y) + op * nn;
+    int rest[KPW];
+    unsigned tp[KPW];
+#pragma unroll
+    for (int kk = 0; kk < KPW; kk++) {
+        const long k = (long)blkl * KPW + kk;
+        const si2 ph = load_const<si2>(a.ph.kphase, (unsigned)(k < a.nk ? k : 0));
+        rest[kk] = ph.x;
+        tp[kk] = ph.y;
+    }
+    // the lane's entries of a row: masked ones read entry 0 and are zeroed at the end
+    int ent[EK];
+    bool krc[EK];
+#pragma unroll
+    for (int u = 0; u < EK; u++) {
+        const int idx = threadIdx.x + 64 * u, r = idx / N, c = idx % N;
+        krc[u] = r < n && c < n;
+        ent[u] = krc[u] ? r * n + c : 0;
+    }
+#pragma unroll
+    for (int kk = 0; kk < KPW; kk++)
+#pragma unroll
+        for (int u = 0; u < EK; u++) acc[kk * EK + u] = mk(0, 0);
+    unsigned todo = KPW >= 32 ? ~0u : (1u << KPW) - 1;
+    while (todo) {
+        // the first k-point left, and those that share its row
+        int row = 0;
+#pragma unroll
+        for (int kk = KPW - 1; kk >= 0; kk--) row = (todo >> kk) & 1 ? rest[kk] : row;
+        unsigned mine = 0;
+#pragma unroll
+        for (int kk = 0; kk < KPW; kk++) mine |= (rest[kk] == row ? 1u : 0u) << kk;
+        mine &= todo;
+        todo &= ~mine;
+        const double2 *yr = Yb + (long)row * M;
+        // cell q of the row (entries y) into the sums of its k-points
+        auto add_cell = [&](int q, const double2 *y) {
+#pragma unroll
+            for (int k4 = 0; k4 < KPW; k4 += KT) {
+                sd2 tw[KT];
+#pragma unroll
+                for (int v = 0; v < KT; v++) tw[v] = load_const<sd2>(a.ph.twL, tp[k4 + v] + q);
+#pragma unroll
+                for (int v = 0; v < KT; v++)
+                    if (KPW == 1 || ((mine >> (k4 + v)) & 1)) {
+                        asm volatile("");  // a branch over the products, not selects behind them
+#pragma unroll
+                        for (int u = 0; u < EK; u++)
+                            acc[(k4 + v) * EK + u] = cfma(mk(tw[v].x, tw[v].y), mk(y[u].x, y[u].y), acc[(k4 + v) * EK + u]);
+                    }
+            }
+        };
+        int q = 0;
+        for (; q + QG <= WL; q += QG) {
+            double2 y[QG][EK];
+#pragma unroll
+            for (int t = 0; t < QG; t++)
+#pragma unroll
+                for (int u = 0; u < EK; u++) y[t][u] = yr[(long)(q + t) * M + ent[u]];
+#pragma unroll
+            for (int t = 0; t < QG; t++) add_cell(q + t, y[t]);
+        }
+        for (; q < WL; q++) {
+            double2 y[EK];
+#pragma unroll
+            for (int u = 0; u < EK; u++) y[u] = yr[(long)q * M + ent[u]];
+            add_cell(q, y);
+        }
+    }
+#pragma unroll
+    for (int kk = 0; kk < KPW; kk++) {
+        const bool kin = (long)blkl * KPW + kk < a.nk;
+#pragma unroll
+        for (int u = 0; u < EK; u++)
+            if (!(kin && krc[u])) acc[kk * EK + u] = mk(0, 0);
+    }
+    return true;
+}
+
+// the same into LDS
+template <int N, int LR, class Lay = SwLay<N>>
+__device__ __forceinline__ bool phase_mats_rows(cd *lds, const StageArgs &a, int op, long blk)
+{
+    using G = Geo<N, LR>;
+    constexpr int EK = G::NN / 64;
+    cd acc[G::KPW * EK];
+    if (!phase_rows<N, LR>(acc, a, op, blk)) return false;
+#pragma unroll
+    for (int kk = 0; kk < G::KPW; kk++)
+#pragma unroll
+        for (int u = 0; u < EK; u++) {
+            const int idx = threadIdx.x + 64 * u;
+            lds[kk * Lay::MS + Lay::at(idx / N, idx % N)] = acc[kk * EK + u];
+        }
+    return true;
+}
+
 // H(k) of operator op (0: H0, 1: H_E) for the wave's k-points into LDS
 // natural layout: the last phase-sum contraction
 //   H(k)[a][b] = sum_r tw_L[i_L(k)][r] Y[rest(k)][r][op][a][b]
 // (the k-points of a wave share rest(k), so the Y rows are L1/L2 hits).
-template <int N, int LR, class Lay = SwLay<N>>
+template <int N, int LR, class Lay = SwLay<N>, bool UNI = false>
 __device__ __forceinline__ void phase_mats(cd *lds, const StageArgs &a, int op, long blk)
 {
     using G = Geo<N, LR>;
+    if constexpr (UNI && N >= 8) {
+        if (phase_mats_rows<N, LR, Lay>(lds, a, op, blk)) return;
+    }
     constexpr int IT = G::KPW * G::NN / 64;  // entries per lane
     constexpr int WQ = 16;                   // largest R extent of the last axis
     const int n = a.n, nn = n * n, M = 2 * nn, WL = a.ph.WL;
@@ -401,7 +538,7 @@ __device__ __forceinline__ void load_rho_nt(cd *lds, const StageArgs &a, long bl
 template <int N, int LR, class Lay = SwLay<N>>
 __device__ __forceinline__ void load_rho(cd *lds, const StageArgs &a, long blk)
 {
-    if constexpr (N <= 4) {
+    if constexpr (N <= 4 || LR == 1) {
         switch (a.in.nt) {
         case 0: load_rho_nt<N, LR, Lay, 0>(lds, a, blk); return;
         case 1: load_rho_nt<N, LR, Lay, 1>(lds, a, blk); return;
@@ -880,6 +1017,19 @@ __device__ __forceinline__ void store_ucache(const StageArgs &a, const cd *lds, 
     }
 }
 
+// the error terms of the special slots (block 0; d/dt of A_t is -E_t for
+// t < dim, the rest 0)
+__device__ __forceinline__ double stage_err_specials(const StageArgs &a, long blk)
+{
+    if (blk != 0 || threadIdx.x >= 8) return 0;
+    const int t = threadIdx.x;
+    double2 kv[6];
+#pragma unroll
+    for (int j = 0; j < 5; j++) kv[j] = reinterpret_cast<const double2 *>(a.in.k[j])[t];
+    kv[5] = make_double2(t < a.dim ? -a.E[t] : 0.0, 0.0);
+    return err_entry(reinterpret_cast<const double2 *>(a.in.x)[t], kv, a.err_e, a.err_ea, a.err_er, a.err_dt);
+}
+
 // Error norm of the attempt over this block's k-points (last stage only): the
 // stage input's x, k1, k3..k6 are read again (HBM that the VALU-bound kernel
 // leaves idle), k7 = d rho/dt comes from LDS natural layout; same lane ->
@@ -908,16 +1058,7 @@ __device__ __forceinline__ double stage_err(const StageArgs &a, const cd *lds, l
             v = fmax(v, err_entry(x2[i], kv, a.err_e, a.err_ea, a.err_er, a.err_dt));
         }
     }
-    if (blk == 0 && threadIdx.x < 8) {
-        // special slots: d/dt of A_t is -E_t (t < dim), the rest 0
-        const int t = threadIdx.x;
-        double2 kv[6];
-#pragma unroll
-        for (int j = 0; j < 5; j++) kv[j] = reinterpret_cast<const double2 *>(a.in.k[j])[t];
-        kv[5] = make_double2(t < a.dim ? -a.E[t] : 0.0, 0.0);
-        v = fmax(v, err_entry(x2[t], kv, a.err_e, a.err_ea, a.err_er, a.err_dt));
-    }
-    return v;
+    return fmax(v, stage_err_specials(a, blk));
 }
 
 // special slots of the stage: d A_t/dt = -E_t (t < dim), and the stage input
@@ -971,7 +1112,7 @@ __device__ __forceinline__ void rhs_stage_body16(const StageArgs &a, const long 
         if (a.warm) {
             // warm start: A = U' (H0 U'^dagger) with U' the previous eigenvectors
             load_mats<N, LR>(S0, a.ucache, nn, 0, n, a.nk, blk);
-            phase_mats<N, LR>(S1, a, 0, blk);  // H_0 -> S1
+            phase_mats<N, LR, SwLay<N>, true>(S1, a, 0, blk);  // H_0 -> S1
             wsync();
             load_u<N, LR>(s0, L, U);
             u_pad_identity<N, LR>(L, n, U);
@@ -994,7 +1135,7 @@ __device__ __forceinline__ void rhs_stage_body16(const StageArgs &a, const long 
             load_xrow<N, LR>(s0, L, A);
             wave_jacobi<N, LR>(A, U, L, a.sweeps, Dg, Ja, Jb, Fa, false);
         } else {
-            phase_mats<N, LR>(S1, a, 0, blk);  // H_0 -> S1
+            phase_mats<N, LR, SwLay<N>, true>(S1, a, 0, blk);  // H_0 -> S1
             wsync();
             load_xrow<N, LR>(s1, L, A);
             wave_jacobi<N, LR>(A, U, L, a.sweeps, Dg, Ja, Jb, Fa);
@@ -1052,7 +1193,7 @@ __device__ __forceinline__ void rhs_stage_body16(const StageArgs &a, const long 
         }
         wsync();
     }
-    phase_mats<N, LR>(S1, a, 1, blk);  // H_E -> S1
+    phase_mats<N, LR, SwLay<N>, true>(S1, a, 1, blk);  // H_E -> S1
     wsync();
     // coherent part -i (H_E rho - rho H_E): D + (-i) X = D + (X.i, -X.r), so
     // it is accumulated as i (rho H_E - H_E rho) with the roles of the real and
@@ -1163,30 +1304,29 @@ __device__ __forceinline__ void rhs_stage_body_r1(const StageArgs &a, const long
     bool he_ready = false;
     auto form_h0 = [&]() {  // H0 -> S
         if constexpr (N <= 4 && PAIR) he_ready = phase_mats_pair<N, 1, Lay>(S, a, blk, he);
-        if (!he_ready) phase_mats<N, 1, Lay>(S, a, 0, blk);
+        if (!he_ready) phase_mats<N, 1, Lay, PAIR>(S, a, 0, blk);
     };
     if (a.dephase) {
         cd A[C];
         if (a.warm) {
             // warm start: A = U' H0 U'^dagger with U' the previous eigenvectors
-            load_mats<N, 1, Lay>(S, a.ucache, nn, 0, n, a.nk, blk);  // U' -> S
+            load_mats<N, 1, Lay, N>(S, a.ucache, nn, 0, n, a.nk, blk);  // U' -> S
             wsync();
             cd T[C];
             slot_load_rows<N>(s, L.i, T);
-            slot_load_cols<N>(s, L.i, U);
             // padded rows and columns of U' are the identity
             u_pad_identity<N, 1>(L, n, T);
-            u_pad_identity<N, 1>(L, n, U);
             wsync();
             form_h0();
             wsync();
             reg_product<N, 0, 0>(T, s, L.i, A);  // U' H0
             wsync();
-            slot_store_cols<N>(s, L.i, U);  // U' -> S
+            slot_store_rows<N>(s, L.i, T);  // U' -> S
             wsync();
 #pragma unroll
             for (int c = 0; c < C; c++) T[c] = A[c];
             reg_product<N, 0, 1>(T, s, L.i, A);  // (U' H0) U'^dagger
+            slot_load_cols<N>(s, L.i, U);
             wave_jacobi<N, 1>(A, U, L, a.sweeps, Dg, Ja, Jb, Fa, false);
         } else {
             form_h0();
@@ -1215,7 +1355,7 @@ __device__ __forceinline__ void rhs_stage_body_r1(const StageArgs &a, const long
         slot_load_rows<N>(s, L.i, rr);
         wsync();
         if (he_ready) store_entries<N, 1, Lay>(S, he);  // H_E -> S
-        else phase_mats<N, 1, Lay>(S, a, 1, blk);
+        else phase_mats<N, 1, Lay, PAIR>(S, a, 1, blk);
         wsync();
         reg_product<N, 0, 0>(rr, s, L.i, T);  // rho H_E
         wsync();
@@ -1319,7 +1459,7 @@ __device__ __forceinline__ void rhs_stage_body(const StageArgs &a, const long bl
     bool he_ready = false;
     auto form_h0 = [&]() {  // H_0 -> S1
         if constexpr (N <= 4 && PAIR) he_ready = phase_mats_pair<N, LR>(S1, a, blk, he);
-        if (!he_ready) phase_mats<N, LR>(S1, a, 0, blk);
+        if (!he_ready) phase_mats<N, LR, SwLay<N>, PAIR>(S1, a, 0, blk);
     };
     if (a.dephase) {
         cd A[C];
@@ -1355,7 +1495,7 @@ __device__ __forceinline__ void rhs_stage_body(const StageArgs &a, const long bl
     if (a.xout) store_state<N, LR>(a.xout, S0, n, a.P, a.nk, blk);
     // coherent part: -i (H_E rho - rho H_E)
     if (he_ready) store_entries<N, LR>(S1, he);  // H_E -> S1
-    else phase_mats<N, LR>(S1, a, 1, blk);
+    else phase_mats<N, LR, SwLay<N>, PAIR>(S1, a, 1, blk);
     wsync();
     {
         cd t1[C];
@@ -1414,13 +1554,14 @@ __device__ __forceinline__ void rhs_stage_body(const StageArgs &a, const long bl
     }
 }
 
-// minimum waves per SIMD the register allocation must allow: the 16-band
+// minimum waves per SIMD the register allocation must allow: the 8-band kernel
+// at one lane per row fits three (at most 168 VGPRs); the 16-band
 // kernel at 4 lanes per row fits four (at most 128 VGPRs; 8.9 KB of LDS per
 // wavefront) when the allocator is told so, instead of two with part of the
 // matrix-core operands in AGPRs; at 2 lanes per row a bound would only buy
 // spills to scratch
 template <int N, int LR>
-constexpr int stage_min_waves() { return (N == 16 && LR == 4) ? 4 : 1; }
+constexpr int stage_min_waves() { return (N == 16 && LR == 4) ? 4 : (N == 8 && LR == 1) ? 3 : 1; }
 
 template <int N, int LR>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(stage_min_waves<N, LR>())))

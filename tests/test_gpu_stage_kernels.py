@@ -1,0 +1,89 @@
+"""The stage kernel at the edges of its phase-sum path,
+against the CPU oracle.  Tolerance: 1e-12 relative, as for every single
+kernel (FP64, sums of at most a few hundred products of order one)."""
+import numpy as np
+import pytest
+
+from sbewh_amd import model
+from sbewh_amd.propagator import SBEContext
+from oracle.oracle_py import Oracle
+from tests import cases
+
+pytestmark = pytest.mark.gpu
+
+
+def small_model(n, ext, seed, copies=1):
+    """Gaussian blocks on the box |R_d| <= ext[d]; copies > 1: every band
+    `copies`-fold degenerate at every k (h x 1)"""
+    rng = np.random.default_rng(seed)
+    m = n // copies
+    cells = np.array([(a, b, 0) for a in range(-ext[0], ext[0] + 1) for b in range(-ext[1], ext[1] + 1)], np.int32)
+    H = np.zeros((len(cells), n, n), complex)
+    D = np.zeros((len(cells), 3, n, n), complex)
+    one = np.eye(copies)
+    for i, c in enumerate(cells.tolist()):
+        j = len(cells) - 1 - i
+        if j < i:
+            continue
+        f = np.exp(-np.hypot(*c[:2]))
+        h = f * 0.1 * (rng.normal(size=(m, m)) + 1j * rng.normal(size=(m, m)))
+        r = f * (rng.normal(size=(2, n, n)) + 1j * rng.normal(size=(2, n, n)))
+        if i == j:
+            h = h + h.conj().T + np.diag(np.linspace(-0.4, 0.4, m))
+            r = r + np.conj(np.swapaxes(r, 1, 2))
+        H[i], H[j] = np.kron(h, one), np.kron(h, one).conj().T
+        D[i, :2], D[j, :2] = r, np.conj(np.swapaxes(r, 1, 2))
+    return model.TBModel(cells, H, D, np.eye(3) * 6.0)
+
+
+def config(n, ext, Nk, Nf, seed=5, copies=1, **kw):
+    pul = model.elliptic_sin2(1.0, 0.4, 3000.0, 4.0)
+    kw = {"sweeps": 12, "T2_fs": 1.0, **kw}
+    return model.Config("edge", small_model(n, ext, seed, copies), 2, (*Nk, 1), (*Nf, 1), pul, **kw)
+
+
+def states(o, count, steps):
+    """states of the same rho with the vector potential moved by `steps`"""
+    x = cases.perturbed_state(o.initial_state(0.0), o.n, o.P, o.num_k, seed=3, amp=0.05)
+    out, A = [], 0.3
+    for q in range(count):
+        s = x.copy()
+        A += steps[q]
+        s[0], s[1] = A, -0.4 * A
+        out.append(s)
+    return out
+
+
+def check_sequence(cfg, steps, ctx=None):
+    g, o = ctx or SBEContext(cfg), Oracle(cfg)
+    for q, x in enumerate(states(o, len(steps), steps)):
+        t = 3.0 + 0.1 * q
+        a, b = g.rhs(x, t), o.rhs(x, t)
+        err = np.abs(a - b).max() / np.abs(b).max()
+        print(f"[gpu] n={cfg.model.num_wann} step {steps[q]:g}: {err:.1e}", flush=True)
+        assert err < 1e-12
+    o.close()
+
+
+# (bands, lanes per row, R extents, k-grid, Fourier block): wavefronts whose
+# k-points lie in one, two and more rows of the phase sum, a last wavefront
+# that is not full, R extents below, at and beyond one memory trip and the
+# 16-cell limit, padded bands
+@pytest.mark.parametrize("n,lr,ext,Nk,Nf", [
+    (8, 1, (1, 0), (6, 1), (3, 1)),
+    (8, 1, (1, 1), (6, 9), (3, 3)),
+    (8, 1, (1, 2), (5, 10), (5, 5)),
+    (8, 1, (2, 7), (5, 15), (5, 15)),
+    (8, 1, (1, 8), (3, 18), (3, 18)),
+    (5, 1, (1, 3), (4, 8), (4, 8)),
+    (8, 2, (1, 2), (5, 15), (5, 5)),
+    (8, 4, (1, 4), (5, 9), (5, 9)),
+    (7, 4, (1, 1), (6, 3), (3, 3)),
+    (16, 2, (1, 3), (3, 8), (3, 8)),
+    (16, 4, (1, 4), (3, 9), (3, 9)),
+    (16, 4, (1, 8), (3, 18), (3, 18)),
+    (11, 4, (1, 0), (6, 1), (3, 1)),
+])
+def test_phase_rows(n, lr, ext, Nk, Nf, monkeypatch):
+    monkeypatch.setenv("SBEWH_STAGE_LR", str(lr))
+    check_sequence(config(n, ext, Nk, Nf), [0.0, 0.01])
