@@ -1084,8 +1084,8 @@ __device__ __forceinline__ void stage_specials(const StageArgs &a, const long bl
     }
 }
 
-// The stage for 16-band layouts: the Jacobi in the XOR-wrapped register
-// layout, every matrix product on the matrix cores, one k-point of the block
+// The stage for 16 bands at two lanes per row: the Jacobi in the XOR-wrapped
+// register layout, every matrix product on the matrix cores, one k-point of the block
 // at a time with all 64 lanes.  A product's result stays in its accumulator
 // and feeds the next product as an operand (acc_right, acc_left_dagger), so
 // two LDS matrices per k-point suffice (8.9 KB for one k-point per block:
@@ -1217,6 +1217,425 @@ __device__ __forceinline__ void rhs_stage_body16(const StageArgs &a, const long 
     store_state<N, LR>(a.dxdt, S0, n, a.P, a.nk, blk);
     if (a.err_partial) {
         const double v = seg_max<64>(stage_err<N, LR>(a, S0, blk));
+        if (threadIdx.x == 0) a.err_partial[blk] = v;
+    }
+}
+
+// ---- 16 bands, four lanes per row: the decomposition refined by products ----
+// Every matrix lives in the accumulator layout (lane l, register j: row
+// 4 j + l / 16, column l % 16), which is also the layout in which a k-point's
+// matrices are loaded and stored contiguously and in which the phase sum leaves
+// H.  acc_right and acc_left_dagger hand a matrix M to a product as right operand
+// M or left operand M^dagger, so a chain of products needs LDS only where a
+// matrix changes from M to M^dagger.
+//
+// This kernel is bound by instruction issue: a v_mfma_f64_16x16x4f64 holds the
+// SIMD for 64 cycles and a vector instruction for 4, and the two do not overlap
+// between the waves of a SIMD (measured: FP64 FMAs, integer operations and MFMAs
+// of different waves take the sum of their times).  A complex product costs
+// 1024 cycles, a Jacobi sweep about 9400 (half of it exchanges, selects and
+// addresses), so warm starts are refined by products: see refine16.
+// Entry (i, j) of a matrix in LDS at 17 i + j: a lane's accumulator entries are
+// one address and constant offsets, and so are those of the transpose; rows and
+// columns walk distinct banks.
+constexpr int ACC_RS = 17, ACC_MS = 16 * ACC_RS;
+struct AccPos {
+    int nat, tr;
+};
+__device__ __forceinline__ AccPos acc_pos()
+{
+    const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
+    return AccPos{q * ACC_RS + r, r * ACC_RS + q};
+}
+__device__ __forceinline__ void acc_put(cd *buf, const AccPos &p, const CAcc &m)
+{
+#pragma unroll
+    for (int j = 0; j < 4; j++) buf[p.nat + 4 * ACC_RS * j] = mk(m.r[j], m.i[j]);
+}
+__device__ __forceinline__ void acc_get(const cd *buf, const AccPos &p, CAcc &m)
+{
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const cd v = buf[p.nat + 4 * ACC_RS * j];
+        m.r[j] = v.x;
+        m.i[j] = v.y;
+    }
+}
+// the adjoint of the matrix in buf
+__device__ __forceinline__ void acc_get_dagger(const cd *buf, const AccPos &p, CAcc &m)
+{
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const cd v = buf[p.tr + 4 * j];
+        m.r[j] = v.x;
+        m.i[j] = -v.y;
+    }
+}
+// M -> M^dagger through the LDS buffer (free on entry and on exit)
+__device__ __forceinline__ void acc_dagger(cd *buf, const AccPos &p, const CAcc &m, CAcc &out)
+{
+    acc_put(buf, p, m);
+    wsync();
+    acc_get_dagger(buf, p, out);
+    wsync();
+}
+
+// acc += A B with A = M^dagger from an accumulator M
+__device__ __forceinline__ void mul_dagger(const CAcc &m, const CAcc &b, CAcc &acc)
+{
+    cd x[4], y[4];
+    acc_left_dagger(m, x);
+    acc_right(b, y);
+    mfma_cmul(x, y, acc);
+}
+
+// 1/x for a normal x: hardware estimate and one Newton step
+__device__ __forceinline__ double rcp_newton(double x)
+{
+    const double y = __builtin_amdgcn_rcp(x);
+    return fma(fma(-x, y, 1.0), y, y);
+}
+
+// Warm start of one k-point's decomposition: U (rows, unitary to rounding)
+// nearly diagonalises H0.  With Q = U^dagger, S = Q^dagger H0 Q and R = 1 - Q^dagger Q
+// (zero in the first pass), an iteration orthonormalises and diagonalises to
+// second order:
+//   lam_i = S_ii / (1 - R_ii),  E = S + (lam R + R lam) / 2 off the diagonal,
+//   X1 = E_ij / (lam_i - lam_j),  C = (X1 + R) E + h.c.,  X = X1 + C_ij / 2 (lam_i - lam_j),
+//   U <- (1 + X + R/2 + X (X + R) / 2) U,
+// which leaves O(x^3) of x = max |X1| off the diagonal and O(x^4) of
+// non-orthonormality, both seen by the next iteration (the quadratic
+// iteration of Ogita and Aishima with its second-order terms; below X2 these are
+// under rounding and left out).  Elements at most thr, the Jacobi threshold,
+// count as zero.  Nothing is iterated after a step with x <= XF: x^3 is below
+// rounding there.  A k-point with x > XB (a near crossing of bands) is left to
+// the Jacobi rotations: the result is false.
+// Typically 3e-3 <= x <= 1e-2 between stages: two iterations, 9 products.
+// Measured against the Jacobi rotations from the same warm start (three waves
+// per SIMD at 146 VGPRs; at 128 VGPRs the spills cost more than the fourth wave
+// gives): four right-hand sides on 48^3 k, 16 bands 6.66 -> 4.88 ms, 63 x 63 k,
+// 11 bands 295 -> 212 us, an integration on 24^3 k 121.4 -> 100.7 ms; per
+// wavefront 242 MFMAs and 1730 vector instructions, formerly 123 and 7300.
+__device__ __forceinline__ bool refine16(cd *buf, const cd *H0, const AccPos &pos, CAcc &U, CAcc &Q, double *Dg,
+                                         int sweeps)
+{
+    constexpr double XB = 0.1, XF = 4e-6, X2 = 1e-8, RF = 1e-14;
+    const int c = cacc_col();
+    double thr2 = 0;
+    for (int it = 0;; it++) {
+        CAcc t, R;
+        {
+            CAcc h;
+            acc_get(H0, pos, h);
+            cacc_zero(t);
+            mul_dagger(h, Q, t);  // H0 Q
+        }
+        CAcc S;
+        cacc_zero(S);
+        mul_dagger(Q, t, S);  // Q^dagger H0 Q
+        cacc_zero(R);
+        if (it > 0) {
+            cd x[4], y[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                R.r[j] = cacc_row(j) == c ? 1.0 : 0.0;
+                x[j] = mk(-Q.r[j], Q.i[j]);
+            }
+            acc_right(Q, y);
+            mfma_cmul(x, y, R);  // 1 - Q^dagger Q
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (cacc_row(j) == c) Dg[c] = S.r[j] / (1.0 - R.r[j]);
+        if (it == 0) {
+            double s = 0;
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (cacc_row(j) <= c) s += fabs(S.r[j]) + fabs(S.i[j]);
+            s = seg_sum<64>(s);
+            const double thr = 1e-15 * (0.5 * s);
+            thr2 = thr * thr;
+        }
+        wsync();
+        const double lc = Dg[c];
+        CAcc E, X;
+        double rd[4], x2 = 0, r2 = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const double lr = Dg[cacc_row(j)];
+            const bool off = cacc_row(j) != c;
+            const double hs = 0.5 * (lr + lc);
+            E.r[j] = off ? fma(hs, R.r[j], S.r[j]) : 0.0;
+            E.i[j] = off ? fma(hs, R.i[j], S.i[j]) : 0.0;
+            const bool keep = off && fma(E.r[j], E.r[j], E.i[j] * E.i[j]) > thr2;
+            const double d = lr - lc;
+            // equal eigenvalues with an element above the threshold: a
+            // quotient beyond every bound, left to the rotations
+            rd[j] = d != 0.0 ? rcp_newton(d) : 1e30;
+            X.r[j] = keep ? E.r[j] * rd[j] : 0.0;
+            X.i[j] = keep ? E.i[j] * rd[j] : 0.0;
+            x2 = fmax(x2, fma(X.r[j], X.r[j], X.i[j] * X.i[j]));
+            r2 = fmax(r2, fma(R.r[j], R.r[j], R.i[j] * R.i[j]));
+        }
+        const bool rot = __any(x2 > 0.0), fix = __any(r2 > RF * RF);
+        if ((!rot && !fix) || sweeps <= 0) return true;
+        bool bad = __any(x2 > XB * XB);
+        const bool second = __any(x2 > X2 * X2);
+        CAcc V;  // the adjoint of the update: 1 - X + R/2 + (X - R) X / 2
+        cacc_zero(V);
+        if (second && !bad) {
+            cd x[4], y[4];
+            CAcc W;
+            cacc_zero(W);
+#pragma unroll
+            for (int j = 0; j < 4; j++) x[j] = mk(R.r[j] - X.r[j], X.i[j] - R.i[j]);  // X1 + R
+            acc_right(E, y);
+            mfma_cmul(x, y, W);
+            CAcc Wd;
+            acc_dagger(buf, pos, W, Wd);
+            double c2 = 0;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const double cr = 0.5 * (W.r[j] + Wd.r[j]), ci = 0.5 * (W.i[j] + Wd.i[j]);
+                const bool off = cacc_row(j) != c;
+                if (!off) Dg[c] += cr;
+                const bool keep = off && 4 * fma(cr, cr, ci * ci) > thr2;
+                const double xr = keep ? cr * rd[j] : 0.0, xi = keep ? ci * rd[j] : 0.0;
+                c2 = fmax(c2, fma(xr, xr, xi * xi));
+                X.r[j] += xr;
+                X.i[j] += xi;
+            }
+            bad = __any(c2 > XB * XB);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                // left (X - R) / 2 = (-(X + R) / 2)^dagger
+                x[j] = mk(-0.5 * (X.r[j] + R.r[j]), 0.5 * (X.i[j] + R.i[j]));
+                y[j] = mk(X.r[j], X.i[j]);
+            }
+            mfma_cmul(x, y, V);
+        }
+        if (bad) {
+            wsync();
+            return false;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            V.r[j] += fma(0.5, R.r[j], (cacc_row(j) == c ? 1.0 : 0.0) - X.r[j]);
+            V.i[j] += fma(0.5, R.i[j], -X.i[j]);
+        }
+        cacc_zero(t);
+        mul_dagger(V, U, t);
+        U = t;
+        acc_dagger(buf, pos, U, Q);
+        if (!__any(x2 > XF * XF) || it + 1 >= sweeps) return true;
+    }
+}
+
+__device__ __forceinline__ void rhs_stage_body16q(const StageArgs &a, const long blk)
+{
+    constexpr int N = 16, LR = 4;
+    using G = Geo<N, LR>;
+    constexpr int C = G::C;
+    __shared__ cd S0[ACC_MS];  // transposes, operands
+    __shared__ cd S1[ACC_MS];  // H0, then rho
+    __shared__ double Dg[N];
+    __shared__ cd Ja[N], Jb[N];
+    __shared__ int Fa[N];
+
+    const AccPos pos = acc_pos();
+    const int n = a.n, nn = n * n, col = cacc_col();
+    // one k-point per block: its index and the addresses of its matrices are wave-uniform
+    const long k = __builtin_amdgcn_readfirstlane((int)blk), kst = 8 + k * a.P;
+    if (k >= a.nk) return;
+    stage_specials(a, blk);
+    bool own[4];  // the lane's registers that are entries of the n x n matrix
+    int ent[4];   // and their index in it
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        own[j] = cacc_row(j) < n && col < n;
+        ent[j] = own[j] ? cacc_row(j) * n + col : 0;
+    }
+    auto load = [&](const double *src, int j) { return reinterpret_cast<const double2 *>(src)[ent[j]]; };
+    auto phase_acc = [&](int op, CAcc &h) {
+        cd v[4];
+        if (!phase_rows<N, LR>(v, a, op, blk)) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = own[j] ? phase_last(a.ph, k, 2 * nn, op * nn + ent[j]) : mk(0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            h.r[j] = v[j].x;
+            h.i[j] = v[j].y;
+        }
+    };
+
+    CAcc U, Q;  // eigenvector rows, and U^dagger
+    if (a.dephase) {
+        double *uc = a.ucache + 2 * k * nn;
+        // the previous call's eigenvectors; padded rows and columns are the identity
+        auto load_prev = [&]() {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const double2 v = load(uc, j);
+                U.r[j] = own[j] ? v.x : (cacc_row(j) == col ? 1.0 : 0.0);
+                U.i[j] = own[j] ? v.y : 0.0;
+            }
+        };
+        bool rotate = true;
+        if (a.warm) load_prev();
+        {
+            CAcc h;
+            phase_acc(0, h);
+            acc_put(S1, pos, h);
+        }
+        if (a.warm) {
+            acc_dagger(S0, pos, U, Q);  // (its sync orders the store of H0 too)
+            rotate = !refine16(S0, S1, pos, U, Q, Dg, a.sweeps);
+        } else {
+            wsync();
+        }
+        if (rotate) {
+            const Lane L = lane_id<N, LR>(a.nk, blk);
+            cd A[C], V[C];
+            CAcc S;
+            if (a.warm) {
+                // S = U H0 U^dagger of the previous call's U
+                load_prev();
+                acc_dagger(S0, pos, U, Q);
+                CAcc h, t;
+                acc_get(S1, pos, h);
+                cacc_zero(t);
+                mul_dagger(h, Q, t);
+                cacc_zero(S);
+                mul_dagger(Q, t, S);
+                cacc_store(S0, U);
+                wsync();
+                load_u<N, LR>(S0, L, V);
+                wsync();
+            } else {
+                acc_get(S1, pos, S);
+            }
+            cacc_store(S0, S);
+            wsync();
+            load_xrow<N, LR>(S0, L, A);
+            wave_jacobi<N, LR>(A, V, L, a.sweeps, Dg, Ja, Jb, Fa, !a.warm);
+            wsync();
+            store_u<N, LR>(S0, L, V);
+            wsync();
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const cd u = S0[sw<16>(cacc_row(j), col)], q = S0[sw<16>(col, cacc_row(j))];
+                U.r[j] = u.x;
+                U.i[j] = u.y;
+                Q.r[j] = q.x;
+                Q.i[j] = -q.y;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (own[j]) reinterpret_cast<double2 *>(uc)[ent[j]] = make_double2(U.r[j], U.i[j]);
+        wsync();
+    }
+    // rho = x + sum_j c_j k_j, left to right
+    CAcc rho;
+    {
+        const StageInput &inp = a.in;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const double2 v = load(inp.x + 2 * kst, j);
+            rho.r[j] = v.x;
+            rho.i[j] = v.y;
+        }
+#pragma unroll
+        for (int d = 0; d < 6; d++)
+            if (d < inp.nt) {
+                const double *kd = inp.k[d] + 2 * kst;
+                const double c = inp.c[d];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const double2 v = load(kd, j);
+                    rho.r[j] += c * v.x;
+                    rho.i[j] += c * v.y;
+                }
+            }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (!own[j]) rho.r[j] = rho.i[j] = 0;
+    }
+    // a matrix of the state from the accumulator, with zero pads
+    auto store = [&](double *dst, const CAcc &m) {
+        double2 *d2 = reinterpret_cast<double2 *>(dst) + kst;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (own[j]) d2[ent[j]] = make_double2(m.r[j], m.i[j]);
+        if ((int)threadIdx.x < a.P - nn) d2[nn + threadIdx.x] = make_double2(0.0, 0.0);
+    };
+    if (a.xout) store(a.xout, rho);
+    acc_put(S1, pos, rho);
+    CAcc D;
+    cacc_zero(D);
+    if (a.dephase) {
+        CAcc t, h;
+        cacc_zero(t);
+        mul_dagger(rho, Q, t);  // rho^dagger U^dagger
+        cacc_zero(h);
+        mul_dagger(Q, t, h);  // (U rho U^dagger)^dagger
+        const double eb = Dg[col];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            double gam;
+            if (a.w < 0) {
+                gam = (cacc_row(j) != col) ? 1.0 : 0.0;
+            } else {
+                const double dE = (Dg[cacc_row(j)] - eb) / a.w;
+                gam = 1 - exp(-dE * dE);
+            }
+            const double f = -gam * a.F2;
+            h.r[j] *= f;
+            h.i[j] *= f;
+        }
+        cacc_zero(t);
+        mul_dagger(h, U, t);  // (D o U rho U^dagger) U
+        mul_dagger(U, t, D);  // U^dagger (..)
+    }
+    // coherent part -i (H_E rho - rho H_E): D + (-i) X = D + (X.i, -X.r), so it is
+    // accumulated as i (rho H_E - H_E rho) with the accumulators' roles exchanged
+    {
+        CAcc he, t;
+        phase_acc(1, he);
+        acc_put(S0, pos, he);
+        wsync();
+        cd x[4], y[4];
+        t.r = D.i;
+        t.i = -D.r;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const cd v = S0[pos.tr + 4 * j];
+            x[j] = mk(-v.x, -v.y);
+        }
+        acc_right(rho, y);
+        mfma_cmul(x, y, t);  // - H_E rho
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[j] = S1[pos.tr + 4 * j];
+        acc_right(he, y);
+        mfma_cmul(x, y, t);  // + rho H_E
+        D.r = -t.i;
+        D.i = t.r;
+    }
+    store(a.dxdt, D);
+    if (a.err_partial) {
+        double v = 0;
+#pragma unroll 2
+        for (int j = 0; j < 4; j++)
+            if (own[j]) {
+                double2 kv[6];
+#pragma unroll
+                for (int d = 0; d < 5; d++) kv[d] = load(a.in.k[d] + 2 * kst, j);
+                kv[5] = make_double2(D.r[j], D.i[j]);
+                v = fmax(v, err_entry(load(a.in.x + 2 * kst, j), kv, a.err_e, a.err_ea, a.err_er, a.err_dt));
+            }
+        v = fmax(v, stage_err_specials(a, blk));
+        v = seg_max<64>(v);
         if (threadIdx.x == 0) a.err_partial[blk] = v;
     }
 }
@@ -1416,7 +1835,10 @@ __device__ __forceinline__ void rhs_stage_body(const StageArgs &a, const long bl
 {
     using G = Geo<N, LR>;
     constexpr int C = G::C;
-    if constexpr (N == 16) {
+    if constexpr (N == 16 && LR == 4) {
+        rhs_stage_body16q(a, blk);
+        return;
+    } else if constexpr (N == 16) {
         rhs_stage_body16<LR>(a, blk);
         return;
     } else if constexpr (LR == 1) {
@@ -1555,13 +1977,11 @@ __device__ __forceinline__ void rhs_stage_body(const StageArgs &a, const long bl
 }
 
 // minimum waves per SIMD the register allocation must allow: the 8-band kernel
-// at one lane per row fits three (at most 168 VGPRs); the 16-band
-// kernel at 4 lanes per row fits four (at most 128 VGPRs; 8.9 KB of LDS per
-// wavefront) when the allocator is told so, instead of two with part of the
-// matrix-core operands in AGPRs; at 2 lanes per row a bound would only buy
-// spills to scratch
+// at one lane per row and the 16-band kernel at four fit three (at most 168
+// VGPRs; a fourth wave of the latter costs spills, see refine16); at 2 lanes per
+// row a bound would only buy spills to scratch
 template <int N, int LR>
-constexpr int stage_min_waves() { return (N == 16 && LR == 4) ? 4 : (N == 8 && LR == 1) ? 3 : 1; }
+constexpr int stage_min_waves() { return (N == 16 && LR == 4) || (N == 8 && LR == 1) ? 3 : 1; }
 
 template <int N, int LR>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(stage_min_waves<N, LR>())))

@@ -1,6 +1,8 @@
-"""The stage kernel at the edges of its phase-sum path,
+"""The stage kernel at the edges of its phase-sum and eigenvector paths,
 against the CPU oracle.  Tolerance: 1e-12 relative, as for every single
 kernel (FP64, sums of at most a few hundred products of order one)."""
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -87,3 +89,44 @@ def check_sequence(cfg, steps, ctx=None):
 def test_phase_rows(n, lr, ext, Nk, Nf, monkeypatch):
     monkeypatch.setenv("SBEWH_STAGE_LR", str(lr))
     check_sequence(config(n, ext, Nk, Nf), [0.0, 0.01])
+
+
+# the warm start after steps of A from rounding to a jump across the zone
+STEPS = [0.0, 0.0, 1e-13, 1e-9, 1e-6, 1e-4, -2e-3, 0.02, -0.1, 0.6, 0.0, 2e-3]
+
+
+@pytest.mark.parametrize("n,copies", [(9, 1), (11, 1), (16, 1), (16, 2), (12, 4)])
+def test_warm_start_steps(n, copies, monkeypatch):
+    """16-band kernels: warm starts refined by products, and those left to
+    the rotations (large steps, near crossings), also with every band
+    degenerate"""
+    monkeypatch.setenv("SBEWH_STAGE_LR", "4")
+    check_sequence(config(n, (2, 2), (6, 5), (6, 5), copies=copies), STEPS)
+
+
+def test_warm_start_without_sweeps(monkeypatch):
+    """no sweep allowed: a warm call keeps the previous eigenvectors in every layout"""
+    cfg = config(16, (1, 1), (3, 4), (3, 4), sweeps=0)
+    out = []
+    for lr in ("2", "4"):
+        monkeypatch.setenv("SBEWH_STAGE_LR", lr)
+        g, o = SBEContext(cfg), Oracle(dataclasses.replace(cfg, sweeps=12))
+        out.append([g.rhs(x, 3.0) for x in states(o, 2, [0.0, 0.05])])
+        o.close()
+    for a, b in zip(*out):
+        assert np.abs(a - b).max() / np.abs(b).max() < 1e-12
+
+
+def test_warm_start_long_chain(monkeypatch):
+    """400 warm starts one after the other leave the decomposition unitary
+    and converged (the last call agrees with the oracle as the first does)"""
+    monkeypatch.setenv("SBEWH_STAGE_LR", "4")
+    cfg = config(16, (2, 2), (6, 5), (6, 5))
+    g, o = SBEContext(cfg), Oracle(cfg)
+    x = states(o, 1, [0.0])[0]
+    for q in range(400):
+        x[0] += 0.004 * np.cos(0.1 * q)
+        a = g.rhs(x, 3.0)
+    b = o.rhs(x, 3.0)
+    o.close()
+    assert np.abs(a - b).max() / np.abs(b).max() < 1e-12
