@@ -28,21 +28,23 @@ struct GemmArgs {
     long ldh, strideH;
     const float *Zin;      // mode 3
     long ldz, strideZ;
+    float *rowsum;         // if set: rowsum[m] = sum_k opA(m, k)
+    long strideRow;
+    int vecA, vecB;        // whole 16-byte vectors (set by launch_gemm)
 };
 hipError_t launch_gemm(const GemmArgs &g, int ta, int tb, int members, hipStream_t s);
 
 // X[e][b][:] = bf16(Xall[perm[e][(step % spe) * batch + b]]), T likewise (fp32);
 // step = *counter.  perm: [members][n_perm]; member e's rows start at row e * cap.
+// perm null: X[e][b][:] = bf16(Xall[first + b]) for every member.
 hipError_t launch_gather(const float *Xall, const float *Tall, int din, int dout, const int *perm, long n_perm,
-                         const int *counter, int spe, int batch, int cap, int members, bf16 *X, float *T,
+                         const int *counter, int spe, int batch, int cap, int members, long first, bf16 *X, float *T,
                          hipStream_t s);
-// dY = 2 (Y - T) / (batch dout) in bf16; loss[e][*counter] = mean (Y - T)^2 (if loss != null);
+// dY = 2 (Y - T) / (batch dout) in bf16; loss[e][*counter] = mean (Y - T)^2 (if loss != null;
+// slot 0 without a counter);
 // member e's rows start at row e * cap
 hipError_t launch_loss_grad(const float *Y, const float *T, int batch, int cap, int dout, int members, bf16 *dY,
                             float *loss, int loss_stride, const int *counter, hipStream_t s);
-// db[e][n] = sum_b dZ[e][b][n]
-hipError_t launch_colsum(const bf16 *dZ, int batch, int n, long strideZ, int members, float *db, long strideDb,
-                         hipStream_t s);
 // Adam on fp32 master parameters (all members, count = members * P) with
 // lr_t = lr * 0.5 (1 + cos(pi step / total)); writes the bf16 copies; step = *counter + 1
 hipError_t launch_adam(float *p, bf16 *pb, float *m, float *v, const float *g, long count, float lr, float b1,

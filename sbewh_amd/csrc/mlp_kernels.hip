@@ -4,13 +4,17 @@
 //
 // GEMM tiling: a 256-thread block owns a 64 x 64 tile of C, each of its four
 // wavefronts a 32 x 32 sub-tile accumulated in 16 FP32 registers per lane.
-// Per MFMA step a lane supplies 8 consecutive k of row (l mod 32) of opA and
-// the same 8 k of column (l mod 32) of opB, k = k0 + 8 (l / 32) + i; the
-// product sums over all 16 k of the step whatever order the unit pairs them
-// in, as long as A and B slots agree.  The 32 x 32 result sits in lane l,
-// register r at column l mod 32, row 8 (r / 4) + 4 (l / 32) + r mod 4.
-// Operands are read straight from global memory (the matrices are at most
-// 4096 x 256; rows are reused from L1/L2), out-of-range k, m, n read as 0.
+// The block's operands pass through LDS in chunks of TK k, both with k
+// contiguous; the next chunk's loads (16 bytes per lane) are in flight under
+// the current chunk's matrix instructions.  Per MFMA step a lane supplies 8
+// consecutive k of row (l mod 32) of opA and the same 8 k of column (l mod 32)
+// of opB, k = k0 + 8 (l / 32) + i; the product sums over all 16 k of the step
+// whatever order the unit pairs them in, as long as A and B slots agree.  The
+// 32 x 32 result sits in lane l, register r at column l mod 32, row
+// 8 (r / 4) + 4 (l / 32) + r mod 4.  Out-of-range k, m, n read as 0.
+// Loading fragments element by element from global memory bound the former
+// kernel: 4096 rows through a 256 x 256 layer of five members took 150 us, now
+// 18 us (the same steps in the same order: the same bits).
 #include "device_common.hpp"
 #include "mlp.hpp"
 
@@ -26,28 +30,101 @@ __device__ __forceinline__ float dsilu(float z)
     return s * (1.0f + z * (1.0f - s));
 }
 
+constexpr int TK = 64;       // k per LDS chunk (128: 21 us where 64 takes 16, twice the LDS per block)
+constexpr int TV = TK / 32;  // vectors per thread and operand of a chunk
+constexpr int TS = TK + 8;   // LDS row stride: rows stay 16-byte aligned, banks spread
+
+// Elements (r, k) of a chunk operand, r = r0 .. r0 + 63, k = k0 .. k0 + TK - 1, TV
+// vectors of 8 per thread.  RC 0: P[r ld + k], a vector runs along k; RC 1:
+// P[k ld + r], a vector runs along r.  vec: every vector inside the matrix is
+// aligned and whole (decided on the host).
+template <int RC>
+__device__ __forceinline__ void chunk_load(const bf16 *P, long ld, int rows, int K, int r0, int k0, int vec, v8bf (&v)[TV])
+{
+    const bf16 zero = (bf16)0.0f;
+#pragma unroll
+    for (int i = 0; i < TV; i++) {
+        const int e = threadIdx.x + 256 * i;
+        const int r = r0 + (RC ? (e & 7) * 8 : e / (TK / 8)), k = k0 + (RC ? e >> 3 : (e % (TK / 8)) * 8);
+        const bool in = r < rows && k < K;
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[i][j] = zero;
+        if (!in) continue;
+        const bf16 *q = P + (RC ? (long)k * ld + r : (long)r * ld + k);
+        if (vec) {
+            v[i] = *reinterpret_cast<const v8bf *>(q);
+        } else {
+            const int left = RC ? rows - r : K - k;
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                if (j < left) v[i][j] = q[j];
+        }
+    }
+}
+
+// the same vectors into the LDS chunk [r][k]
+template <int RC>
+__device__ __forceinline__ void chunk_store(bf16 *L, const v8bf (&v)[TV])
+{
+#pragma unroll
+    for (int i = 0; i < TV; i++) {
+        const int e = threadIdx.x + 256 * i;
+        if (RC) {
+            const int r = (e & 7) * 8, k = e >> 3;
+#pragma unroll
+            for (int j = 0; j < 8; j++) L[(r + j) * TS + k] = v[i][j];
+        } else {
+            *reinterpret_cast<v8bf *>(L + e / (TK / 8) * TS + e % (TK / 8) * 8) = v[i];
+        }
+    }
+}
+
 template <int TA, int TB>
 __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g)
 {
+    __shared__ __align__(16) bf16 As[64 * TS], Bs[64 * TS];
     const int e = blockIdx.z;
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-    const int m0 = blockIdx.y * 64 + (w >> 1) * 32, n0 = blockIdx.x * 64 + (w & 1) * 32;
+    const int mb = blockIdx.y * 64, nb = blockIdx.x * 64;
+    const int m0 = mb + (w >> 1) * 32, n0 = nb + (w & 1) * 32;
     const bf16 *A = g.A + e * g.strideA, *B = g.B + e * g.strideB;
-    const int row = m0 + (l & 31), col = n0 + (l & 31), kg = 8 * (l >> 5);
+    const int col = n0 + (l & 31);
+    const bf16 *fa = As + ((w >> 1) * 32 + (l & 31)) * TS + 8 * (l >> 5);
+    const bf16 *fb = Bs + ((w & 1) * 32 + (l & 31)) * TS + 8 * (l >> 5);
+    const bool sums = g.rowsum && blockIdx.x == 0;
+    float rs = 0.0f;
     v16f acc;
 #pragma unroll
     for (int r = 0; r < 16; r++) acc[r] = 0.0f;
-    const bf16 zero = (bf16)0.0f;
-    for (int k0 = 0; k0 < g.K; k0 += 16) {
-        v8bf a, b;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int k = k0 + kg + i;
-            const bool kin = k < g.K;
-            a[i] = (kin && row < g.M) ? (TA ? A[(long)k * g.lda + row] : A[(long)row * g.lda + k]) : zero;
-            b[i] = (kin && col < g.N) ? (TB ? B[(long)col * g.ldb + k] : B[(long)k * g.ldb + col]) : zero;
+    v8bf va[TV], vb[TV];
+    chunk_load<TA>(A, g.lda, g.M, g.K, mb, 0, g.vecA, va);
+    chunk_load<!TB>(B, g.ldb, g.N, g.K, nb, 0, g.vecB, vb);
+    for (int k0 = 0; k0 < g.K; k0 += TK) {
+        if (k0) __syncthreads();
+        chunk_store<TA>(As, va);
+        chunk_store<!TB>(Bs, vb);
+        __syncthreads();
+        if (k0 + TK < g.K) {
+            chunk_load<TA>(A, g.lda, g.M, g.K, mb, k0 + TK, g.vecA, va);
+            chunk_load<!TB>(B, g.ldb, g.N, g.K, nb, k0 + TK, g.vecB, vb);
         }
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+#pragma unroll
+        for (int s = 0; s < TK / 16; s++)
+            if (k0 + 16 * s < g.K)
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const v8bf *>(fa + 16 * s),
+                                                              *reinterpret_cast<const v8bf *>(fb + 16 * s), acc, 0, 0, 0);
+        if (sums) {
+            // four threads per row of opA, a quarter of the chunk each
+            const bf16 *q = As + (threadIdx.x >> 2) * TS + (threadIdx.x & 3) * (TK / 4);
+#pragma unroll
+            for (int j = 0; j < TK / 4; j++) rs += (float)q[j];
+        }
+    }
+    if (sums) {
+        rs += __shfl_xor(rs, 1);
+        rs += __shfl_xor(rs, 2);
+        const int m = mb + (threadIdx.x >> 2);
+        if ((threadIdx.x & 3) == 0 && m < g.M) g.rowsum[e * g.strideRow + m] = rs;
     }
     const int n = col;
     if (n >= g.N) return;
@@ -72,8 +149,16 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g)
     }
 }
 
-hipError_t launch_gemm(const GemmArgs &g, int ta, int tb, int members, hipStream_t s)
+hipError_t launch_gemm(const GemmArgs &g0, int ta, int tb, int members, hipStream_t s)
 {
+    // 16-byte loads: the vectors of 8 along an operand's contiguous index are
+    // whole (its extent and every row and member start are multiples of 8)
+    GemmArgs g = g0;
+    auto whole = [](const bf16 *p, long extent, long ld, long stride) {
+        return ((reinterpret_cast<unsigned long long>(p) & 15) | ((extent | ld | stride) & 7)) == 0;
+    };
+    g.vecA = whole(g.A, ta ? g.M : g.K, g.lda, members > 1 ? g.strideA : 0);
+    g.vecB = whole(g.B, tb ? g.K : g.N, g.ldb, members > 1 ? g.strideB : 0);
     dim3 grid((unsigned)((g.N + 63) / 64), (unsigned)((g.M + 63) / 64), (unsigned)members), blk(256);
     switch (ta * 2 + tb) {
     case 0: hipLaunchKernelGGL((gemm_kernel<0, 0>), grid, blk, 0, s, g); break;
@@ -86,78 +171,56 @@ hipError_t launch_gemm(const GemmArgs &g, int ta, int tb, int members, hipStream
 
 // grid (batch, members), block 64
 __global__ void gather_kernel(const float *Xall, const float *Tall, int din, int dout, const int *perm, long n_perm,
-                              const int *counter, int spe, int batch, int cap, bf16 *X, float *T)
+                              const int *counter, int spe, int batch, int cap, long first, bf16 *X, float *T)
 {
     const int b = blockIdx.x, e = blockIdx.y;
-    const long idx = perm[e * n_perm + (long)(*counter % spe) * batch + b];
+    const long idx = perm ? perm[e * n_perm + (long)(*counter % spe) * batch + b] : first + b;
     const long row = (long)e * cap + b;
     for (int i = threadIdx.x; i < din; i += 64) X[row * din + i] = (bf16)Xall[idx * din + i];
     for (int i = threadIdx.x; i < dout; i += 64) T[row * dout + i] = Tall[idx * dout + i];
 }
 
 hipError_t launch_gather(const float *Xall, const float *Tall, int din, int dout, const int *perm, long n_perm,
-                         const int *counter, int spe, int batch, int cap, int members, bf16 *X, float *T,
+                         const int *counter, int spe, int batch, int cap, int members, long first, bf16 *X, float *T,
                          hipStream_t s)
 {
     hipLaunchKernelGGL(gather_kernel, dim3((unsigned)batch, (unsigned)members), dim3(64), 0, s, Xall, Tall, din, dout,
-                       perm, n_perm, counter, spe, batch, cap, X, T);
+                       perm, n_perm, counter, spe, batch, cap, first, X, T);
     return hipGetLastError();
 }
 
-__device__ __forceinline__ float block_sum256(float v)
-{
-    __shared__ float red[256];
-    red[threadIdx.x] = v;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    return red[0];
-}
-
 // one block per member, fixed summation order
-__global__ __launch_bounds__(256) void loss_grad_kernel(const float *Y, const float *T, int batch, int cap, int dout,
-                                                        bf16 *dY, float *loss, int loss_stride, const int *counter)
+constexpr int LOSS_T = 1024;
+__global__ __launch_bounds__(LOSS_T) void loss_grad_kernel(const float *Y, const float *T, int batch, int cap, int dout,
+                                                           bf16 *dY, float *loss, int loss_stride, const int *counter)
 {
+    __shared__ float red[LOSS_T / 64];
     const int e = blockIdx.x;
     const long cnt = (long)batch * dout, off = (long)e * cap * dout;
     const float sc = 2.0f / (float)cnt;
     float acc = 0.0f;
-    for (long i = threadIdx.x; i < cnt; i += 256) {
+#pragma unroll 4
+    for (long i = threadIdx.x; i < cnt; i += LOSS_T) {
         const float d = Y[off + i] - T[off + i];
         dY[off + i] = (bf16)(sc * d);
         acc += d * d;
     }
-    acc = block_sum256(acc);
-    if (loss && threadIdx.x == 0) loss[(long)e * loss_stride + *counter] = acc / (float)cnt;
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) acc += __shfl_xor(acc, m);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0 && loss) {
+        float t = 0.0f;
+        for (int w = 0; w < LOSS_T / 64; w++) t += red[w];
+        loss[(long)e * loss_stride + (counter ? *counter : 0)] = t / (float)cnt;
+    }
 }
 
 hipError_t launch_loss_grad(const float *Y, const float *T, int batch, int cap, int dout, int members, bf16 *dY,
                             float *loss, int loss_stride, const int *counter, hipStream_t s)
 {
-    hipLaunchKernelGGL(loss_grad_kernel, dim3((unsigned)members), dim3(256), 0, s, Y, T, batch, cap, dout, dY, loss,
+    hipLaunchKernelGGL(loss_grad_kernel, dim3((unsigned)members), dim3(LOSS_T), 0, s, Y, T, batch, cap, dout, dY, loss,
                        loss_stride, counter);
-    return hipGetLastError();
-}
-
-// grid (ceil(n / 256), members): thread per column, sum over the batch in order
-__global__ __launch_bounds__(256) void colsum_kernel(const bf16 *dZ, int batch, int n, long strideZ, float *db,
-                                                     long strideDb)
-{
-    const int c = blockIdx.x * 256 + threadIdx.x, e = blockIdx.y;
-    if (c >= n) return;
-    const bf16 *z = dZ + e * strideZ;
-    float acc = 0.0f;
-    for (int b = 0; b < batch; b++) acc += (float)z[(long)b * n + c];
-    db[e * strideDb + c] = acc;
-}
-
-hipError_t launch_colsum(const bf16 *dZ, int batch, int n, long strideZ, int members, float *db, long strideDb,
-                         hipStream_t s)
-{
-    hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((n + 255) / 256), (unsigned)members), dim3(256), 0, s, dZ,
-                       batch, n, strideZ, db, strideDb);
     return hipGetLastError();
 }
 

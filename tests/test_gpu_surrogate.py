@@ -74,6 +74,28 @@ def test_gradient_matches_oracle(rows):
         assert rel2(g[e], g64) <= 5e-2, (e, rel2(g[e], g64))
 
 
+# widths and row counts at the edges of the 64-wide tiles and of the 16-byte
+# vectors: whole vectors, remainders, one element, more than one chunk of k
+@pytest.mark.parametrize("dims,rows", [((1, 1, 1), 1), ((5, 33, 7), 63), ((8, 64, 64, 3), 64), ((6, 72, 65, 40), 65),
+                                       ((16, 130, 8), 129), ((3, 136, 200, 5), 200)])
+def test_tile_edges(dims, rows):
+    """every element by itself: within the rounding of the BF16 values it is
+    made of (2^-8 of the products' sum at most, for a layer or two)"""
+    ens = MLPEnsemble(dims, 3, seed=46)
+    rng = np.random.default_rng(sum(dims) + rows)
+    x = rng.uniform(-1, 1, size=(rows, dims[0])).astype(np.float32)
+    t = rng.normal(size=(rows, dims[-1])).astype(np.float32)
+    y = ens.forward(x)
+    loss, g = ens.gradient(x, t)
+    for e in range(3):
+        p = ens.get_params(e).astype(np.float64)
+        ref = mlp_ref.forward(p, list(dims), x.astype(np.float64), bf16=True)
+        lr, gr = mlp_ref.loss_and_grad(p, list(dims), x.astype(np.float64), t.astype(np.float64), bf16=True)
+        assert np.abs(y[e] - ref).max() <= 2 ** -7 * max(1.0, np.abs(ref).max())
+        assert abs(loss[e] - lr) <= 1e-2 * lr
+        assert np.abs(g[e] - gr).max() <= 2 ** -6 * np.abs(gr).max()
+
+
 def test_training_reduces_loss_and_members_differ():
     say("[gpu] mlp training, 2048 rows, 60 epochs")
     rng = np.random.default_rng(5)
