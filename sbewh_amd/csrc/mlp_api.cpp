@@ -70,10 +70,16 @@ struct sbe_mlp {
     std::vector<float *> Z;       // [L-1] pre-activations
     std::vector<bf16 *> H;        // [L-1] activations
     float *Y = nullptr, *T = nullptr;
+    // rows and targets as the caller gives them, up to io_cap rows, and the
+    // members' losses: kept from call to call, given back with the object
+    int io_cap = 0;
+    float *io_x = nullptr, *io_t = nullptr, *io_loss = nullptr;
 
     ~sbe_mlp()
     {
         free_batch();
+        for (void *q : {(void *)io_x, (void *)io_t, (void *)io_loss})
+            if (q) (void)hipFree(q);
         for (void *q : {(void *)p, (void *)m, (void *)v, (void *)g, (void *)pb, (void *)counter})
             if (q) (void)hipFree(q);
         if (stream) (void)hipStreamDestroy(stream);
@@ -105,6 +111,20 @@ struct sbe_mlp {
         dY = dmalloc<bf16>((size_t)E * rows * d[L]);
         dZa = dmalloc<bf16>((size_t)E * rows * wmax);
         dZb = dmalloc<bf16>((size_t)E * rows * wmax);
+    }
+
+    void ensure_io(int rows)
+    {
+        if (!io_loss) io_loss = dmalloc<float>(E);
+        if (rows <= io_cap) return;
+        io_cap = 0;
+        for (float **q : {&io_x, &io_t}) {
+            if (*q) MCHK(hipFree(*q));
+            *q = nullptr;
+        }
+        io_x = dmalloc<float>((size_t)rows * d[0]);
+        io_t = dmalloc<float>((size_t)rows * d[L]);
+        io_cap = rows;
     }
 
     // forward of all members on the `rows` rows staged in X; Y receives the output
@@ -310,37 +330,22 @@ int sbe_mlp_forward(sbe_mlp *mlp, int count, const float *x, float *y)
         const int chunk = 4096;
         n.ensure_batch(std::min(count, chunk));
         const int din = n.d[0], dout = n.d[n.L];
-        std::vector<int> perm;
-        int *dperm = dmalloc<int>((size_t)n.E * n.cap);
-        int *dctr = dmalloc<int>(1);
-        float *dx = dmalloc<float>((size_t)count * din);
-        std::vector<float> yb((size_t)n.E * n.cap * dout);
-        try {
-            MCHK(hipMemcpyAsync(dx, x, (size_t)count * din * sizeof(float), hipMemcpyHostToDevice, n.stream));
-            MCHK(hipMemsetAsync(dctr, 0, sizeof(int), n.stream));
-            for (int s0 = 0; s0 < count; s0 += n.cap) {
-                const int rows = std::min(n.cap, count - s0);
-                perm.assign((size_t)n.E * n.cap, 0);
-                for (int e = 0; e < n.E; e++)
-                    for (int b = 0; b < rows; b++) perm[(size_t)e * n.cap + b] = s0 + b;
-                MCHK(hipMemcpyAsync(dperm, perm.data(), perm.size() * sizeof(int), hipMemcpyHostToDevice, n.stream));
-                MCHK(launch_gather(dx, dx, din, 0, dperm, n.cap, dctr, 1, rows, n.cap, n.E, 0, n.X, n.T, n.stream));
-                n.forward(rows);
-                MCHK(hipMemcpyAsync(yb.data(), n.Y, yb.size() * sizeof(float), hipMemcpyDeviceToHost, n.stream));
-                MCHK(hipStreamSynchronize(n.stream));
-                for (int e = 0; e < n.E; e++)
-                    std::memcpy(y + ((size_t)e * count + s0) * dout, yb.data() + (size_t)e * n.cap * dout,
-                                (size_t)rows * dout * sizeof(float));
-            }
-        } catch (...) {
-            (void)hipFree(dperm);
-            (void)hipFree(dctr);
-            (void)hipFree(dx);
-            throw;
+        // A call's device buffers and permutation used to be allocated, filled
+        // and freed each time, and the output staged through a host vector:
+        // 4096 rows of five members took 850 us on the host beside 72 us of kernels.
+        n.ensure_io(n.cap);
+        for (int s0 = 0; s0 < count; s0 += n.cap) {
+            const int rows = std::min(n.cap, count - s0);
+            MCHK(hipMemcpyAsync(n.io_x, x + (size_t)s0 * din, (size_t)rows * din * sizeof(float),
+                                hipMemcpyHostToDevice, n.stream));
+            MCHK(launch_gather(n.io_x, n.io_x, din, 0, nullptr, 0, nullptr, 1, rows, n.cap, n.E, 0, n.X, n.T,
+                               n.stream));
+            n.forward(rows);
+            for (int e = 0; e < n.E; e++)
+                MCHK(hipMemcpyAsync(y + ((size_t)e * count + s0) * dout, n.Y + (size_t)e * n.cap * dout,
+                                    (size_t)rows * dout * sizeof(float), hipMemcpyDeviceToHost, n.stream));
+            MCHK(hipStreamSynchronize(n.stream));
         }
-        MCHK(hipFree(dperm));
-        MCHK(hipFree(dctr));
-        MCHK(hipFree(dx));
     });
 }
 
@@ -351,30 +356,17 @@ int sbe_mlp_gradient(sbe_mlp *mlp, int count, const float *x, const float *t, fl
         sbe_mlp &n = *mlp;
         n.ensure_batch(count);
         const int din = n.d[0], dout = n.d[n.L];
-        std::vector<int> perm((size_t)n.E * count);
-        for (int e = 0; e < n.E; e++)
-            for (int b = 0; b < count; b++) perm[(size_t)e * count + b] = b;
-        int *dperm = dmalloc<int>(perm.size());
-        int *dctr = dmalloc<int>(1);
-        float *dx = dmalloc<float>((size_t)count * din), *dt = dmalloc<float>((size_t)count * dout);
-        float *dl = dmalloc<float>(n.E);
-        try {
-            MCHK(hipMemcpyAsync(dperm, perm.data(), perm.size() * sizeof(int), hipMemcpyHostToDevice, n.stream));
-            MCHK(hipMemcpyAsync(dx, x, (size_t)count * din * sizeof(float), hipMemcpyHostToDevice, n.stream));
-            MCHK(hipMemcpyAsync(dt, t, (size_t)count * dout * sizeof(float), hipMemcpyHostToDevice, n.stream));
-            MCHK(hipMemsetAsync(dctr, 0, sizeof(int), n.stream));
-            MCHK(launch_gather(dx, dt, din, dout, dperm, count, dctr, 1, count, n.cap, n.E, 0, n.X, n.T, n.stream));
-            n.forward(count);
-            MCHK(launch_loss_grad(n.Y, n.T, count, n.cap, dout, n.E, n.dY, dl, 1, dctr, n.stream));
-            n.backward(count);
-            MCHK(hipMemcpyAsync(loss, dl, n.E * sizeof(float), hipMemcpyDeviceToHost, n.stream));
-            MCHK(hipMemcpyAsync(grad, n.g, (size_t)n.E * n.P * sizeof(float), hipMemcpyDeviceToHost, n.stream));
-            MCHK(hipStreamSynchronize(n.stream));
-        } catch (...) {
-            for (void *q : {(void *)dperm, (void *)dctr, (void *)dx, (void *)dt, (void *)dl}) (void)hipFree(q);
-            throw;
-        }
-        for (void *q : {(void *)dperm, (void *)dctr, (void *)dx, (void *)dt, (void *)dl}) MCHK(hipFree(q));
+        n.ensure_io(count);
+        MCHK(hipMemcpyAsync(n.io_x, x, (size_t)count * din * sizeof(float), hipMemcpyHostToDevice, n.stream));
+        MCHK(hipMemcpyAsync(n.io_t, t, (size_t)count * dout * sizeof(float), hipMemcpyHostToDevice, n.stream));
+        MCHK(launch_gather(n.io_x, n.io_t, din, dout, nullptr, 0, nullptr, 1, count, n.cap, n.E, 0, n.X, n.T,
+                           n.stream));
+        n.forward(count);
+        MCHK(launch_loss_grad(n.Y, n.T, count, n.cap, dout, n.E, n.dY, n.io_loss, 1, nullptr, n.stream));
+        n.backward(count);
+        MCHK(hipMemcpyAsync(loss, n.io_loss, n.E * sizeof(float), hipMemcpyDeviceToHost, n.stream));
+        MCHK(hipMemcpyAsync(grad, n.g, (size_t)n.E * n.P * sizeof(float), hipMemcpyDeviceToHost, n.stream));
+        MCHK(hipStreamSynchronize(n.stream));
     });
 }
 
