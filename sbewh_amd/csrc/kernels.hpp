@@ -249,8 +249,10 @@ struct ObsArgs {
     int pstride;           // row stride of partial (3 for the current alone)
 };
 hipError_t launch_observe_j(const ObsArgs &a, hipStream_t s);
-// entry j owns blocks [block0[j], block0[j] + nk_j) (one block per k-point)
-hipError_t launch_observe_j_batched(const ObsArgs *d_args, const long *d_block0, int m, long blocks, hipStream_t s);
+// k-points per block of the per-k current for n bands
+int observe_block_k(int n);
+// entry j owns blocks [block0[j], block0[j] + ceil(nk_j / observe_block_k(n)))
+hipError_t launch_observe_j_batched(int n, const ObsArgs *d_args, const long *d_block0, int m, long blocks, hipStream_t s);
 // the per-k current alone: partial[k * pstride + d] = j_k,d (d < 3), no reduction
 hipError_t launch_observe_jk(const ObsArgs &a, hipStream_t s);
 

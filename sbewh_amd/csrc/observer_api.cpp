@@ -44,7 +44,11 @@ int sbe_observer_create(sbe_ctx *ctx, const sbe_region *regions, int num_regions
         }
         o->reg = dalloc<RegionDev>(num_regions);
         HIPCHK(hipMemcpy(o->reg, rd.data(), rd.size() * sizeof(RegionDev), hipMemcpyHostToDevice));
-        o->chunk = 4096;
+        // chunks of k small enough that regions x quantities x chunks fill the
+        // GPU (2048 blocks), of 256 k-points at least and 4096 at most (many regions)
+        const long per_chunk = (long)o->R * ((o->Qmax + 63) / 64);
+        const long want = std::max(1L, (2048 + per_chunk - 1) / per_chunk);
+        o->chunk = std::min(4096L, std::max(256L, ((c.nk + want - 1) / want + 255) / 256 * 256));
         o->chunks = (int)((c.nk + o->chunk - 1) / o->chunk);
         o->X = dalloc<double>((size_t)c.nk * o->Q);
         o->part = dalloc<double>((size_t)o->R * o->chunks * o->Qmax);

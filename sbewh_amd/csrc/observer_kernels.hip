@@ -10,18 +10,192 @@
 #include "device_common.hpp"
 #include "kernels.hpp"
 #include "observer_device.hpp"
+#include "stage_device.hpp"
 
 namespace sbe {
 
+// The per-k current for matrices that fill wavefronts (N = 8, 16): KB consecutive
+// k-points per wavefront.  Lane entry (a, b) of a k-point's matrices holds T_ba and
+// rho_ba, and the sum over (a, b) goes before the one over the last axis' cells r,
+//   j_d = Re sum_r tw_r sum_ab [ i D_d(r)_ab T_ba - dH_d(r)_ab rho_ba ],
+// so a phase-sum entry is loaded once for all k-points of its row and no operator
+// is formed.  One k-point per wavefront read (1 + 2 dim) n n W_L entries from L2 and
+// as many twiddles per k-point: @JK@.
+template <int N>
+constexpr int jk_block_k() { return N == 16 ? 2 : 8; }
+
+template <int N>
+__device__ __forceinline__ void jk_rows_body(const ObsArgs &a, const long blk)
+{
+    constexpr int KB = jk_block_k<N>(), EK = N * N / 64;
+    const int n = a.n, nn = n * n, M = (1 + 2 * a.dim) * nn, WL = a.ph.WL;
+    const int k0 = __builtin_amdgcn_readfirstlane((int)blk) * KB;
+    int ent[EK];
+    bool own[EK];
+#pragma unroll
+    for (int u = 0; u < EK; u++) {
+        const int idx = threadIdx.x + 64 * u;
+        own[u] = idx / N < n && idx % N < n;
+        ent[u] = own[u] ? idx / N * n + idx % N : 0;
+    }
+    cd H[KB * EK];  // H0(k)
+    if (!phase_rows<N, KB>(H, a.ph, a.nk, n, M, 0, k0)) {
+#pragma unroll
+        for (int kk = 0; kk < KB; kk++)
+#pragma unroll
+            for (int u = 0; u < EK; u++)
+                H[kk * EK + u] = own[u] && k0 + kk < a.nk ? phase_last(a.ph, k0 + kk, M, ent[u]) : mk(0, 0);
+    }
+    cd R[KB * EK], T[KB * EK];
+#pragma unroll
+    for (int kk = 0; kk < KB; kk++)
+#pragma unroll
+        for (int u = 0; u < EK; u++) {
+            const bool in = own[u] && k0 + kk < a.nk;
+            const double2 v = reinterpret_cast<const double2 *>(a.x)[in ? 8 + (k0 + kk) * (long)a.P + ent[u] : 8];
+            R[kk * EK + u] = in ? mk(v.x, v.y) : mk(0, 0);
+        }
+    // T = H0 rho - rho H0, then T and rho transposed
+    if constexpr (N == 16) {
+        __shared__ cd B0[ACC_MS], B1[ACC_MS];
+        const AccPos pos = acc_pos();
+#pragma unroll
+        for (int kk = 0; kk < KB; kk++) {
+            cd *h = H + kk * EK, *r = R + kk * EK, x[4], y[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                B0[pos.nat + 4 * ACC_RS * j] = h[j];
+                B1[pos.nat + 4 * ACC_RS * j] = r[j];
+            }
+            wsync();
+            CAcc t;
+            cacc_zero(t);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                x[j] = B0[pos.tr + 4 * j];
+                y[j] = B1[pos.tr + 4 * j];
+            }
+            mfma_cmul(x, r, t);
+#pragma unroll
+            for (int j = 0; j < 4; j++) x[j] = mk(-y[j].x, -y[j].y);
+            mfma_cmul(x, h, t);
+            wsync();
+            acc_put(B0, pos, t);
+            wsync();
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                T[kk * EK + j] = B0[pos.tr + 4 * j];
+                r[j] = y[j];
+            }
+            wsync();
+        }
+    } else {
+        __shared__ cd Hs[N * (N + 1)], Rs[N * (N + 1)];
+        const int ra = threadIdx.x / N, cb = threadIdx.x % N;
+#pragma unroll
+        for (int kk = 0; kk < KB; kk++) {
+            Hs[ra * (N + 1) + cb] = H[kk];
+            Rs[ra * (N + 1) + cb] = R[kk];
+            wsync();
+            cd t = mk(0, 0);  // T[b][a]
+#pragma unroll
+            for (int l = 0; l < N; l++) {
+                const cd rb = Rs[cb * (N + 1) + l];
+                t = cfma(Hs[cb * (N + 1) + l], Rs[l * (N + 1) + ra], t);
+                t = cfma(mk(-rb.x, -rb.y), Hs[l * (N + 1) + ra], t);
+            }
+            T[kk] = t;
+            R[kk] = Rs[cb * (N + 1) + ra];
+            wsync();
+        }
+    }
+    int rest[KB];
+    unsigned tp[KB];
+    phase_map<KB>(a.ph, a.nk, k0, rest, tp);
+    double jl[KB][3];
+#pragma unroll
+    for (int kk = 0; kk < KB; kk++)
+#pragma unroll
+        for (int d = 0; d < 3; d++) jl[kk][d] = 0;
+    unsigned todo = (1u << KB) - 1;
+    while (todo) {
+        int row;
+        const unsigned mine = next_row_group<KB>(todo, rest, row);
+        const double2 *yr = reinterpret_cast<const double2 *>(a.ph.Y) + (long)row * M;
+#pragma unroll 2
+        for (int q = 0; q < WL; q++) {
+            sd2 tw[KB];
+#pragma unroll
+            for (int kk = 0; kk < KB; kk++) tw[kk] = load_const<sd2>(a.ph.twL, tp[kk] + q);
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+                if (d < a.dim) {
+                    double2 yd[EK], yh[EK];
+#pragma unroll
+                    for (int u = 0; u < EK; u++) {
+                        yd[u] = yr[(long)q * M + (1 + d) * nn + ent[u]];
+                        yh[u] = yr[(long)q * M + (1 + a.dim + d) * nn + ent[u]];
+                    }
+#pragma unroll
+                    for (int kk = 0; kk < KB; kk++)
+                        if ((mine >> kk) & 1) {
+                            asm volatile("");  // a branch over the products, not selects behind them
+                            cd z = mk(0, 0), w = mk(0, 0);
+#pragma unroll
+                            for (int u = 0; u < EK; u++) {
+                                z = cfma(mk(yd[u].x, yd[u].y), T[kk * EK + u], z);
+                                w = cfma(mk(yh[u].x, yh[u].y), R[kk * EK + u], w);
+                            }
+                            // Re tw (i z - w)
+                            jl[kk][d] += tw[kk].x * (-z.y - w.x) - tw[kk].y * (z.x - w.y);
+                        }
+                }
+        }
+    }
+#pragma unroll
+    for (int kk = 0; kk < KB; kk++)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const double v = seg_sum<64>(jl[kk][d]);
+            if (threadIdx.x == 0 && k0 + kk < a.nk) a.partial[(long)a.pstride * (k0 + kk) + d] = v;
+        }
+}
+
+template <int N>
+__global__ __launch_bounds__(64) void jk_rows_kernel(ObsArgs a)
+{
+    jk_rows_body<N>(a, xcd_block(blockIdx.x, gridDim.x));
+}
+
 __global__ __launch_bounds__(64) void jk_kernel(ObsArgs a) { jk_body(a, blockIdx.x); }
 
-// one block per k-point; entry j owns blocks [block0[j], block0[j] + nk_j)
+// entry j owns blocks [block0[j], block0[j] + ceil(nk_j / observe_block_k))
+template <int N>
+__global__ __launch_bounds__(64) void jk_rows_batched_kernel(const ObsArgs *args, const long *block0, int m)
+{
+    const long gb = xcd_block(blockIdx.x, gridDim.x);
+    const int j = find_entry_wave(block0, m, gb);
+    jk_rows_body<N>(args[j], gb - block0[j]);
+}
+
 __global__ __launch_bounds__(64) void jk_batched_kernel(const ObsArgs *args, const long *block0, int m)
 {
     const long gb = blockIdx.x;
     const int j = find_entry_wave(block0, m, gb);
     const ObsArgs a = args[j];
     jk_body(a, gb - block0[j]);
+}
+
+int observe_block_k(int n) { return n > 8 ? jk_block_k<16>() : n > 4 ? jk_block_k<8>() : 1; }
+
+static hipError_t launch_jk(const ObsArgs &a, hipStream_t s)
+{
+    const int kb = observe_block_k(a.n);
+    const dim3 grid((unsigned)((a.nk + kb - 1) / kb)), blk(64);
+    if (a.n > 8) hipLaunchKernelGGL(jk_rows_kernel<16>, grid, blk, 0, s, a);
+    else if (a.n > 4) hipLaunchKernelGGL(jk_rows_kernel<8>, grid, blk, 0, s, a);
+    else hipLaunchKernelGGL(jk_kernel, grid, blk, 0, s, a);
+    return hipGetLastError();
 }
 
 __device__ __forceinline__ void jreduce_body(const double *partial, long nk, double *j_out, int pstride)
@@ -54,8 +228,7 @@ __global__ __launch_bounds__(256) void jreduce_batched_kernel(const ObsArgs *arg
 hipError_t launch_observe_j(const ObsArgs &a, hipStream_t s)
 {
     if (a.n > OBS_MAXN) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(jk_kernel, dim3((unsigned)a.nk), dim3(64), 0, s, a);
-    hipError_t e = hipGetLastError();
+    hipError_t e = launch_jk(a, s);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(jreduce_kernel, dim3(1), dim3(256), 0, s, a.partial, a.nk, a.j_out, a.pstride);
     return hipGetLastError();
@@ -64,8 +237,7 @@ hipError_t launch_observe_j(const ObsArgs &a, hipStream_t s)
 hipError_t launch_observe_jk(const ObsArgs &a, hipStream_t s)
 {
     if (a.n > OBS_MAXN || a.pstride < 3) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(jk_kernel, dim3((unsigned)a.nk), dim3(64), 0, s, a);
-    return hipGetLastError();
+    return launch_jk(a, s);
 }
 
 // ---- k-space regions ------------------------------------------------------
@@ -106,20 +278,23 @@ __device__ __forceinline__ void region_offsets(const RegionArgs &a, double off[3
     }
 }
 
-__device__ __forceinline__ double region_src(const RegionArgs &a, long k, int q)
-{
-    if (q < a.Q) return a.X[k * a.Q + q];
-    if (q == a.Q) return 1.0;
-    return a.x[2 * (8 + k * (long)a.P) + (q - a.Q - 1)];
-}
-
 // grid (R, chunks, ceil(Qtot / 64)), 256 threads: wavefront w of the block
 // takes every fourth group of 64 k-points of the chunk; lane l evaluates the
 // weight of k-point l of the group, then every lane accumulates its quantity
-// q over the 64 k-points with the weights broadcast lane by lane.  Block 0 of
-// region 0 also keeps min / max over k of the smeared occupations.
+// q over the 64 k-points with the weights broadcast lane by lane, eight
+// k-points' values in flight.  Block 0 of region 0 also keeps min / max over k
+// of the smeared occupations.  With one load per trip and 4096 k-points per
+// chunk a record of 24^3 k, 16 bands and two regions took 400 us, now 25 us with the density matrix and 9 without.
+__device__ __forceinline__ double lane_value(double v, int l)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
 __global__ __launch_bounds__(256) void region_sum_kernel(RegionArgs a)
 {
+    constexpr int U = 8;
     const int r = blockIdx.x, ch = blockIdx.y;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int Qtot = a.Q + 1 + (a.density ? 2 * a.n * a.n : 0);
@@ -129,22 +304,33 @@ __global__ __launch_bounds__(256) void region_sum_kernel(RegionArgs a)
     region_offsets(a, off, negA);
     const long k0 = (long)ch * a.chunk, k1 = min(a.nk, k0 + a.chunk);
     const bool mm = (r == 0 && blockIdx.z == 0 && q >= 3 && q < 3 + a.n);
+    // the quantity of this lane over k: a row of X, 1, or an entry of rho
+    const bool one = q == a.Q || q >= Qtot;
+    const double *src = one || q < a.Q ? a.X + (one ? 0 : q) : a.x + 16 + (q - a.Q - 1);
+    const long step = one || q < a.Q ? a.Q : 2 * (long)a.P;
     double acc = 0, mn = INFINITY, mx = -INFINITY;
+    auto add = [&](double w, double v) {
+        if (one) v = 1.0;
+        acc += w * v;
+        if (mm) {
+            mn = fmin(mn, v);
+            mx = fmax(mx, v);
+        }
+    };
     for (long g = k0 + 64 * wv; g < k1; g += 256) {
         const long kl = g + lane;
         const double wl = kl < k1 ? region_w(a, rg, kl, off, negA) : 0.0;
         const int cnt = (int)min((long)64, k1 - g);
-        for (int m = 0; m < cnt; m++) {
-            const double w = __shfl(wl, m);
-            if (q < Qtot) {
-                const double v = region_src(a, g + m, q);
-                acc += w * v;
-                if (mm) {
-                    mn = fmin(mn, v);
-                    mx = fmax(mx, v);
-                }
-            }
+        const double *p = src + g * step;
+        int m = 0;
+        for (; m + U <= cnt; m += U) {
+            double v[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) v[u] = p[(m + u) * step];
+#pragma unroll
+            for (int u = 0; u < U; u++) add(lane_value(wl, m + u), v[u]);
         }
+        for (; m < cnt; m++) add(lane_value(wl, m), p[m * step]);
     }
     __shared__ double sh[3][256];
     sh[0][threadIdx.x] = acc;
@@ -166,32 +352,50 @@ __global__ __launch_bounds__(256) void region_sum_kernel(RegionArgs a)
     }
 }
 
-// one block per region: sums the chunks in order, divides by the weight sum
-// (normalizeExpectationValues, code/src/ObserverCPU.cpp:293-308) and writes
-// the record; block 0 also writes A and the min / max over k
+// grid (R, ceil(Qtot / 64)), 256 threads: four wavefronts sum every fourth chunk of
+// the block's quantities and of the weights, then divide by the weight sum
+// (normalizeExpectationValues, code/src/ObserverCPU.cpp:293-308) and write the
+// record; block 0 also writes A and the min / max over k
 __global__ __launch_bounds__(256) void region_final_kernel(RegionArgs a)
 {
     const int r = blockIdx.x;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int Qtot = a.Q + 1 + (a.density ? 2 * a.n * a.n : 0);
-    double ws = 0;
-    for (int c = 0; c < a.chunks; c++) ws += a.part[((long)r * a.chunks + c) * Qtot + a.Q];
-    double *out = a.rec + 3 + (long)r * a.rstride;
-    for (int q = threadIdx.x; q < Qtot; q += 256) {
-        double t = 0;
-        for (int c = 0; c < a.chunks; c++) t += a.part[((long)r * a.chunks + c) * Qtot + q];
-        out[q] = (q == a.Q) ? t : t / ws;
+    const int q = blockIdx.y * 64 + lane, qs = q < Qtot ? q : a.Q;
+    const double *part = a.part + (long)r * a.chunks * Qtot;
+    double t = 0, ws = 0;
+#pragma unroll 4
+    for (int c = wv; c < a.chunks; c += 4) {
+        t += part[(long)c * Qtot + qs];
+        ws += part[(long)c * Qtot + a.Q];
     }
-    if (r == 0) {
+    __shared__ double sh[2][256];
+    sh[0][threadIdx.x] = t;
+    sh[1][threadIdx.x] = ws;
+    __syncthreads();
+    if (wv == 0 && q < Qtot) {
+        for (int w2 = 1; w2 < 4; w2++) {
+            t += sh[0][lane + 64 * w2];
+            ws += sh[1][lane + 64 * w2];
+        }
+        a.rec[3 + (long)r * a.rstride + q] = (q == a.Q) ? t : t / ws;
+    }
+    if (r == 0 && blockIdx.y == 0) {
         if (threadIdx.x < 3) a.rec[threadIdx.x] = a.x[2 * threadIdx.x];
         double *mnmx = a.rec + 3 + (long)a.R * a.rstride;
-        for (int b = threadIdx.x; b < a.n; b += 256) {
-            double lo = INFINITY, hi = -INFINITY;
-            for (int c = 0; c < a.chunks; c++) {
-                lo = fmin(lo, a.pmin[(long)c * a.n + b]);
-                hi = fmax(hi, a.pmax[(long)c * a.n + b]);
+        // min by the first wavefront, max by the second: lane = band + 16 x (every fourth chunk)
+        const int b = lane & 15, c0 = lane >> 4;
+        if (wv < 2 && b < a.n) {
+            double v = wv ? -INFINITY : INFINITY;
+            for (int c = c0; c < a.chunks; c += 4) {
+                const double p = (wv ? a.pmax : a.pmin)[(long)c * a.n + b];
+                v = wv ? fmax(v, p) : fmin(v, p);
             }
-            mnmx[b] = lo;
-            mnmx[a.n + b] = hi;
+            for (int m = 16; m < 64; m <<= 1) {
+                const double o = __shfl_xor(v, m);
+                v = wv ? fmax(v, o) : fmin(v, o);
+            }
+            if (c0 == 0) mnmx[wv * a.n + b] = v;
         }
     }
 }
@@ -205,14 +409,18 @@ hipError_t launch_region_sums(const RegionArgs &a, hipStream_t s)
                        dim3(256), 0, s, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(region_final_kernel, dim3((unsigned)a.R), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(region_final_kernel, dim3((unsigned)a.R, (unsigned)((Qtot + 63) / 64)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
-hipError_t launch_observe_j_batched(const ObsArgs *d_args, const long *d_block0, int m, long blocks, hipStream_t s)
+hipError_t launch_observe_j_batched(int n, const ObsArgs *d_args, const long *d_block0, int m, long blocks,
+                                    hipStream_t s)
 {
     if (m <= 0 || blocks <= 0) return hipSuccess;
-    hipLaunchKernelGGL(jk_batched_kernel, dim3((unsigned)blocks), dim3(64), 0, s, d_args, d_block0, m);
+    const dim3 grid((unsigned)blocks), blk(64);
+    if (n > 8) hipLaunchKernelGGL(jk_rows_batched_kernel<16>, grid, blk, 0, s, d_args, d_block0, m);
+    else if (n > 4) hipLaunchKernelGGL(jk_rows_batched_kernel<8>, grid, blk, 0, s, d_args, d_block0, m);
+    else hipLaunchKernelGGL(jk_batched_kernel, grid, blk, 0, s, d_args, d_block0, m);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(jreduce_batched_kernel, dim3((unsigned)m), dim3(256), 0, s, d_args);

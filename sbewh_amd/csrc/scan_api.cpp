@@ -290,7 +290,7 @@ struct sbe_scan {
         std::vector<ObsArgs> oa(m);
         std::vector<long> b0(m);
         long tot = 0;
-        const int oc = output_count;
+        const int oc = output_count, kb = observe_block_k(n);
         for (int j = 0; j < m; j++) {
             sbe_ctx &c = *inst[ids[j]];
             StageInput in{};
@@ -308,14 +308,14 @@ struct sbe_scan {
             o.j_out = d_jout + 3 * ((long)ids[j] * oc + ctl[ids[j]].out);
             o.pstride = 3;
             b0[j] = tot;
-            tot += c.nk;
+            tot += (c.nk + kb - 1) / kb;
         }
         twiddles(tw, nullptr);
         partial(cs, E, inst[ids[0]]->obs_ops, true);
         ObsArgs *da = add(oa.data(), m);
         long *db = add(b0.data(), m);
         flush();
-        HIPCHK(launch_observe_j_batched(da, db, m, tot, stream));
+        HIPCHK(launch_observe_j_batched(n, da, db, m, tot, stream));
     }
 
     // one Dormand-Prince attempt of every listed instance; errors into h_err[j]

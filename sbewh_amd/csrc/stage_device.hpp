@@ -160,13 +160,40 @@ __device__ __forceinline__ V load_const(const void *p, unsigned i)
     return *(vptr)((cptr)(unsigned long long)p + (unsigned)(i * sizeof(V)));
 }
 
-// H(k) of operator op for layouts whose matrices fill whole wavefronts, into
-// registers: acc[kk N^2 / 64 + u] is entry threadIdx.x + 64 u (row-major, N x N) of k-point kk
-// (N >= 8: register u of a lane belongs to k-point kk = 64 u / N^2 for all 64
-// lanes): everything that depends on the k-point alone is wave-uniform, so the
-// phase map and the twiddles come through scalar loads, and a phase-sum row is
-// loaded once for all k-points of the wavefront that share it, QG cells in one
-// memory trip.  Consecutive k-points share rest(k) along a Fourier block's last
+// The next group of k-points of a wavefront that share a phase-sum row: takes them
+// out of todo (a bit per k-point) and returns their bits
+template <int KPW>
+__device__ __forceinline__ unsigned next_row_group(unsigned &todo, const int (&rest)[KPW], int &row)
+{
+    row = 0;
+#pragma unroll
+    for (int kk = KPW - 1; kk >= 0; kk--) row = (todo >> kk) & 1 ? rest[kk] : row;
+    unsigned mine = 0;
+#pragma unroll
+    for (int kk = 0; kk < KPW; kk++) mine |= (rest[kk] == row ? 1u : 0u) << kk;
+    mine &= todo;
+    todo &= ~mine;
+    return mine;
+}
+// phase map of the k-points k0 .. k0 + KPW - 1 (k0 wave-uniform): row and twiddle offset
+template <int KPW>
+__device__ __forceinline__ void phase_map(const PhaseLast &ph, long nk, int k0, int (&rest)[KPW], unsigned (&tp)[KPW])
+{
+#pragma unroll
+    for (int kk = 0; kk < KPW; kk++) {
+        const long k = (long)k0 + kk;
+        const si2 m = load_const<si2>(ph.kphase, (unsigned)(k < nk ? k : 0));
+        rest[kk] = m.x;
+        tp[kk] = m.y;
+    }
+}
+
+// One operator (entries off .. off + n n of an M-wide phase-sum row) of the k-points
+// k0 .. k0 + KPW - 1 into registers, for matrices that fill whole wavefronts (N >= 8):
+// acc[kk N^2 / 64 + u] is entry threadIdx.x + 64 u (row-major, N x N) of k-point kk.  A
+// register belongs to the same k-point in all 64 lanes, so the phase map and the
+// twiddles come through scalar loads, and a phase-sum row is loaded once for all
+// k-points of the wavefront that share it, QG cells in one memory trip.  Consecutive k-points share rest(k) along a Fourier block's last
 // axis, so a wavefront has one or two distinct rows; each gets a pass.
 // false, with nothing done, for an R box wider than 16 cells along the last
 // axis.  Sums in the order of phase_mats.
@@ -174,27 +201,20 @@ __device__ __forceinline__ V load_const(const void *p, unsigned i)
 // (104 in series for 8 bands and 13 cells) kept the 8-band kernel waiting; four
 // right-hand sides on 150 x 150 k, 8 bands: 362 -> 316 us, an integration there
 // 64.3 -> 54.3 ms; 48^3 k, 16 bands: 6.86 -> 6.66 ms.
-template <int N, int LR>
-__device__ __forceinline__ bool phase_rows(cd *acc, const StageArgs &a, int op, long blk)
+template <int N, int KPW>
+__device__ __forceinline__ bool phase_rows(cd *acc, const PhaseLast &ph, long nk, int n, int M, int off, long k0)
 {
-    using G = Geo<N, LR>;
-    static_assert(G::NN % 64 == 0, "a k-point's matrix fills whole wavefronts");
-    constexpr int EK = G::NN / 64;                 // entries per lane and k-point
-    constexpr int KPW = G::KPW, KT = KPW < 4 ? KPW : 4;
+    static_assert(N * N % 64 == 0, "a k-point's matrix fills whole wavefronts");
+    constexpr int EK = N * N / 64;                 // entries per lane and k-point
+    constexpr int KT = KPW < 4 ? KPW : 4;
     constexpr int QG = EK == 1 ? 4 : 2;            // cells per memory trip
-    const int n = a.n, nn = n * n, M = 2 * nn, WL = a.ph.WL;
+    const int WL = ph.WL;
     if (WL > 16) return false;
-    const int blkl = __builtin_amdgcn_readfirstlane((int)blk);
-    const double2 *Yb = reinterpret_cast<const double2 *>(a.ph.Y) + op * nn;
+    const int kf = __builtin_amdgcn_readfirstlane((int)k0);
+    const double2 *Yb = reinterpret_cast<const double2 *>(ph.Y) + off;
     int rest[KPW];
     unsigned tp[KPW];
-#pragma unroll
-    for (int kk = 0; kk < KPW; kk++) {
-        const long k = (long)blkl * KPW + kk;
-        const si2 ph = load_const<si2>(a.ph.kphase, (unsigned)(k < a.nk ? k : 0));
-        rest[kk] = ph.x;
-        tp[kk] = ph.y;
-    }
+    phase_map<KPW>(ph, nk, kf, rest, tp);
     // the lane's entries of a row: masked ones read entry 0 and are zeroed at the end
     int ent[EK];
     bool krc[EK];
@@ -210,15 +230,8 @@ __device__ __forceinline__ bool phase_rows(cd *acc, const StageArgs &a, int op, 
         for (int u = 0; u < EK; u++) acc[kk * EK + u] = mk(0, 0);
     unsigned todo = KPW >= 32 ? ~0u : (1u << KPW) - 1;
     while (todo) {
-        // the first k-point left, and those that share its row
-        int row = 0;
-#pragma unroll
-        for (int kk = KPW - 1; kk >= 0; kk--) row = (todo >> kk) & 1 ? rest[kk] : row;
-        unsigned mine = 0;
-#pragma unroll
-        for (int kk = 0; kk < KPW; kk++) mine |= (rest[kk] == row ? 1u : 0u) << kk;
-        mine &= todo;
-        todo &= ~mine;
+        int row;
+        const unsigned mine = next_row_group<KPW>(todo, rest, row);
         const double2 *yr = Yb + (long)row * M;
         // cell q of the row (entries y) into the sums of its k-points
         auto add_cell = [&](int q, const double2 *y) {
@@ -226,7 +239,7 @@ __device__ __forceinline__ bool phase_rows(cd *acc, const StageArgs &a, int op, 
             for (int k4 = 0; k4 < KPW; k4 += KT) {
                 sd2 tw[KT];
 #pragma unroll
-                for (int v = 0; v < KT; v++) tw[v] = load_const<sd2>(a.ph.twL, tp[k4 + v] + q);
+                for (int v = 0; v < KT; v++) tw[v] = load_const<sd2>(ph.twL, tp[k4 + v] + q);
 #pragma unroll
                 for (int v = 0; v < KT; v++)
                     if (KPW == 1 || ((mine >> (k4 + v)) & 1)) {
@@ -256,7 +269,7 @@ __device__ __forceinline__ bool phase_rows(cd *acc, const StageArgs &a, int op, 
     }
 #pragma unroll
     for (int kk = 0; kk < KPW; kk++) {
-        const bool kin = (long)blkl * KPW + kk < a.nk;
+        const bool kin = (long)kf + kk < nk;
 #pragma unroll
         for (int u = 0; u < EK; u++)
             if (!(kin && krc[u])) acc[kk * EK + u] = mk(0, 0);
@@ -271,7 +284,8 @@ __device__ __forceinline__ bool phase_mats_rows(cd *lds, const StageArgs &a, int
     using G = Geo<N, LR>;
     constexpr int EK = G::NN / 64;
     cd acc[G::KPW * EK];
-    if (!phase_rows<N, LR>(acc, a, op, blk)) return false;
+    const int nn = a.n * a.n;
+    if (!phase_rows<N, G::KPW>(acc, a.ph, a.nk, a.n, 2 * nn, op * nn, blk * G::KPW)) return false;
 #pragma unroll
     for (int kk = 0; kk < G::KPW; kk++)
 #pragma unroll
@@ -1458,7 +1472,7 @@ __device__ __forceinline__ void rhs_stage_body16q(const StageArgs &a, const long
     auto load = [&](const double *src, int j) { return reinterpret_cast<const double2 *>(src)[ent[j]]; };
     auto phase_acc = [&](int op, CAcc &h) {
         cd v[4];
-        if (!phase_rows<N, LR>(v, a, op, blk)) {
+        if (!phase_rows<N, 1>(v, a.ph, a.nk, n, 2 * nn, op * nn, k)) {
 #pragma unroll
             for (int j = 0; j < 4; j++) v[j] = own[j] ? phase_last(a.ph, k, 2 * nn, op * nn + ent[j]) : mk(0, 0);
         }
@@ -2077,6 +2091,18 @@ __device__ __forceinline__ void obs_h0_mats(cd *lds, const OccArgs &a, long blk)
 {
     using G = Geo<N, LR>;
     const int n = a.n;
+    if constexpr (N >= 8) {
+        constexpr int EK = G::NN / 64;
+        cd h[G::KPW * EK];
+        if (phase_rows<N, G::KPW>(h, a.ph, a.nk, n, a.M, 0, blk * G::KPW)) {
+#pragma unroll
+            for (int i = 0; i < G::KPW * EK; i++) {
+                const int idx = (threadIdx.x + 64 * i) % G::NN;
+                lds[i / EK * G::NN + sw<N>(idx / N, idx % N)] = h[i];
+            }
+            return;
+        }
+    }
     for (int e = threadIdx.x; e < G::KPW * G::NN; e += 64) {
         const int kk = e / G::NN, idx = e % G::NN;
         const int r = idx / N, c = idx % N;

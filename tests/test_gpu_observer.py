@@ -71,6 +71,35 @@ def test_observer_record_matches_oracle(name, smear_eV):
     g.close()
 
 
+# bands beside the padded sizes, wavefronts whose k-points lie in several
+# phase-sum rows, a last wavefront that is not full, an R box wider than 16
+# cells, more than one chunk of k (and with many regions, larger chunks)
+@pytest.mark.parametrize("n,ext,Nk,Nf,regions", [
+    (5, (1, 1), (6, 9), (3, 3), 1), (8, (1, 2), (5, 10), (5, 5), 2), (7, (1, 8), (3, 18), (3, 18), 1),
+    (9, (1, 1), (6, 3), (3, 3), 2), (11, (1, 3), (3, 8), (3, 8), 1), (16, (1, 8), (3, 18), (3, 18), 1),
+    (3, (1, 1), (27, 27), (3, 3), 3), (2, (1, 1), (24, 24), (3, 3), 2100)])
+def test_observer_edges(n, ext, Nk, Nf, regions):
+    from tests.test_gpu_stage_kernels import config
+    cfg = config(n, ext, Nk, Nf)
+    say(f"[gpu] full observer n={n} R extents {ext} k {Nk} {regions} regions")
+    g, o = SBEContext(cfg), Oracle(cfg)
+    x = cases.perturbed_state(o.initial_state(0.0), o.n, o.P, o.num_k, seed=9, amp=0.05)
+    regs = [WHOLE_ZONE] + [Region((0.001 * i, 0.3, 0.0), 0.3, i % 2 == 0, "r") for i in range(regions - 1)]
+    ob = FullObserver(g, regs, smearing_width=0.01, density_stride=1, capacity=2)
+    ob.record(x, 2.0)
+    r = ob.collectExpectationValues()
+    ref = o.observe_full(x, as_tuples(regs), 0.01, density=True)
+    for key, rk in (("kPointWeightSum", "weight_sum"), ("j", "j"), ("occupationHam", "occ_ham"),
+                    ("occupationWan", "occ_wan"), ("occupationHamMin", "occ_min"), ("occupationHamMax", "occ_max"),
+                    ("wan", "wan")):
+        ok, err = close(r[key][0], ref[rk], 1e-12)
+        assert ok, (key, err)
+    assert close(g.observe(x), ref["j"][0], 1e-12)[0]
+    ob.close()
+    g.close()
+    o.close()
+
+
 def test_observer_density_stride_and_capacity():
     cfg = cases.chain(sweeps=8)
     g = SBEContext(cfg)
