@@ -219,6 +219,46 @@ struct sbe_ctx {
         return mm;
     }
 
+    // 1-D chains of two bands run in registers, a lane per matrix entry
+    // (chain_kernels.hip), with no layout to tune and no eigenvector cache: a
+    // quarter to half of the general path's time on 256 k, and a smaller share of
+    // it the larger the grid.  A sweep bound of 0 (no rotation after the first
+    // call) and a layout forced through SBEWH_STAGE_LR keep the general path;
+    // decided at the first use, as the layout is.
+    int chain_mode = -1;
+    bool chain()
+    {
+        if (chain_mode < 0) {
+            chain_mode = dim == 1 && n == 2 && prm.sweep_count > 0 && !lr;
+            int lrs[8];
+            if (const char *env = std::getenv("SBEWH_STAGE_LR"))
+                for (int v = 0, nv = stage_variants(N, lrs, 8); v < nv; v++)
+                    if (lrs[v] == std::atoi(env)) chain_mode = 0;
+        }
+        return chain_mode == 1;
+    }
+    ChainArgs chain_args() const
+    {
+        ChainArgs c{};
+        c.P = P;
+        c.nk = nk;
+        c.W = geom.W[0];
+        c.rmin = geom.rmin[0];
+        c.Nk = geom.Nk[0];
+        for (int d = 0; d < 3; d++) {
+            c.a0[d] = geom.lattice[d];
+            c.kshift_au[d] = geom.kshift_au[d];
+        }
+        c.Hb = Hb;
+        c.Db = Db;
+        c.dHb = dHb;
+        c.kphase = kphase;
+        c.F2 = prm.relaxation_F2;
+        c.w = prm.soothing_width;
+        c.dephase = prm.relaxation_F2 > 0;
+        return c;
+    }
+
     // dxdt = f(rho_in, t) on device with rho_in = in.x + sum_j in.c[j] in.k[j];
     // xout (optional) receives rho_in
     void rhs_dev(const StageInput &in, double *dxdt, double t, hipStream_t s, double *xout = nullptr)
@@ -329,13 +369,29 @@ struct sbe_ctx {
 
     void rhs_dev(const double *x_in, double *dxdt, double t, hipStream_t s)
     {
+        if (chain()) {
+            double E[3];
+            E_at(t, E);
+            HIPCHK(launch_chain_rhs(chain_args(), x_in, dxdt, E[0], s));
+            rhs_calls++;
+            return;
+        }
         StageInput in{};
         in.x = x_in;
         rhs_dev(in, dxdt, t, s);
     }
 
-    void observe_dev(const double *xs, double *jdst, hipStream_t s)
+    // j of xs into jdst; with k1 also the first derivative of the interval that
+    // starts there at time t, if it can share the launch (returns whether it did)
+    bool observe_dev(const double *xs, double *jdst, hipStream_t s, double *k1 = nullptr, double t = 0)
     {
+        if (chain()) {
+            double E[3] = {0, 0, 0};
+            if (k1) E_at(t, E);
+            HIPCHK(launch_chain_output(chain_args(), xs, jdst, partial, k1, E[0], err_ticket, s));
+            if (k1) rhs_calls++;
+            return k1 != nullptr;
+        }
         StageInput in{};
         in.x = xs;
         HIPCHK(launch_twiddles(geom, &in, 1, tw, s));
@@ -351,6 +407,7 @@ struct sbe_ctx {
         o.j_out = jdst;
         o.pstride = 3;
         HIPCHK(launch_observe_j(o, s));
+        return false;
     }
 
     // one Dormand-Prince attempt from (x, k1, t, dt) -> xn, k7; returns the error norm.
@@ -382,6 +439,31 @@ struct sbe_ctx {
         for (int q = 0; q < 6; q++) E_at(ts[q], E[q]);
         // error coefficients of k1, k3, k4, k5, k6, k7
         const double err_e[6] = {dt * DC1, dt * DC3, dt * DC4, dt * DC5, dt * DC6, dt * DC7};
+        if (chain()) {
+            ChainAttempt a{};
+            a.x = X;
+            a.k1 = k1;
+            a.xn = xn;
+            a.k7 = k7;
+            for (int q = 0; q < 6; q++) {
+                for (int j = 0; j < ins[q].nt; j++) a.c[q][j] = ins[q].c[j];
+                a.E[q] = E[q][0];
+                a.err_e[q] = err_e[q];
+            }
+            a.ea = prm.eps_abs;
+            a.er = prm.eps_rel;
+            a.dt = dt;
+            a.partial = err_partial;
+            a.ticket = err_ticket;
+            a.err_out = err_host_dev;
+            *reinterpret_cast<volatile unsigned long long *>(err_host) = ERR_PENDING;
+            // (timing: no phase sum of its own)
+            for (int e = 0; timing && e < 2; e++) HIPCHK(hipEventRecord(next_event(), s));
+            HIPCHK(launch_chain_attempt(chain_args(), a, s));
+            if (timing) HIPCHK(hipEventRecord(next_event(), s));
+            rhs_calls += 6;
+            return wait_error(s);
+        }
         const long blocks = lr ? (nk + stage_k_per_block(N, lr) - 1) / stage_k_per_block(N, lr) : 0;
         const bool fused = lr && !timing && blocks < fuse_below_blocks;
         // the last kernel of the attempt overwrites this with the norm

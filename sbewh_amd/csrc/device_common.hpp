@@ -30,6 +30,16 @@ __device__ __forceinline__ cd cfma_jc(cd a, cd b, cd acc)
 {
     return cd{fma(a.x, b.x, fma(a.y, b.y, acc.x)), fma(-a.x, b.y, fma(a.y, b.x, acc.y))};
 }
+// 1/sqrt(x) for a positive normal x: the hardware estimate and one
+// second-order correction y (1 + e/2 + 3 e^2/8), e = 1 - x y^2 (the device
+// library's rsqrt without its handling of zero, infinity and NaN)
+__device__ __forceinline__ double rsqrt_pos(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
 // Relative error term of one state entry of a Dormand-Prince attempt,
 //   |sum_j e[j] k_j| / (ea + er (|x| + dt |k_0|)),  k_0..k_5 = k1, k3, k4, k5, k6, k7
 // (the controller's error checker, code/src/main/runSBE.cpp:178-180 via

@@ -236,6 +236,36 @@ hipError_t launch_error_final(const double *partial, long nb, unsigned long long
 hipError_t launch_error_final_batched(const long *d_block0, int m, long blocks, const double *partial, double *out,
                                      hipStream_t s);
 
+// ---- 1-D chains of two bands (chain_kernels.hip) ---------------------------
+struct ChainArgs {
+    int P;
+    long nk;
+    int W, rmin, Nk;                  // R box and k-grid along the chain
+    double a0[3], kshift_au[3];       // lattice vector, k shift
+    const double *Hb, *Db, *dHb;      // [W][4]: H, r_0, i R_0 H
+    const int *kphase;                // int2 per k: (., i W)
+    double F2, w;
+    int dephase;
+};
+hipError_t launch_chain_rhs(const ChainArgs &c, const double *x, double *dxdt, double E, hipStream_t s);
+// j(t) of x into j[3]; with k1 also the derivative of x.  partial: one double per
+// block of 16 k-points; ticket: zero between launches
+hipError_t launch_chain_output(const ChainArgs &c, const double *x, double *j, double *partial, double *k1, double E,
+                               unsigned *ticket, hipStream_t s);
+// One Dormand-Prince attempt: stage q reads x + sum_j c[q][j] k_j (k_1 .. k_{q+1};
+// k_1, k_3 .. k_6 for q = 5) in the field E[q]; x_new, k7 and the error norm (as
+// StageSet: err_e of k_1, k_3 .. k_7) come out, the other derivatives stay inside.
+struct ChainAttempt {
+    const double *x, *k1;
+    double *xn, *k7;
+    double c[6][5], E[6];
+    double err_e[6], ea, er, dt;
+    double *partial;
+    unsigned *ticket;
+    unsigned long long *err_out;
+};
+hipError_t launch_chain_attempt(const ChainArgs &c, const ChainAttempt &a, hipStream_t s);
+
 // ---- observer (observer_kernels.hip) -------------------------------------
 struct ObsArgs {
     const double *x;       // state

@@ -239,8 +239,11 @@ bool resident_integrate(sbe_ctx &c, int output_count, std::vector<double> &tv, l
     if (!c.lr) {
         // the layout tuner runs on a first stage (not part of the integration)
         const long calls = c.rhs_calls;
-        c.rhs_dev(c.x(), c.st[1], c.t_start(), c.stream);
+        StageInput in{};
+        in.x = c.x();
+        c.rhs_dev(in, c.st[1], c.t_start(), c.stream);
         c.rhs_calls = calls;
+        c.ucache_valid = false;
     }
     const long kpb = stage_k_per_block(c.N, c.lr), blocks = (c.nk + kpb - 1) / kpb;
     if (blocks > resident_max_blocks(c.N, c.lr)) return false;
@@ -370,19 +373,21 @@ long sbe_host::integrate_impl(sbe_ctx *ctx, double *state, int output_count, dou
         int out = 0, rp = 0;
         std::vector<double> tv;
         while (less_eq_with_sign(time + dt_out, t_end)) {
+            bool first = true;
             if (out < output_count) {
                 tv.push_back(time);
-                c.observe_dev(c.x(), c.jbuf + 3 * out, c.stream);
+                // (the interval's first derivative may come with the output)
+                first = !c.observe_dev(c.x(), c.jbuf + 3 * out, c.stream,
+                                       replay || less_with_sign(time, time + dt_out) ? c.st[1] : nullptr, time);
                 if (obs) obs->record_dev(c.x(), time, c.stream);
             }
             out++;
             double start = time, end = time + dt_out;
-            bool first = true;
             int fails = 0;
             if (replay) {
                 // replay: the logged accepted attempts whose start lies in this
                 // output interval, with the logged (t, dt)
-                c.rhs_dev(c.x(), c.st[1], start, c.stream);
+                if (first) c.rhs_dev(c.x(), c.st[1], start, c.stream);
                 const double tol = 1e-9 * std::max(1.0, std::fabs(end));
                 for (;;) {
                     while (rp < replay->count && rp < replay->capacity && !replay->accepted[rp]) rp++;
@@ -550,20 +555,20 @@ int sbe_bench_steps(sbe_ctx *ctx, const double *state, double t, double dt, int 
         if (rhs) *rhs = c.rhs_calls - r0;
         // optional second pass: per-kernel durations from events around each launch
         if (stage_ms || phase_ms) {
+            const long r1 = c.rhs_calls;
             c.timing = true;
             c.evused = 0;
             run(std::min(steps, 20));
             HIPCHK(hipStreamSynchronize(c.stream));
             c.timing = false;
             double sm = 0, pm = 0;
-            long nr = 0;
+            const long nr = c.rhs_calls - r1;
             for (size_t e = 0; e + 2 < c.evused; e += 3) {
                 float a = 0, b = 0;
                 HIPCHK(hipEventElapsedTime(&a, c.evpool[e], c.evpool[e + 1]));
                 HIPCHK(hipEventElapsedTime(&b, c.evpool[e + 1], c.evpool[e + 2]));
                 pm += a;
                 sm += b;
-                nr++;
             }
             if (stage_ms) *stage_ms = nr ? sm / nr : 0;
             if (phase_ms) *phase_ms = nr ? pm / nr : 0;

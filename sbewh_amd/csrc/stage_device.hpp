@@ -805,16 +805,6 @@ __device__ __forceinline__ void cacc_store(cd *lds, const CAcc &c)
     for (int j = 0; j < 4; j++) lds[sw<16>(cacc_row(j), cacc_col())] = mk(c.r[j], c.i[j]);
 }
 
-// 1/sqrt(x) for a positive normal x: the hardware estimate and one
-// second-order correction y (1 + e/2 + 3 e^2/8), e = 1 - x y^2 (the device
-// library's rsqrt without its handling of zero, infinity and NaN)
-__device__ __forceinline__ double rsqrt_pos(double x)
-{
-    const double y = __builtin_amdgcn_rsq(x);
-    const double e = fma(-x * y, y, 1.0);
-    return fma(y * e, fma(e, 0.375, 0.5), y);
-}
-
 // an optimisation barrier: the N accumulators are complete here, and no
 // memory access moves across it (keeps a product's loads per step bounded)
 template <int N>
