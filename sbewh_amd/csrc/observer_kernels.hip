@@ -14,20 +14,21 @@
 
 namespace sbe {
 
-// The per-k current for matrices that fill wavefronts (N = 8, 16): KB consecutive
-// k-points per wavefront.  Lane entry (a, b) of a k-point's matrices holds T_ba and
+// The per-k current for 16 bands: KB consecutive k-points per wavefront, in the
+// accumulator layout.  Lane entry (a, b) of a k-point's matrices holds T_ba and
 // rho_ba, and the sum over (a, b) goes before the one over the last axis' cells r,
 //   j_d = Re sum_r tw_r sum_ab [ i D_d(r)_ab T_ba - dH_d(r)_ab rho_ba ],
 // so a phase-sum entry is loaded once for all k-points of its row and no operator
 // is formed.  One k-point per wavefront read (1 + 2 dim) n n W_L entries from L2 and
-// as many twiddles per k-point: @JK@.
-template <int N>
-constexpr int jk_block_k() { return N == 16 ? 2 : 8; }
+// as many twiddles per k-point: 24^3 k 375 -> 125 us (KB 2; 3: 114, 4: 152 and two
+// waves per SIMD).  Up to 8 bands keep a wavefront per k-point: the same with 8 or
+// 2 k-points per wavefront took 49 us instead of 61 on 150 x 150 k, but 43 and 23
+// instead of 11 on 15 x 15, the latency of one wavefront.
+constexpr int JK_KB = 2;
 
-template <int N>
 __device__ __forceinline__ void jk_rows_body(const ObsArgs &a, const long blk)
 {
-    constexpr int KB = jk_block_k<N>(), EK = N * N / 64;
+    constexpr int N = 16, KB = JK_KB, EK = N * N / 64;
     const int n = a.n, nn = n * n, M = (1 + 2 * a.dim) * nn, WL = a.ph.WL;
     const int k0 = __builtin_amdgcn_readfirstlane((int)blk) * KB;
     int ent[EK];
@@ -56,58 +57,37 @@ __device__ __forceinline__ void jk_rows_body(const ObsArgs &a, const long blk)
             R[kk * EK + u] = in ? mk(v.x, v.y) : mk(0, 0);
         }
     // T = H0 rho - rho H0, then T and rho transposed
-    if constexpr (N == 16) {
-        __shared__ cd B0[ACC_MS], B1[ACC_MS];
-        const AccPos pos = acc_pos();
+    __shared__ cd B0[ACC_MS], B1[ACC_MS];
+    const AccPos pos = acc_pos();
 #pragma unroll
-        for (int kk = 0; kk < KB; kk++) {
-            cd *h = H + kk * EK, *r = R + kk * EK, x[4], y[4];
+    for (int kk = 0; kk < KB; kk++) {
+        cd *h = H + kk * EK, *r = R + kk * EK, x[4], y[4];
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                B0[pos.nat + 4 * ACC_RS * j] = h[j];
-                B1[pos.nat + 4 * ACC_RS * j] = r[j];
-            }
-            wsync();
-            CAcc t;
-            cacc_zero(t);
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                x[j] = B0[pos.tr + 4 * j];
-                y[j] = B1[pos.tr + 4 * j];
-            }
-            mfma_cmul(x, r, t);
-#pragma unroll
-            for (int j = 0; j < 4; j++) x[j] = mk(-y[j].x, -y[j].y);
-            mfma_cmul(x, h, t);
-            wsync();
-            acc_put(B0, pos, t);
-            wsync();
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                T[kk * EK + j] = B0[pos.tr + 4 * j];
-                r[j] = y[j];
-            }
-            wsync();
+        for (int j = 0; j < 4; j++) {
+            B0[pos.nat + 4 * ACC_RS * j] = h[j];
+            B1[pos.nat + 4 * ACC_RS * j] = r[j];
         }
-    } else {
-        __shared__ cd Hs[N * (N + 1)], Rs[N * (N + 1)];
-        const int ra = threadIdx.x / N, cb = threadIdx.x % N;
+        wsync();
+        CAcc t;
+        cacc_zero(t);
 #pragma unroll
-        for (int kk = 0; kk < KB; kk++) {
-            Hs[ra * (N + 1) + cb] = H[kk];
-            Rs[ra * (N + 1) + cb] = R[kk];
-            wsync();
-            cd t = mk(0, 0);  // T[b][a]
-#pragma unroll
-            for (int l = 0; l < N; l++) {
-                const cd rb = Rs[cb * (N + 1) + l];
-                t = cfma(Hs[cb * (N + 1) + l], Rs[l * (N + 1) + ra], t);
-                t = cfma(mk(-rb.x, -rb.y), Hs[l * (N + 1) + ra], t);
-            }
-            T[kk] = t;
-            R[kk] = Rs[cb * (N + 1) + ra];
-            wsync();
+        for (int j = 0; j < 4; j++) {
+            x[j] = B0[pos.tr + 4 * j];
+            y[j] = B1[pos.tr + 4 * j];
         }
+        mfma_cmul(x, r, t);
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[j] = mk(-y[j].x, -y[j].y);
+        mfma_cmul(x, h, t);
+        wsync();
+        acc_put(B0, pos, t);
+        wsync();
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            T[kk * EK + j] = B0[pos.tr + 4 * j];
+            r[j] = y[j];
+        }
+        wsync();
     }
     int rest[KB];
     unsigned tp[KB];
@@ -161,21 +141,19 @@ __device__ __forceinline__ void jk_rows_body(const ObsArgs &a, const long blk)
         }
 }
 
-template <int N>
 __global__ __launch_bounds__(64) void jk_rows_kernel(ObsArgs a)
 {
-    jk_rows_body<N>(a, xcd_block(blockIdx.x, gridDim.x));
+    jk_rows_body(a, xcd_block(blockIdx.x, gridDim.x));
 }
 
 __global__ __launch_bounds__(64) void jk_kernel(ObsArgs a) { jk_body(a, blockIdx.x); }
 
 // entry j owns blocks [block0[j], block0[j] + ceil(nk_j / observe_block_k))
-template <int N>
 __global__ __launch_bounds__(64) void jk_rows_batched_kernel(const ObsArgs *args, const long *block0, int m)
 {
     const long gb = xcd_block(blockIdx.x, gridDim.x);
     const int j = find_entry_wave(block0, m, gb);
-    jk_rows_body<N>(args[j], gb - block0[j]);
+    jk_rows_body(args[j], gb - block0[j]);
 }
 
 __global__ __launch_bounds__(64) void jk_batched_kernel(const ObsArgs *args, const long *block0, int m)
@@ -186,14 +164,13 @@ __global__ __launch_bounds__(64) void jk_batched_kernel(const ObsArgs *args, con
     jk_body(a, gb - block0[j]);
 }
 
-int observe_block_k(int n) { return n > 8 ? jk_block_k<16>() : n > 4 ? jk_block_k<8>() : 1; }
+int observe_block_k(int n) { return n > 8 ? JK_KB : 1; }
 
 static hipError_t launch_jk(const ObsArgs &a, hipStream_t s)
 {
     const int kb = observe_block_k(a.n);
     const dim3 grid((unsigned)((a.nk + kb - 1) / kb)), blk(64);
-    if (a.n > 8) hipLaunchKernelGGL(jk_rows_kernel<16>, grid, blk, 0, s, a);
-    else if (a.n > 4) hipLaunchKernelGGL(jk_rows_kernel<8>, grid, blk, 0, s, a);
+    if (a.n > 8) hipLaunchKernelGGL(jk_rows_kernel, grid, blk, 0, s, a);
     else hipLaunchKernelGGL(jk_kernel, grid, blk, 0, s, a);
     return hipGetLastError();
 }
@@ -418,8 +395,7 @@ hipError_t launch_observe_j_batched(int n, const ObsArgs *d_args, const long *d_
 {
     if (m <= 0 || blocks <= 0) return hipSuccess;
     const dim3 grid((unsigned)blocks), blk(64);
-    if (n > 8) hipLaunchKernelGGL(jk_rows_batched_kernel<16>, grid, blk, 0, s, d_args, d_block0, m);
-    else if (n > 4) hipLaunchKernelGGL(jk_rows_batched_kernel<8>, grid, blk, 0, s, d_args, d_block0, m);
+    if (n > 8) hipLaunchKernelGGL(jk_rows_batched_kernel, grid, blk, 0, s, d_args, d_block0, m);
     else hipLaunchKernelGGL(jk_batched_kernel, grid, blk, 0, s, d_args, d_block0, m);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
