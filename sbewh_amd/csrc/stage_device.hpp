@@ -116,6 +116,38 @@ __device__ __forceinline__ void for_chunks(F &&f)
 // wave-local sync: blocks are exactly one wavefront
 __device__ __forceinline__ void wsync() { __syncthreads(); }
 
+// Entry i of a lane in the wavefront's KPW matrices (consecutive lanes, consecutive
+// entries).  A matrix that fills whole wavefronts (N >= 8) has the same k-point
+// in all lanes and a fixed row and column per lane, so its addresses are a scalar
+// base and one lane offset.
+template <int N>
+struct Entry {
+    int kk, r, c;
+    __device__ __forceinline__ explicit Entry(int i)
+    {
+        if constexpr (N * N >= 64) {
+            const int idx = threadIdx.x + 64 * i % (N * N);
+            kk = 64 * i / (N * N);
+            r = idx / N;
+            c = idx % N;
+        } else {
+            const int e = threadIdx.x + 64 * i, idx = e % (N * N);
+            kk = e / (N * N);
+            r = idx / N;
+            c = idx % N;
+        }
+    }
+    // inside the n x n matrix; its index there, or a valid one
+    __device__ __forceinline__ bool in(int n) const { return r < n && c < n; }
+    __device__ __forceinline__ int at(int n) const { return in(n) ? r * n + c : 0; }
+};
+// first k-point of logical block blk (wave-uniform)
+template <int N, int LR>
+__device__ __forceinline__ long first_k(long blk)
+{
+    return (long)__builtin_amdgcn_readfirstlane((int)blk) * Geo<N, LR>::KPW;
+}
+
 // coalesced copy of the wave's KPW matrices (n x n at src + k*stride + off,
 // complex) into LDS natural layout [kk][N][N], zero padded.
 template <int N, int LR, class Lay = SwLay<N>, int CHUNK = Lay::CHUNK>
@@ -125,25 +157,21 @@ __device__ __forceinline__ void load_mats(cd *lds, const double *src, long strid
     constexpr int IT = G::KPW * G::NN / 64;  // entries per lane
     constexpr int CH = N >= 16 ? 4 : (CHUNK < IT ? CHUNK : IT);     // entries whose loads are in flight together
     const double2 *s2 = reinterpret_cast<const double2 *>(src);
-    // unconditional loads (masked entries read entry `off` of k-point 0)
+    const long k0 = first_k<N, LR>(blk);
+    // unconditional loads (masked entries read entry `off` of a k-point)
     for_chunks<IT, CH>([&](auto i0c) {
         constexpr int i0 = decltype(i0c)::value;
         double2 v[CH];
-        bool ok[CH];
 #pragma unroll
         for (int u = 0; u < CH; u++) {
-            const int e = threadIdx.x + 64 * (i0 + u);
-            const int kk = e / G::NN, idx = e % G::NN;
-            const int a = idx / N, b = idx % N;
-            const long k = blk * G::KPW + kk;
-            ok[u] = a < n && b < n && k < nk;
-            v[u] = s2[ok[u] ? k * stride + off + a * n + b : off];
+            const Entry<N> e(i0 + u);
+            const long k = k0 + e.kk;
+            v[u] = (s2 + ((k < nk ? k : 0) * stride + off))[e.at(n)];
         }
 #pragma unroll
         for (int u = 0; u < CH; u++) {
-            const int e = threadIdx.x + 64 * (i0 + u);
-            const int idx = e % G::NN;
-            lds[(e / G::NN) * Lay::MS + Lay::at(idx / N, idx % N)] = ok[u] ? mk(v[u].x, v[u].y) : mk(0, 0);
+            const Entry<N> e(i0 + u);
+            lds[e.kk * Lay::MS + Lay::at(e.r, e.c)] = e.in(n) && k0 + e.kk < nk ? mk(v[u].x, v[u].y) : mk(0, 0);
         }
     });
 }
@@ -513,25 +541,19 @@ __device__ __forceinline__ void load_rho_nt(cd *lds, const StageArgs &a, long bl
         src[j + 1] = reinterpret_cast<const double2 *>(in.k[j]);
         cf[j + 1] = in.c[j];
     }
+    const long k0 = first_k<N, LR>(blk);
     for_chunks<IT, CH>([&](auto i0c) {
         constexpr int i0 = decltype(i0c)::value;
-        long idx_[CH];
-        bool ok[CH];
-#pragma unroll
-        for (int u = 0; u < CH; u++) {
-            const int e = threadIdx.x + 64 * (i0 + u);
-            const int kk = e / G::NN, idx = e % G::NN;
-            const int r = idx / N, c = idx % N;
-            const long k = blk * G::KPW + kk;
-            ok[u] = r < n && c < n && k < a.nk;
-            // masked entries read state entry 8 (valid) and are zeroed at the end
-            idx_[u] = ok[u] ? 8 + k * a.P + r * n + c : 8;
-        }
+        // masked entries read a valid entry and are zeroed at the end
         double2 v[NT + 1][CH];
 #pragma unroll
         for (int j = 0; j <= NT; j++)
 #pragma unroll
-            for (int u = 0; u < CH; u++) v[j][u] = src[j][idx_[u]];
+            for (int u = 0; u < CH; u++) {
+                const Entry<N> e(i0 + u);
+                const long k = k0 + e.kk;
+                v[j][u] = (src[j] + (8 + (k < a.nk ? k : 0) * a.P))[e.at(n)];
+            }
 #pragma unroll
         for (int u = 0; u < CH; u++) {
             double re = v[0][u].x, im = v[0][u].y;
@@ -540,9 +562,8 @@ __device__ __forceinline__ void load_rho_nt(cd *lds, const StageArgs &a, long bl
                 re += cf[j] * v[j][u].x;
                 im += cf[j] * v[j][u].y;
             }
-            const int e = threadIdx.x + 64 * (i0 + u);
-            const int idx = e % G::NN;
-            lds[(e / G::NN) * Lay::MS + Lay::at(idx / N, idx % N)] = ok[u] ? mk(re, im) : mk(0, 0);
+            const Entry<N> e(i0 + u);
+            lds[e.kk * Lay::MS + Lay::at(e.r, e.c)] = e.in(n) && k0 + e.kk < a.nk ? mk(re, im) : mk(0, 0);
         }
     });
 }
@@ -568,44 +589,37 @@ __device__ __forceinline__ void load_rho(cd *lds, const StageArgs &a, long blk)
     const StageInput &in = a.in;
     constexpr int IT = G::KPW * G::NN / 64;  // entries per lane
     constexpr int CH = N >= 16 ? 4 : (Lay::CHUNK < IT ? Lay::CHUNK : IT);     // entries whose loads are in flight together
+    const long k0 = first_k<N, LR>(blk);
     for_chunks<IT, CH>([&](auto i0c) {
         constexpr int i0 = decltype(i0c)::value;
-        long idx_[CH];
-        bool ok[CH];
-#pragma unroll
-        for (int u = 0; u < CH; u++) {
-            const int e = threadIdx.x + 64 * (i0 + u);
-            const int kk = e / G::NN, idx = e % G::NN;
-            const int r = idx / N, c = idx % N;
-            const long k = blk * G::KPW + kk;
-            ok[u] = r < n && c < n && k < a.nk;
-            // masked entries read state entry 8 (valid) and are zeroed at the end
-            idx_[u] = ok[u] ? 8 + k * a.P + r * n + c : 8;
-        }
+        // masked entries read a valid entry and are zeroed at the end
+        auto load = [&](const double *src, int u) {
+            const Entry<N> e(i0 + u);
+            const long k = k0 + e.kk;
+            return (reinterpret_cast<const double2 *>(src) + (8 + (k < a.nk ? k : 0) * a.P))[e.at(n)];
+        };
         double re[CH], im[CH];
 #pragma unroll
         for (int u = 0; u < CH; u++) {
-            const double2 xv = reinterpret_cast<const double2 *>(in.x)[idx_[u]];
+            const double2 xv = load(in.x, u);
             re[u] = xv.x;
             im[u] = xv.y;
         }
 #pragma unroll
         for (int j = 0; j < 6; j++)
             if (j < in.nt) {
-                const double2 *kj = reinterpret_cast<const double2 *>(in.k[j]);
                 const double cj = in.c[j];
 #pragma unroll
                 for (int u = 0; u < CH; u++) {
-                    const double2 kv = kj[idx_[u]];
+                    const double2 kv = load(in.k[j], u);
                     re[u] += cj * kv.x;
                     im[u] += cj * kv.y;
                 }
             }
 #pragma unroll
         for (int u = 0; u < CH; u++) {
-            const int e = threadIdx.x + 64 * (i0 + u);
-            const int idx = e % G::NN;
-            lds[(e / G::NN) * Lay::MS + Lay::at(idx / N, idx % N)] = ok[u] ? mk(re[u], im[u]) : mk(0, 0);
+            const Entry<N> e(i0 + u);
+            lds[e.kk * Lay::MS + Lay::at(e.r, e.c)] = e.in(n) && k0 + e.kk < a.nk ? mk(re[u], im[u]) : mk(0, 0);
         }
     });
 }
@@ -617,15 +631,22 @@ __device__ __forceinline__ void store_state(double *dst, const cd *lds, int n, i
 {
     using G = Geo<N, LR>;
     const int nn = n * n;
-    const long k0 = blk * G::KPW;
-    for (int e = threadIdx.x; e < G::KPW * P; e += 64) {
-        int kk = e / P, p = e % P;
-        long k = k0 + kk;
-        if (k >= nk) break;
-        cd v = mk(0, 0);
-        if (p < nn) v = lds[kk * Lay::MS + Lay::at(p / n, p % n)];
-        reinterpret_cast<double2 *>(dst)[8 + k * P + p] = make_double2(v.x, v.y);
+    const long k0 = first_k<N, LR>(blk);
+    double2 *d2 = reinterpret_cast<double2 *>(dst) + 8;
+#pragma unroll
+    for (int i = 0; i < G::KPW * G::NN / 64; i++) {
+        const Entry<N> e(i);
+        const long k = k0 + e.kk;
+        if (k < nk && e.in(n)) {
+            const cd v = lds[e.kk * Lay::MS + Lay::at(e.r, e.c)];
+            (d2 + k * P)[e.at(n)] = make_double2(v.x, v.y);
+        }
     }
+    if (P > nn)
+        for (int t = threadIdx.x; t < G::KPW * (P - nn); t += 64) {
+            const long k = k0 + t / (P - nn);
+            if (k < nk) d2[k * P + nn + t % (P - nn)] = make_double2(0.0, 0.0);
+        }
 }
 
 // out[c] = sum_l X[i][l] Y[l][j_c] with X, Y in LDS (natural layout);
@@ -1009,14 +1030,14 @@ __device__ __forceinline__ void store_ucache(const StageArgs &a, const cd *lds, 
 {
     using G = Geo<N, LR>;
     const int n = a.n, nn = n * n;
+    const long k0 = first_k<N, LR>(blk);
 #pragma unroll
-    for (int e = threadIdx.x; e < G::KPW * G::NN; e += 64) {
-        const int kk = e / G::NN, idx = e % G::NN;
-        const int r = idx / N, c = idx % N;
-        const long k = blk * G::KPW + kk;
-        if (r < n && c < n && k < a.nk) {
-            const cd v = lds[kk * Lay::MS + Lay::at(r, c)];
-            reinterpret_cast<double2 *>(a.ucache)[k * nn + r * n + c] = make_double2(v.x, v.y);
+    for (int i = 0; i < G::KPW * G::NN / 64; i++) {
+        const Entry<N> e(i);
+        const long k = k0 + e.kk;
+        if (k < a.nk && e.in(n)) {
+            const cd v = lds[e.kk * Lay::MS + Lay::at(e.r, e.c)];
+            (reinterpret_cast<double2 *>(a.ucache) + k * nn)[e.at(n)] = make_double2(v.x, v.y);
         }
     }
 }
@@ -1043,23 +1064,23 @@ __device__ __forceinline__ double stage_err(const StageArgs &a, const cd *lds, l
 {
     using G = Geo<N, LR>;
     const int n = a.n;
-    const long k0 = blk * G::KPW;
-    const double2 *x2 = reinterpret_cast<const double2 *>(a.in.x);
+    const long k0 = first_k<N, LR>(blk);
     double v = 0;
     constexpr int IT = G::KPW * G::NN / 64;
 #pragma unroll 2
     for (int u = 0; u < IT; u++) {
-        const int e = threadIdx.x + 64 * u;
-        const int kk = e / G::NN, idx = e % G::NN, r = idx / N, c = idx % N;
-        const long k = k0 + kk;
-        if (r < n && c < n && k < a.nk) {
-            const long i = 8 + k * a.P + r * n + c;
+        const Entry<N> e(u);
+        const long k = k0 + e.kk;
+        if (e.in(n) && k < a.nk) {
+            auto load = [&](const double *src) {
+                return (reinterpret_cast<const double2 *>(src) + (8 + k * a.P))[e.at(n)];
+            };
             double2 kv[6];
 #pragma unroll
-            for (int j = 0; j < 5; j++) kv[j] = reinterpret_cast<const double2 *>(a.in.k[j])[i];
-            const cd d = lds[kk * Lay::MS + Lay::at(r, c)];
+            for (int j = 0; j < 5; j++) kv[j] = load(a.in.k[j]);
+            const cd d = lds[e.kk * Lay::MS + Lay::at(e.r, e.c)];
             kv[5] = make_double2(d.x, d.y);
-            v = fmax(v, err_entry(x2[i], kv, a.err_e, a.err_ea, a.err_er, a.err_dt));
+            v = fmax(v, err_entry(load(a.in.x), kv, a.err_e, a.err_ea, a.err_er, a.err_dt));
         }
     }
     return fmax(v, stage_err_specials(a, blk));
@@ -1801,13 +1822,11 @@ __device__ __forceinline__ void rhs_stage_body_r1(const StageArgs &a, const long
         const double di = Dg[L.kk * N + L.i];
 #pragma unroll
         for (int c = 0; c < C; c++) {
-            const int j = L.i ^ c;
-            double gam;
-            if (a.w < 0) {
-                gam = (L.i != j) ? 1.0 : 0.0;
-            } else {
-                const double dE = (di - Dg[L.kk * N + j]) / a.w;
-                gam = 1 - exp(-dE * dE);
+            double gam = c ? 1 : 0;
+            if (!(a.w < 0)) {
+                const double dE = (di - Dg[L.kk * N + (L.i ^ c)]) / a.w;
+                // the diagonal (dE = 0) does not dephase
+                gam = c ? 1 - exp(-dE * dE) : dE * dE;
             }
             T[c] = cscale(T[c], -gam * a.F2);
         }
