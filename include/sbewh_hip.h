@@ -197,9 +197,9 @@ int sbe_hk_mesh(sbe_ctx *ctx, const double A[3], const double E[3], double *out)
  * code/src/CuDiagonalizator.cu:45-51). */
 int sbe_jacobi_batch(int n, int sweeps, long count, const double *H, double *U, double *eig);
 
-/* Layout chosen for the fused stage kernel by the built-in tuner (lanes per
- * matrix row; 0 before the first RHS evaluation, and for 1-D chains of two bands,
- * which have one layout) and, if the tuner ran, the
+/* Layout of the fused stage kernel (lanes per matrix row; 0 before the first RHS
+ * evaluation, and for 1-D chains of two bands, which have one layout), chosen by
+ * rule or by the built-in tuner, and, if the tuner ran, the
  * timed variants (up to 8) with their average launch time in ms.  No
  * reference counterpart: the reference's GPU path has no tunable kernels. */
 int sbe_stage_tuning(const sbe_ctx *ctx, int *lanes_per_row, int *count, int *variants, double *ms);

@@ -135,6 +135,15 @@ struct sbe_ctx {
     int tune_count = 0;
 
     static int default_lr(int N) { return N <= 4 ? 1 : 2; }
+    // The layouts that refine a warm start by products (stage_device.hpp) are the
+    // fastest on every grid timed once calls are warm: 8 bands at one / two / four
+    // lanes per row 299 / 254 / 344 us per four right-hand sides on 150 x 150 k and
+    // 14.2 / 6.7 / 7.2 ms per propagation on 15 x 15 k.  So only calls that
+    // diagonalise from the identity each time, or not at all, are timed: a new
+    // state's first right-hand side then takes 0.35 instead of 1.9 ms on that
+    // grid and 7.5 instead of 38 ms with 16 bands on 48^3 k.
+    static int warm_layout(int N) { return N == 8 ? 2 : N == 16 ? 4 : 0; }
+    bool lr_forced = false;
 
     // Jacobi sweep bound of one diagonalisation.  A call that starts from the
     // previous call's eigenvectors at the same k (warm) runs at most the
@@ -152,8 +161,8 @@ struct sbe_ctx {
         return std::max(prm.sweep_count, COLD_SWEEPS);
     }
 
-    // Time every compiled layout variant of the stage kernel on the current
-    // inputs (3 timed launches after one warm-up each) and keep the fastest.
+    // Unless warm_layout() decides, time every compiled layout variant of the stage
+    // kernel on the current inputs (3 timed launches after one warm-up each) and keep the fastest.
     // SBEWH_STAGE_LR in the environment forces a variant.
     void tune_stage(const StageArgs &a, hipStream_t s)
     {
@@ -163,8 +172,11 @@ struct sbe_ctx {
             int want = std::atoi(env);
             for (int v = 0; v < nv; v++)
                 if (lrs[v] == want) lr = want;
+            lr_forced = lr != 0;
             if (lr) return;
         }
+        if (a.dephase && !(prm.flags & SBE_FLAG_COLD_JACOBI)) lr = warm_layout(N);
+        if (lr) return;
         if (nv == 1) {
             lr = lrs[0];
             return;

@@ -57,15 +57,15 @@ __device__ __forceinline__ void jk_rows_body(const ObsArgs &a, const long blk)
             R[kk * EK + u] = in ? mk(v.x, v.y) : mk(0, 0);
         }
     // T = H0 rho - rho H0, then T and rho transposed
-    __shared__ cd B0[ACC_MS], B1[ACC_MS];
-    const AccPos pos = acc_pos();
+    __shared__ cd B0[Frag16::MS], B1[Frag16::MS];
+    const AccPos pos = acc_pos<Frag16>();
 #pragma unroll
     for (int kk = 0; kk < KB; kk++) {
         cd *h = H + kk * EK, *r = R + kk * EK, x[4], y[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            B0[pos.nat + 4 * ACC_RS * j] = h[j];
-            B1[pos.nat + 4 * ACC_RS * j] = r[j];
+            B0[pos.nat + Frag16::nat_step(j)] = h[j];
+            B1[pos.nat + Frag16::nat_step(j)] = r[j];
         }
         wsync();
         CAcc t;
@@ -80,7 +80,7 @@ __device__ __forceinline__ void jk_rows_body(const ObsArgs &a, const long blk)
         for (int j = 0; j < 4; j++) x[j] = mk(-y[j].x, -y[j].y);
         mfma_cmul(x, h, t);
         wsync();
-        acc_put(B0, pos, t);
+        acc_put<Frag16>(B0, pos, t);
         wsync();
 #pragma unroll
         for (int j = 0; j < 4; j++) {

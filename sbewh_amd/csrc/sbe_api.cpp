@@ -245,8 +245,13 @@ bool resident_integrate(sbe_ctx &c, int output_count, std::vector<double> &tv, l
         c.rhs_calls = calls;
         c.ucache_valid = false;
     }
-    const long kpb = stage_k_per_block(c.N, c.lr), blocks = (c.nk + kpb - 1) / kpb;
-    if (blocks > resident_max_blocks(c.N, c.lr)) return false;
+    auto blocks_at = [&](int lr) { return (c.nk + stage_k_per_block(c.N, lr) - 1) / stage_k_per_block(c.N, lr); };
+    // Here 8 bands at two lanes per row are not refined by products (twiddles of the
+    // same launch cannot come through scalar loads), and four or one are faster
+    int lr = c.lr;
+    if (c.N == 8 && lr == 2 && !c.lr_forced) lr = blocks_at(4) <= resident_max_blocks(8, 4) ? 4 : 1;
+    const long blocks = blocks_at(lr);
+    if (blocks > resident_max_blocks(c.N, lr)) return false;
     // the observer operators do not depend on E: formed once
     HIPCHK(launch_phase_partial(c.geom, c.pbufs(), c.obs_ops, 0, 0, 0, c.Yobs, nullptr, c.stream));
     struct Buf {
@@ -302,7 +307,7 @@ bool resident_integrate(sbe_ctx &c, int output_count, std::vector<double> &tv, l
     r.output_count = output_count;
     r.max_attempts = 100000000L;
     r.status = static_cast<long *>(status.p);
-    const hipError_t e = launch_resident(c.N, c.lr, r, c.stream);
+    const hipError_t e = launch_resident(c.N, lr, r, c.stream);
     if (e == hipErrorCooperativeLaunchTooLarge) {
         (void)hipGetLastError();
         return false;

@@ -199,7 +199,7 @@ struct sbe_scan {
             a.warm = (c.ucache_valid && !(c.prm.flags & SBE_FLAG_COLD_JACOBI)) ? 1 : 0;
             a.sweeps = c.sweeps_for(a.warm);
         }
-        if (!lr) tune_stage(args);
+        if (!lr) tune_stage(rq, args);
         const int kpb = stage_k_per_block(N, lr);
         std::vector<long> b0(m);
         long tot = 0;
@@ -231,9 +231,9 @@ struct sbe_scan {
         }
     }
 
-    // time every layout variant on this batched launch (cold Jacobi, 3 timed
+    // unless sbe_ctx::warm_layout() decides, time every layout variant on this batched launch (cold Jacobi, 3 timed
     // launches after a warm-up) and keep the fastest; SBEWH_STAGE_LR forces one
-    void tune_stage(std::vector<StageArgs> args)
+    void tune_stage(const std::vector<RhsReq> &rq, std::vector<StageArgs> args)
     {
         int lrs[8];
         int nv = stage_variants(N, lrs, 8);
@@ -243,6 +243,11 @@ struct sbe_scan {
                 if (lrs[v] == want) lr = want;
             if (lr) return;
         }
+        bool warm = true;
+        for (int j = 0; j < (int)rq.size(); j++)
+            warm = warm && args[j].dephase && !(rq[j].c->prm.flags & SBE_FLAG_COLD_JACOBI);
+        if (warm) lr = sbe_ctx::warm_layout(N);
+        if (lr) return;
         if (nv == 1) {
             lr = lrs[0];
             return;

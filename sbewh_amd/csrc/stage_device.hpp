@@ -220,9 +220,13 @@ __device__ __forceinline__ void phase_map(const PhaseLast &ph, long nk, int k0, 
 // k0 .. k0 + KPW - 1 into registers, for matrices that fill whole wavefronts (N >= 8):
 // acc[kk N^2 / 64 + u] is entry threadIdx.x + 64 u (row-major, N x N) of k-point kk.  A
 // register belongs to the same k-point in all 64 lanes, so the phase map and the
-// twiddles come through scalar loads, and a phase-sum row is loaded once for all
-// k-points of the wavefront that share it, QG cells in one memory trip.  Consecutive k-points share rest(k) along a Fourier block's last
-// axis, so a wavefront has one or two distinct rows; each gets a pass.
+// twiddles come through scalar loads (QT cells of up to four k-points at a time: a
+// scalar load per cell waited 26 times, four right-hand sides on 150 x 150 k, 8 bands
+// 265 -> 256 us, the scan 38.9 -> 35.1 ms; eight k-points would run out of SGPRs),
+// and a phase-sum row is loaded once for all k-points of the wavefront that share
+// it, QG cells in one memory trip.  Consecutive k-points share rest(k) along a
+// Fourier block's last axis, so a wavefront has one or two distinct rows; each gets
+// a pass.
 // false, with nothing done, for an R box wider than 16 cells along the last
 // axis.  Sums in the order of phase_mats.
 // Why: one wave-uniform branch and one memory trip per cell and pair of entries
@@ -234,8 +238,9 @@ __device__ __forceinline__ bool phase_rows(cd *acc, const PhaseLast &ph, long nk
 {
     static_assert(N * N % 64 == 0, "a k-point's matrix fills whole wavefronts");
     constexpr int EK = N * N / 64;                 // entries per lane and k-point
-    constexpr int KT = KPW < 4 ? KPW : 4;
-    constexpr int QG = EK == 1 ? 4 : 2;            // cells per memory trip
+    constexpr int KT = KPW < 4 ? KPW : 4;          // k-points and
+    // cells whose twiddles are fetched together (SGPRs), cells per memory trip (VGPRs)
+    constexpr int QT = KPW >= 8 ? 1 : EK == 1 ? 4 : 2, QG = KPW >= 8 ? 4 : KPW == 4 ? 8 : QT;
     const int WL = ph.WL;
     if (WL > 16) return false;
     const int kf = __builtin_amdgcn_readfirstlane((int)k0);
@@ -261,39 +266,49 @@ __device__ __forceinline__ bool phase_rows(cd *acc, const PhaseLast &ph, long nk
         int row;
         const unsigned mine = next_row_group<KPW>(todo, rest, row);
         const double2 *yr = Yb + (long)row * M;
-        // cell q of the row (entries y) into the sums of its k-points
-        auto add_cell = [&](int q, const double2 *y) {
+        // NQ cells from cell q on (entries y) into the sums of their k-points
+        auto add_cells = [&](auto nq, int q, const double2 (*y)[EK]) {
+            constexpr int NQ = decltype(nq)::value;
 #pragma unroll
             for (int k4 = 0; k4 < KPW; k4 += KT) {
-                sd2 tw[KT];
+                sd2 tw[KT][NQ];
 #pragma unroll
-                for (int v = 0; v < KT; v++) tw[v] = load_const<sd2>(ph.twL, tp[k4 + v] + q);
+                for (int v = 0; v < KT; v++)
+#pragma unroll
+                    for (int t = 0; t < NQ; t++) tw[v][t] = load_const<sd2>(ph.twL, tp[k4 + v] + q + t);
 #pragma unroll
                 for (int v = 0; v < KT; v++)
                     if (KPW == 1 || ((mine >> (k4 + v)) & 1)) {
                         asm volatile("");  // a branch over the products, not selects behind them
 #pragma unroll
-                        for (int u = 0; u < EK; u++)
-                            acc[(k4 + v) * EK + u] = cfma(mk(tw[v].x, tw[v].y), mk(y[u].x, y[u].y), acc[(k4 + v) * EK + u]);
+                        for (int t = 0; t < NQ; t++)
+#pragma unroll
+                            for (int u = 0; u < EK; u++) {
+                                cd &s = acc[(k4 + v) * EK + u];
+                                s = cfma(mk(tw[v][t].x, tw[v][t].y), mk(y[t][u].x, y[t][u].y), s);
+                            }
                     }
             }
         };
-        int q = 0;
-        for (; q + QG <= WL; q += QG) {
-            double2 y[QG][EK];
+        // NY cells in one memory trip
+        auto trip = [&](auto ny, int q) {
+            constexpr int NY = decltype(ny)::value, NT = QT < NY ? QT : NY;
+            double2 y[NY][EK];
 #pragma unroll
-            for (int t = 0; t < QG; t++)
+            for (int t = 0; t < NY; t++)
 #pragma unroll
                 for (int u = 0; u < EK; u++) y[t][u] = yr[(long)(q + t) * M + ent[u]];
 #pragma unroll
-            for (int t = 0; t < QG; t++) add_cell(q + t, y[t]);
-        }
-        for (; q < WL; q++) {
-            double2 y[EK];
-#pragma unroll
-            for (int u = 0; u < EK; u++) y[u] = yr[(long)q * M + ent[u]];
-            add_cell(q, y);
-        }
+            for (int t = 0; t < NY; t += NT) add_cells(std::integral_constant<int, NT>{}, q + t, y + t);
+        };
+        int q = 0;
+        for (; q + QG <= WL; q += QG) trip(std::integral_constant<int, QG>{}, q);
+        if constexpr (QG == 8)
+            if (q + 4 <= WL) {
+                trip(std::integral_constant<int, 4>{}, q);
+                q += 4;
+            }
+        for (; q < WL; q++) trip(std::integral_constant<int, 1>{}, q);
     }
 #pragma unroll
     for (int kk = 0; kk < KPW; kk++) {
@@ -1246,72 +1261,162 @@ __device__ __forceinline__ void rhs_stage_body16(const StageArgs &a, const long 
     }
 }
 
-// ---- 16 bands, four lanes per row: the decomposition refined by products ----
-// Every matrix lives in the accumulator layout (lane l, register j: row
-// 4 j + l / 16, column l % 16), which is also the layout in which a k-point's
-// matrices are loaded and stored contiguously and in which the phase sum leaves
-// H.  acc_right and acc_left_dagger hand a matrix M to a product as right operand
-// M or left operand M^dagger, so a chain of products needs LDS only where a
-// matrix changes from M to M^dagger.
+// ---- the decomposition refined by products (16 bands, 8 bands) ------------
+// Every matrix lives in the accumulator layout of the FP64 matrix instructions, as
+// four entries per lane (Frag16, Frag8).  Right operand M and left operand
+// M^dagger of a product are the accumulators of M as they are, so a chain of
+// products needs LDS only where a matrix changes from M to M^dagger.
 //
-// This kernel is bound by instruction issue: a v_mfma_f64_16x16x4f64 holds the
-// SIMD for 64 cycles and a vector instruction for 4, and the two do not overlap
-// between the waves of a SIMD (measured: FP64 FMAs, integer operations and MFMAs
-// of different waves take the sum of their times).  A complex product costs
-// 1024 cycles, a Jacobi sweep about 9400 (half of it exchanges, selects and
-// addresses), so warm starts are refined by products: see refine16.
-// Entry (i, j) of a matrix in LDS at 17 i + j: a lane's accumulator entries are
-// one address and constant offsets, and so are those of the transpose; rows and
-// columns walk distinct banks.
-constexpr int ACC_RS = 17, ACC_MS = 16 * ACC_RS;
+// These kernels are bound by instruction issue: a v_mfma_f64_16x16x4f64 holds the
+// SIMD for 64 cycles, a v_mfma_f64_4x4x4f64 for 16 and a vector instruction for 4,
+// and they do not overlap between the waves of a SIMD (measured: FP64 FMAs, integer
+// operations and MFMAs of different waves take the sum of their times).  A
+// complex 16-band product costs 1024 cycles, a Jacobi sweep about 9400 (half of it
+// exchanges, selects and addresses), so warm starts are refined by products: see
+// refine.
+
+// 16 bands, one k-point: register j of lane l is entry (4 j + l / 16, l % 16).  An
+// entry (r, c) in LDS is at 17 r + c: a lane's entries are one address and constant
+// offsets, and so are those of the transpose; rows and columns walk distinct banks.
+struct Frag16 {
+    static constexpr int N = 16, LR = 4, KPW = 1, RS = 17, MS = 16 * RS;
+    static __device__ __forceinline__ int kk() { return 0; }
+    static __device__ __forceinline__ int row(int j) { return cacc_row(j); }
+    static __device__ __forceinline__ int col(int) { return cacc_col(); }
+    static constexpr int nat_step(int j) { return 4 * RS * j; }
+    static constexpr int tr_step(int j) { return 4 * j; }
+    static __device__ __forceinline__ double sum(double v) { return seg_sum<64>(v); }
+    static __device__ __forceinline__ double max(double v) { return __shfl(seg_max<64>(v), 0); }
+    static __device__ __forceinline__ void cmul(const cd *a, const cd *b, CAcc &acc) { mfma_cmul(a, b, acc); }
+    // left operand M^dagger
+    static __device__ __forceinline__ void cmul_dagger(const CAcc &m, const cd *b, CAcc &acc)
+    {
+        cd x[4];
+        acc_left_dagger(m, x);
+        mfma_cmul(x, b, acc);
+    }
+};
+
+// 8 bands, four k-points: a v_mfma_f64_4x4x4f64 multiplies four independent 4 x 4
+// matrices, here one of each k-point, so register j = 2 I + J holds the 4 x 4 block
+// (I, J) of all four: lane l is entry (4 I + l / 16, 4 J + l % 4) of k-point
+// (l / 4) % 4, no lane idles and no operand is rearranged.  LDS strides: the four
+// k-points and the four rows or columns of a block walk distinct banks.
+struct Frag8 {
+    static constexpr int N = 8, LR = 2, KPW = 4, RS = 9, MS = 76;
+    static __device__ __forceinline__ int lane() { return threadIdx.x & 63; }
+    static __device__ __forceinline__ int kk() { return (lane() >> 2) & 3; }
+    static __device__ __forceinline__ int row(int j) { return 4 * (j >> 1) + (lane() >> 4); }
+    static __device__ __forceinline__ int col(int j) { return 4 * (j & 1) + (lane() & 3); }
+    static constexpr int nat_step(int j) { return 4 * RS * (j >> 1) + 4 * (j & 1); }
+    static constexpr int tr_step(int j) { return 4 * RS * (j & 1) + 4 * (j >> 1); }
+    // over the lanes of a k-point
+    static __device__ __forceinline__ double sum(double v)
+    {
+        v += __shfl_xor(v, 1);
+        v += __shfl_xor(v, 2);
+        v += __shfl_xor(v, 16);
+        return v + __shfl_xor(v, 32);
+    }
+    static __device__ __forceinline__ double max(double v)
+    {
+        v = fmax(v, __shfl_xor(v, 1));
+        v = fmax(v, __shfl_xor(v, 2));
+        v = fmax(v, __shfl_xor(v, 16));
+        return fmax(v, __shfl_xor(v, 32));
+    }
+    // d + a b and d - a b of the blocks
+    static __device__ __forceinline__ double fma4(double a, double b, double d)
+    {
+        return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, d, 0, 0, 0);
+    }
+    static __device__ __forceinline__ double fms4(double a, double b, double d)
+    {
+        return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, d, 0, 0, 1);
+    }
+    static __device__ __forceinline__ void cmul(const cd *a, const cd *b, CAcc &acc)
+    {
+#pragma unroll
+        for (int k = 0; k < 4; k += 2)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const cd x = a[k + (j >> 1)], y = b[k + (j & 1)];
+                acc.r[j] = fma4(x.x, y.x, acc.r[j]);
+                acc.i[j] = fma4(x.x, y.y, acc.i[j]);
+                acc.r[j] = fms4(x.y, y.y, acc.r[j]);
+                acc.i[j] = fma4(x.y, y.x, acc.i[j]);
+            }
+    }
+    static __device__ __forceinline__ void cmul_dagger(const CAcc &m, const cd *b, CAcc &acc)
+    {
+#pragma unroll
+        for (int k = 0; k < 4; k += 2)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const double xr = m.r[k + (j >> 1)], xi = m.i[k + (j >> 1)];
+                const cd y = b[k + (j & 1)];
+                acc.r[j] = fma4(xr, y.x, acc.r[j]);
+                acc.i[j] = fma4(xr, y.y, acc.i[j]);
+                acc.r[j] = fma4(xi, y.y, acc.r[j]);
+                acc.i[j] = fms4(xi, y.x, acc.i[j]);
+            }
+    }
+};
+
+// LDS address of the lane's first entry, natural and transposed
 struct AccPos {
     int nat, tr;
 };
+template <class F>
 __device__ __forceinline__ AccPos acc_pos()
 {
-    const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
-    return AccPos{q * ACC_RS + r, r * ACC_RS + q};
+    const int r = F::row(0), c = F::col(0), k = F::kk() * F::MS;
+    return AccPos{k + r * F::RS + c, k + c * F::RS + r};
 }
+template <class F>
 __device__ __forceinline__ void acc_put(cd *buf, const AccPos &p, const CAcc &m)
 {
 #pragma unroll
-    for (int j = 0; j < 4; j++) buf[p.nat + 4 * ACC_RS * j] = mk(m.r[j], m.i[j]);
+    for (int j = 0; j < 4; j++) buf[p.nat + F::nat_step(j)] = mk(m.r[j], m.i[j]);
 }
+template <class F>
 __device__ __forceinline__ void acc_get(const cd *buf, const AccPos &p, CAcc &m)
 {
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        const cd v = buf[p.nat + 4 * ACC_RS * j];
+        const cd v = buf[p.nat + F::nat_step(j)];
         m.r[j] = v.x;
         m.i[j] = v.y;
     }
 }
 // the adjoint of the matrix in buf
+template <class F>
 __device__ __forceinline__ void acc_get_dagger(const cd *buf, const AccPos &p, CAcc &m)
 {
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        const cd v = buf[p.tr + 4 * j];
+        const cd v = buf[p.tr + F::tr_step(j)];
         m.r[j] = v.x;
         m.i[j] = -v.y;
     }
 }
 // M -> M^dagger through the LDS buffer (free on entry and on exit)
+template <class F>
 __device__ __forceinline__ void acc_dagger(cd *buf, const AccPos &p, const CAcc &m, CAcc &out)
 {
-    acc_put(buf, p, m);
+    acc_put<F>(buf, p, m);
     wsync();
-    acc_get_dagger(buf, p, out);
+    acc_get_dagger<F>(buf, p, out);
     wsync();
 }
 
 // acc += A B with A = M^dagger from an accumulator M
+template <class F>
 __device__ __forceinline__ void mul_dagger(const CAcc &m, const CAcc &b, CAcc &acc)
 {
-    cd x[4], y[4];
-    acc_left_dagger(m, x);
+    cd y[4];
     acc_right(b, y);
-    mfma_cmul(x, y, acc);
+    F::cmul_dagger(m, y, acc);
 }
 
 // 1/x for a normal x: hardware estimate and one Newton step
@@ -1333,62 +1438,72 @@ __device__ __forceinline__ double rcp_newton(double x)
 // iteration of Ogita and Aishima with its second-order terms; below X2 these are
 // under rounding and left out).  Elements at most thr, the Jacobi threshold,
 // count as zero.  Nothing is iterated after a step with x <= XF: x^3 is below
-// rounding there.  A k-point with x > XB (a near crossing of bands) is left to
-// the Jacobi rotations: the result is false.
+// rounding there.  An element with X1 > XB couples nearly degenerate bands.  Where
+// it is no larger than what the other elements make at second order (degenerate
+// bands: their block only looks coupled until the others are gone) it waits for the
+// next iteration, and up to 4 thr, the rounding of the products, it stays;
+// otherwise (a near crossing) the wavefront is left to the Jacobi rotations: the
+// result is false.
 // Typically 3e-3 <= x <= 1e-2 between stages: two iterations, 9 products.
 // Measured against the Jacobi rotations from the same warm start (three waves
 // per SIMD at 146 VGPRs; at 128 VGPRs the spills cost more than the fourth wave
 // gives): four right-hand sides on 48^3 k, 16 bands 6.66 -> 4.88 ms, 63 x 63 k,
 // 11 bands 295 -> 212 us, an integration on 24^3 k 121.4 -> 100.7 ms; per
 // wavefront 242 MFMAs and 1730 vector instructions, formerly 123 and 7300.
-__device__ __forceinline__ bool refine16(cd *buf, const cd *H0, const AccPos &pos, CAcc &U, CAcc &Q, double *Dg,
-                                         int sweeps)
+// 8 bands against the rotations at one lane per row (the faster layout of those on
+// this grid): four right-hand sides on 150 x 150 k 296 -> 254 us, an integration there
+// 49.4 -> 44.4 ms; per four k-points 480 4 x 4 MFMAs and 2100 vector instructions,
+// formerly 3700 and twice the LDS traffic.  On 15 x 15 k, where a wavefront's
+// latency counts, 8.1 -> 7.2 ms per propagation against four lanes per row.
+// With every band twofold degenerate: 362 -> 278 us and 46.7 -> 33.2 ms.
+template <class F>
+__device__ __forceinline__ bool refine(cd *buf, const cd *H0, const AccPos &pos, CAcc &U, CAcc &Q, double *Dgs,
+                                       int sweeps)
 {
     constexpr double XB = 0.1, XF = 4e-6, X2 = 1e-8, RF = 1e-14;
-    const int c = cacc_col();
+    double *Dg = Dgs + F::kk() * F::N;
     double thr2 = 0;
     for (int it = 0;; it++) {
         CAcc t, R;
         {
             CAcc h;
-            acc_get(H0, pos, h);
+            acc_get<F>(H0, pos, h);
             cacc_zero(t);
-            mul_dagger(h, Q, t);  // H0 Q
+            mul_dagger<F>(h, Q, t);  // H0 Q
         }
         CAcc S;
         cacc_zero(S);
-        mul_dagger(Q, t, S);  // Q^dagger H0 Q
+        mul_dagger<F>(Q, t, S);  // Q^dagger H0 Q
         cacc_zero(R);
         if (it > 0) {
             cd x[4], y[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                R.r[j] = cacc_row(j) == c ? 1.0 : 0.0;
+                R.r[j] = F::row(j) == F::col(j) ? 1.0 : 0.0;
                 x[j] = mk(-Q.r[j], Q.i[j]);
             }
             acc_right(Q, y);
-            mfma_cmul(x, y, R);  // 1 - Q^dagger Q
+            F::cmul(x, y, R);  // 1 - Q^dagger Q
         }
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            if (cacc_row(j) == c) Dg[c] = S.r[j] / (1.0 - R.r[j]);
+            if (F::row(j) == F::col(j)) Dg[F::col(j)] = S.r[j] / (1.0 - R.r[j]);
         if (it == 0) {
             double s = 0;
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                if (cacc_row(j) <= c) s += fabs(S.r[j]) + fabs(S.i[j]);
-            s = seg_sum<64>(s);
+                if (F::row(j) <= F::col(j)) s += fabs(S.r[j]) + fabs(S.i[j]);
+            s = F::sum(s);
             const double thr = 1e-15 * (0.5 * s);
             thr2 = thr * thr;
         }
         wsync();
-        const double lc = Dg[c];
         CAcc E, X;
         double rd[4], x2 = 0, r2 = 0;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const double lr = Dg[cacc_row(j)];
-            const bool off = cacc_row(j) != c;
+            const double lr = Dg[F::row(j)], lc = Dg[F::col(j)];
+            const bool off = F::row(j) != F::col(j);
             const double hs = 0.5 * (lr + lc);
             E.r[j] = off ? fma(hs, R.r[j], S.r[j]) : 0.0;
             E.i[j] = off ? fma(hs, R.i[j], S.i[j]) : 0.0;
@@ -1404,7 +1519,32 @@ __device__ __forceinline__ bool refine16(cd *buf, const cd *H0, const AccPos &po
         }
         const bool rot = __any(x2 > 0.0), fix = __any(r2 > RF * RF);
         if ((!rot && !fix) || sweeps <= 0) return true;
-        bool bad = __any(x2 > XB * XB);
+        bool bad = false, wait = false;
+        if (__any(x2 > XB * XB)) {
+            double e2 = 0;
+            x2 = 0;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const double q = fma(X.r[j], X.r[j], X.i[j] * X.i[j]);
+                if (q <= XB * XB) {
+                    x2 = fmax(x2, q);
+                    e2 = fmax(e2, fma(E.r[j], E.r[j], E.i[j] * E.i[j]));
+                }
+            }
+            const double second2 = F::N * F::N * F::max(e2) * F::max(x2);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (fma(X.r[j], X.r[j], X.i[j] * X.i[j]) > XB * XB) {
+                    const double m2 = fma(E.r[j], E.r[j], E.i[j] * E.i[j]);
+                    X.r[j] = X.i[j] = rd[j] = 0;
+                    if (m2 > 16 * thr2) {
+                        wait = true;
+                        bad = bad || !(m2 <= second2);
+                    }
+                }
+            bad = __any(bad);
+            wait = __any(wait);
+        }
         const bool second = __any(x2 > X2 * X2);
         CAcc V;  // the adjoint of the update: 1 - X + R/2 + (X - R) X / 2
         cacc_zero(V);
@@ -1415,15 +1555,15 @@ __device__ __forceinline__ bool refine16(cd *buf, const cd *H0, const AccPos &po
 #pragma unroll
             for (int j = 0; j < 4; j++) x[j] = mk(R.r[j] - X.r[j], X.i[j] - R.i[j]);  // X1 + R
             acc_right(E, y);
-            mfma_cmul(x, y, W);
+            F::cmul(x, y, W);
             CAcc Wd;
-            acc_dagger(buf, pos, W, Wd);
+            acc_dagger<F>(buf, pos, W, Wd);
             double c2 = 0;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const double cr = 0.5 * (W.r[j] + Wd.r[j]), ci = 0.5 * (W.i[j] + Wd.i[j]);
-                const bool off = cacc_row(j) != c;
-                if (!off) Dg[c] += cr;
+                const bool off = F::row(j) != F::col(j);
+                if (!off) Dg[F::col(j)] += cr;
                 const bool keep = off && 4 * fma(cr, cr, ci * ci) > thr2;
                 const double xr = keep ? cr * rd[j] : 0.0, xi = keep ? ci * rd[j] : 0.0;
                 c2 = fmax(c2, fma(xr, xr, xi * xi));
@@ -1437,7 +1577,7 @@ __device__ __forceinline__ bool refine16(cd *buf, const cd *H0, const AccPos &po
                 x[j] = mk(-0.5 * (X.r[j] + R.r[j]), 0.5 * (X.i[j] + R.i[j]));
                 y[j] = mk(X.r[j], X.i[j]);
             }
-            mfma_cmul(x, y, V);
+            F::cmul(x, y, V);
         }
         if (bad) {
             wsync();
@@ -1445,111 +1585,126 @@ __device__ __forceinline__ bool refine16(cd *buf, const cd *H0, const AccPos &po
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            V.r[j] += fma(0.5, R.r[j], (cacc_row(j) == c ? 1.0 : 0.0) - X.r[j]);
+            V.r[j] += fma(0.5, R.r[j], (F::row(j) == F::col(j) ? 1.0 : 0.0) - X.r[j]);
             V.i[j] += fma(0.5, R.i[j], -X.i[j]);
         }
         cacc_zero(t);
-        mul_dagger(V, U, t);
+        mul_dagger<F>(V, U, t);
         U = t;
-        acc_dagger(buf, pos, U, Q);
-        if (!__any(x2 > XF * XF) || it + 1 >= sweeps) return true;
+        acc_dagger<F>(buf, pos, U, Q);
+        if ((!wait && !__any(x2 > XF * XF)) || it + 1 >= sweeps) return true;
     }
 }
 
-__device__ __forceinline__ void rhs_stage_body16q(const StageArgs &a, const long blk)
+template <class F>
+__device__ __forceinline__ void rhs_stage_body_acc(const StageArgs &a, const long blk)
 {
-    constexpr int N = 16, LR = 4;
+    constexpr int N = F::N, LR = F::LR, KPW = F::KPW;
     using G = Geo<N, LR>;
+    static_assert(G::KPW == KPW && KPW * N * N == 256, "four entries per lane");
     constexpr int C = G::C;
-    __shared__ cd S0[ACC_MS];  // transposes, operands
-    __shared__ cd S1[ACC_MS];  // H0, then rho
-    __shared__ double Dg[N];
-    __shared__ cd Ja[N], Jb[N];
-    __shared__ int Fa[N];
+    __shared__ cd S0[KPW * F::MS];  // transposes, operands
+    __shared__ cd S1[KPW * F::MS];  // H0, then rho
+    __shared__ double Dgs[KPW * N];
+    __shared__ cd Ja[KPW * N], Jb[KPW * N];
+    __shared__ int Fa[KPW * N];
 
-    const AccPos pos = acc_pos();
-    const int n = a.n, nn = n * n, col = cacc_col();
-    // one k-point per block: its index and the addresses of its matrices are wave-uniform
-    const long k = __builtin_amdgcn_readfirstlane((int)blk), kst = 8 + k * a.P;
-    if (k >= a.nk) return;
+    const AccPos pos = acc_pos<F>();
+    const int n = a.n, nn = n * n;
+    double *Dg = Dgs + F::kk() * N;
+    // the block's first k-point and the addresses of its matrices are wave-uniform;
+    // lanes of a k-point beyond the last one work on the last one and store nothing
+    const long k0 = first_k<N, LR>(blk), kst = 8 + k0 * a.P;
+    if (k0 >= a.nk) return;
+    const bool kin = k0 + F::kk() < a.nk;
+    const int kk = kin ? F::kk() : (int)(a.nk - 1 - k0);
     stage_specials(a, blk);
     bool own[4];  // the lane's registers that are entries of the n x n matrix
     int ent[4];   // and their index in it
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        own[j] = cacc_row(j) < n && col < n;
-        ent[j] = own[j] ? cacc_row(j) * n + col : 0;
+        own[j] = F::row(j) < n && F::col(j) < n;
+        ent[j] = own[j] ? F::row(j) * n + F::col(j) : 0;
     }
-    auto load = [&](const double *src, int j) { return reinterpret_cast<const double2 *>(src)[ent[j]]; };
-    auto phase_acc = [&](int op, CAcc &h) {
+    auto load = [&](const double *src, int j) { return reinterpret_cast<const double2 *>(src)[kk * a.P + ent[j]]; };
+    // an operator into an LDS buffer (a sync of the caller's later)
+    auto phase_put = [&](int op, cd *buf) {
         cd v[4];
-        if (!phase_rows<N, 1>(v, a.ph, a.nk, n, 2 * nn, op * nn, k)) {
+        if (phase_rows<N, KPW>(v, a.ph, a.nk, n, 2 * nn, op * nn, k0)) {
+            // register q of the rows: entry i of k-point q / EK
+            constexpr int EK = N * N / 64;
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = own[j] ? phase_last(a.ph, k, 2 * nn, op * nn + ent[j]) : mk(0, 0);
-        }
+            for (int q = 0; q < 4; q++) {
+                const int i = threadIdx.x + 64 * (q % EK);
+                buf[q / EK * F::MS + i / N * F::RS + i % N] = v[q];
+            }
+        } else {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            h.r[j] = v[j].x;
-            h.i[j] = v[j].y;
+            for (int j = 0; j < 4; j++)
+                buf[pos.nat + F::nat_step(j)] =
+                    own[j] && kin ? phase_last(a.ph, k0 + kk, 2 * nn, op * nn + ent[j]) : mk(0, 0);
         }
     };
 
     CAcc U, Q;  // eigenvector rows, and U^dagger
     if (a.dephase) {
-        double *uc = a.ucache + 2 * k * nn;
+        double2 *uc = reinterpret_cast<double2 *>(a.ucache) + k0 * nn;
         // the previous call's eigenvectors; padded rows and columns are the identity
         auto load_prev = [&]() {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const double2 v = load(uc, j);
-                U.r[j] = own[j] ? v.x : (cacc_row(j) == col ? 1.0 : 0.0);
+                const double2 v = uc[kk * nn + ent[j]];
+                U.r[j] = own[j] ? v.x : (F::row(j) == F::col(j) ? 1.0 : 0.0);
                 U.i[j] = own[j] ? v.y : 0.0;
             }
         };
         bool rotate = true;
         if (a.warm) load_prev();
-        {
-            CAcc h;
-            phase_acc(0, h);
-            acc_put(S1, pos, h);
-        }
+        phase_put(0, S1);
         if (a.warm) {
-            acc_dagger(S0, pos, U, Q);  // (its sync orders the store of H0 too)
-            rotate = !refine16(S0, S1, pos, U, Q, Dg, a.sweeps);
+            acc_dagger<F>(S0, pos, U, Q);  // (its sync orders the store of H0 too)
+            rotate = !refine<F>(S0, S1, pos, U, Q, Dgs, a.sweeps);
         } else {
             wsync();
         }
         if (rotate) {
+            // the layout of the row functions
+            auto put_sw = [&](const CAcc &m) {
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    S0[F::kk() * G::NN + sw<N>(F::row(j), F::col(j))] = mk(m.r[j], m.i[j]);
+            };
             const Lane L = lane_id<N, LR>(a.nk, blk);
-            cd A[C], V[C];
+            cd A[C], V[C], *sk = S0 + L.kk * G::NN;
             CAcc S;
             if (a.warm) {
                 // S = U H0 U^dagger of the previous call's U
                 load_prev();
-                acc_dagger(S0, pos, U, Q);
+                acc_dagger<F>(S0, pos, U, Q);
                 CAcc h, t;
-                acc_get(S1, pos, h);
+                acc_get<F>(S1, pos, h);
                 cacc_zero(t);
-                mul_dagger(h, Q, t);
+                mul_dagger<F>(h, Q, t);
                 cacc_zero(S);
-                mul_dagger(Q, t, S);
-                cacc_store(S0, U);
+                mul_dagger<F>(Q, t, S);
+                put_sw(U);
                 wsync();
-                load_u<N, LR>(S0, L, V);
+                load_u<N, LR>(sk, L, V);
                 wsync();
             } else {
-                acc_get(S1, pos, S);
+                acc_get<F>(S1, pos, S);
             }
-            cacc_store(S0, S);
+            put_sw(S);
             wsync();
-            load_xrow<N, LR>(S0, L, A);
-            wave_jacobi<N, LR>(A, V, L, a.sweeps, Dg, Ja, Jb, Fa, !a.warm);
+            load_xrow<N, LR>(sk, L, A);
+            wave_jacobi<N, LR>(A, V, L, a.sweeps, Dgs, Ja, Jb, Fa, !a.warm);
             wsync();
-            store_u<N, LR>(S0, L, V);
+            store_u<N, LR>(sk, L, V);
             wsync();
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const cd u = S0[sw<16>(cacc_row(j), col)], q = S0[sw<16>(col, cacc_row(j))];
+                const cd *s = S0 + F::kk() * G::NN;
+                const cd u = s[sw<N>(F::row(j), F::col(j))], q = s[sw<N>(F::col(j), F::row(j))];
                 U.r[j] = u.x;
                 U.i[j] = u.y;
                 Q.r[j] = q.x;
@@ -1558,31 +1713,47 @@ __device__ __forceinline__ void rhs_stage_body16q(const StageArgs &a, const long
         }
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            if (own[j]) reinterpret_cast<double2 *>(uc)[ent[j]] = make_double2(U.r[j], U.i[j]);
+            if (own[j] && kin) uc[kk * nn + ent[j]] = make_double2(U.r[j], U.i[j]);
         wsync();
     }
     // rho = x + sum_j c_j k_j, left to right
     CAcc rho;
     {
         const StageInput &inp = a.in;
+        // two entries per memory trip, all terms
+        auto sum = [&](auto terms) {
+            constexpr int NT = decltype(terms)::value;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const double2 v = load(inp.x + 2 * kst, j);
-            rho.r[j] = v.x;
-            rho.i[j] = v.y;
-        }
+            for (int j0 = 0; j0 < 4; j0 += 2) {
+                double2 v[NT + 1][2];
 #pragma unroll
-        for (int d = 0; d < 6; d++)
-            if (d < inp.nt) {
-                const double *kd = inp.k[d] + 2 * kst;
-                const double c = inp.c[d];
+                for (int j = 0; j < 2; j++) {
+                    v[NT][j] = load(inp.x + 2 * kst, j0 + j);
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const double2 v = load(kd, j);
-                    rho.r[j] += c * v.x;
-                    rho.i[j] += c * v.y;
+                    for (int d = 0; d < NT; d++) v[d][j] = load(inp.k[d] + 2 * kst, j0 + j);
+                }
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    double re = v[NT][j].x, im = v[NT][j].y;
+#pragma unroll
+                    for (int d = 0; d < NT; d++) {
+                        re += inp.c[d] * v[d][j].x;
+                        im += inp.c[d] * v[d][j].y;
+                    }
+                    rho.r[j0 + j] = re;
+                    rho.i[j0 + j] = im;
                 }
             }
+        };
+        switch (inp.nt) {
+        case 0: sum(std::integral_constant<int, 0>{}); break;
+        case 1: sum(std::integral_constant<int, 1>{}); break;
+        case 2: sum(std::integral_constant<int, 2>{}); break;
+        case 3: sum(std::integral_constant<int, 3>{}); break;
+        case 4: sum(std::integral_constant<int, 4>{}); break;
+        case 5: sum(std::integral_constant<int, 5>{}); break;
+        default: sum(std::integral_constant<int, 6>{}); break;
+        }
 #pragma unroll
         for (int j = 0; j < 4; j++)
             if (!own[j]) rho.r[j] = rho.i[j] = 0;
@@ -1592,27 +1763,29 @@ __device__ __forceinline__ void rhs_stage_body16q(const StageArgs &a, const long
         double2 *d2 = reinterpret_cast<double2 *>(dst) + kst;
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            if (own[j]) d2[ent[j]] = make_double2(m.r[j], m.i[j]);
-        if ((int)threadIdx.x < a.P - nn) d2[nn + threadIdx.x] = make_double2(0.0, 0.0);
+            if (own[j] && kin) d2[kk * a.P + ent[j]] = make_double2(m.r[j], m.i[j]);
+        for (int t = threadIdx.x; t < KPW * (a.P - nn); t += 64) {
+            const int q = t / (a.P - nn);
+            if (k0 + q < a.nk) d2[q * a.P + nn + t % (a.P - nn)] = make_double2(0.0, 0.0);
+        }
     };
     if (a.xout) store(a.xout, rho);
-    acc_put(S1, pos, rho);
+    acc_put<F>(S1, pos, rho);
     CAcc D;
     cacc_zero(D);
     if (a.dephase) {
         CAcc t, h;
         cacc_zero(t);
-        mul_dagger(rho, Q, t);  // rho^dagger U^dagger
+        mul_dagger<F>(rho, Q, t);  // rho^dagger U^dagger
         cacc_zero(h);
-        mul_dagger(Q, t, h);  // (U rho U^dagger)^dagger
-        const double eb = Dg[col];
+        mul_dagger<F>(Q, t, h);  // (U rho U^dagger)^dagger
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             double gam;
             if (a.w < 0) {
-                gam = (cacc_row(j) != col) ? 1.0 : 0.0;
+                gam = (F::row(j) != F::col(j)) ? 1.0 : 0.0;
             } else {
-                const double dE = (Dg[cacc_row(j)] - eb) / a.w;
+                const double dE = (Dg[F::row(j)] - Dg[F::col(j)]) / a.w;
                 gam = 1 - exp(-dE * dE);
             }
             const double f = -gam * a.F2;
@@ -1620,30 +1793,30 @@ __device__ __forceinline__ void rhs_stage_body16q(const StageArgs &a, const long
             h.i[j] *= f;
         }
         cacc_zero(t);
-        mul_dagger(h, U, t);  // (D o U rho U^dagger) U
-        mul_dagger(U, t, D);  // U^dagger (..)
+        mul_dagger<F>(h, U, t);  // (D o U rho U^dagger) U
+        mul_dagger<F>(U, t, D);  // U^dagger (..)
     }
     // coherent part -i (H_E rho - rho H_E): D + (-i) X = D + (X.i, -X.r), so it is
     // accumulated as i (rho H_E - H_E rho) with the accumulators' roles exchanged
     {
         CAcc he, t;
-        phase_acc(1, he);
-        acc_put(S0, pos, he);
+        phase_put(1, S0);
         wsync();
+        acc_get<F>(S0, pos, he);
         cd x[4], y[4];
         t.r = D.i;
         t.i = -D.r;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const cd v = S0[pos.tr + 4 * j];
+            const cd v = S0[pos.tr + F::tr_step(j)];
             x[j] = mk(-v.x, -v.y);
         }
         acc_right(rho, y);
-        mfma_cmul(x, y, t);  // - H_E rho
+        F::cmul(x, y, t);  // - H_E rho
 #pragma unroll
-        for (int j = 0; j < 4; j++) x[j] = S1[pos.tr + 4 * j];
+        for (int j = 0; j < 4; j++) x[j] = S1[pos.tr + F::tr_step(j)];
         acc_right(he, y);
-        mfma_cmul(x, y, t);  // + rho H_E
+        F::cmul(x, y, t);  // + rho H_E
         D.r = -t.i;
         D.i = t.r;
     }
@@ -1652,7 +1825,7 @@ __device__ __forceinline__ void rhs_stage_body16q(const StageArgs &a, const long
         double v = 0;
 #pragma unroll 2
         for (int j = 0; j < 4; j++)
-            if (own[j]) {
+            if (own[j] && kin) {
                 double2 kv[6];
 #pragma unroll
                 for (int d = 0; d < 5; d++) kv[d] = load(a.in.k[d] + 2 * kst, j);
@@ -1859,7 +2032,10 @@ __device__ __forceinline__ void rhs_stage_body(const StageArgs &a, const long bl
     using G = Geo<N, LR>;
     constexpr int C = G::C;
     if constexpr (N == 16 && LR == 4) {
-        rhs_stage_body16q(a, blk);
+        rhs_stage_body_acc<Frag16>(a, blk);
+        return;
+    } else if constexpr (N == 8 && LR == 2 && PAIR) {
+        rhs_stage_body_acc<Frag8>(a, blk);
         return;
     } else if constexpr (N == 16) {
         rhs_stage_body16<LR>(a, blk);
@@ -1999,12 +2175,11 @@ __device__ __forceinline__ void rhs_stage_body(const StageArgs &a, const long bl
     }
 }
 
-// minimum waves per SIMD the register allocation must allow: the 8-band kernel
-// at one lane per row and the 16-band kernel at four fit three (at most 168
-// VGPRs; a fourth wave of the latter costs spills, see refine16); at 2 lanes per
-// row a bound would only buy spills to scratch
+// minimum waves per SIMD the register allocation must allow: the 8-band kernels
+// at one and two lanes per row and the 16-band kernel at four fit three (at most 168
+// VGPRs; a fourth wave of the latter costs spills, see refine)
 template <int N, int LR>
-constexpr int stage_min_waves() { return (N == 16 && LR == 4) || (N == 8 && LR == 1) ? 3 : 1; }
+constexpr int stage_min_waves() { return (N == 16 && LR == 4) || (N == 8 && LR <= 2) ? 3 : 1; }
 
 template <int N, int LR>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(stage_min_waves<N, LR>())))

@@ -130,3 +130,32 @@ def test_warm_start_long_chain(monkeypatch):
     b = o.rhs(x, 3.0)
     o.close()
     assert np.abs(a - b).max() / np.abs(b).max() < 1e-12
+
+
+# the grid leaves the last of the four-k wavefronts with two k-points
+@pytest.mark.parametrize("n,copies", [(5, 1), (7, 1), (8, 1), (6, 2), (8, 2), (8, 4)])
+def test_warm_start_steps_8_bands(n, copies, monkeypatch):
+    monkeypatch.setenv("SBEWH_STAGE_LR", "2")
+    check_sequence(config(n, (2, 2), (6, 5), (6, 5), copies=copies), STEPS)
+
+
+@pytest.mark.parametrize("n,ext,Nk,Nf", [
+    (8, (1, 0), (6, 1), (3, 1)), (8, (1, 1), (6, 9), (3, 3)), (8, (2, 7), (5, 15), (5, 15)),
+    (8, (1, 8), (3, 18), (3, 18)), (5, (1, 3), (4, 8), (4, 8)), (8, (1, 0), (3, 1), (3, 1))])
+def test_phase_rows_8_bands(n, ext, Nk, Nf, monkeypatch):
+    monkeypatch.setenv("SBEWH_STAGE_LR", "2")
+    check_sequence(config(n, ext, Nk, Nf), [0.0, 0.01])
+
+
+def test_layout_rule():
+    """warm calls of 8 and 16 bands take the layouts refined by products, calls
+    that start from the identity the fastest timed one"""
+    for n, lr in ((8, 2), (11, 4)):
+        cfg = config(n, (1, 1), (3, 4), (3, 4))
+        for cold in (False, True):
+            g = SBEContext(dataclasses.replace(cfg, cold_jacobi=cold))
+            o = Oracle(cfg)
+            g.rhs(states(o, 1, [0.0])[0], 3.0)
+            o.close()
+            t = g.stage_tuning()
+            assert t["lanes_per_row"] == lr if not cold else len(t["timed"]) > 1
