@@ -233,14 +233,21 @@ __device__ __forceinline__ void phase_map(const PhaseLast &ph, long nk, int k0, 
 // (104 in series for 8 bands and 13 cells) kept the 8-band kernel waiting; four
 // right-hand sides on 150 x 150 k, 8 bands: 362 -> 316 us, an integration there
 // 64.3 -> 54.3 ms; 48^3 k, 16 bands: 6.86 -> 6.66 ms.
-template <int N, int KPW>
+//
+// NOP = 2 forms that operator and the next in one pass (acc + KPW N^2 / 64: the second),
+// for grids too small to hide a memory trip behind another wavefront: as many
+// cells per trip as registers allow without that wavefront, the last trip's cells
+// clamped to the row's end.
+template <int N, int KPW, int NOP = 1>
 __device__ __forceinline__ bool phase_rows(cd *acc, const PhaseLast &ph, long nk, int n, int M, int off, long k0)
 {
     static_assert(N * N % 64 == 0, "a k-point's matrix fills whole wavefronts");
-    constexpr int EK = N * N / 64;                 // entries per lane and k-point
+    constexpr int EO = N * N / 64;                 // entries per lane and k-point of an operator
+    constexpr int EK = NOP * EO;                   // and of all
     constexpr int KT = KPW < 4 ? KPW : 4;          // k-points and
     // cells whose twiddles are fetched together (SGPRs), cells per memory trip (VGPRs)
-    constexpr int QT = KPW >= 8 ? 1 : EK == 1 ? 4 : 2, QG = KPW >= 8 ? 4 : KPW == 4 ? 8 : QT;
+    constexpr int QT = KPW >= 8 ? 1 : EO == 1 ? 4 : 2;
+    constexpr int QG = NOP > 1 ? 32 / EK : KPW >= 8 ? 4 : KPW == 4 ? 8 : QT;
     const int WL = ph.WL;
     if (WL > 16) return false;
     const int kf = __builtin_amdgcn_readfirstlane((int)k0);
@@ -253,14 +260,16 @@ __device__ __forceinline__ bool phase_rows(cd *acc, const PhaseLast &ph, long nk
     bool krc[EK];
 #pragma unroll
     for (int u = 0; u < EK; u++) {
-        const int idx = threadIdx.x + 64 * u, r = idx / N, c = idx % N;
+        const int idx = threadIdx.x + 64 * (u % EO), r = idx / N, c = idx % N;
         krc[u] = r < n && c < n;
-        ent[u] = krc[u] ? r * n + c : 0;
+        ent[u] = (krc[u] ? r * n + c : 0) + u / EO * n * n;
     }
+    // entry u of k-point kk
+    auto at = [](int kk, int u) { return (u / EO * KPW + kk) * EO + u % EO; };
 #pragma unroll
     for (int kk = 0; kk < KPW; kk++)
 #pragma unroll
-        for (int u = 0; u < EK; u++) acc[kk * EK + u] = mk(0, 0);
+        for (int u = 0; u < EK; u++) acc[at(kk, u)] = mk(0, 0);
     unsigned todo = KPW >= 32 ? ~0u : (1u << KPW) - 1;
     while (todo) {
         int row;
@@ -284,7 +293,7 @@ __device__ __forceinline__ bool phase_rows(cd *acc, const PhaseLast &ph, long nk
                         for (int t = 0; t < NQ; t++)
 #pragma unroll
                             for (int u = 0; u < EK; u++) {
-                                cd &s = acc[(k4 + v) * EK + u];
+                                cd &s = acc[at(k4 + v, u)];
                                 s = cfma(mk(tw[v][t].x, tw[v][t].y), mk(y[t][u].x, y[t][u].y), s);
                             }
                     }
@@ -302,20 +311,40 @@ __device__ __forceinline__ bool phase_rows(cd *acc, const PhaseLast &ph, long nk
             for (int t = 0; t < NY; t += NT) add_cells(std::integral_constant<int, NT>{}, q + t, y + t);
         };
         int q = 0;
-        for (; q + QG <= WL; q += QG) trip(std::integral_constant<int, QG>{}, q);
-        if constexpr (QG == 8)
-            if (q + 4 <= WL) {
-                trip(std::integral_constant<int, 4>{}, q);
-                q += 4;
+        if constexpr (NOP > 1) {
+            for (; q < WL; q += QG) {
+                double2 y[QG][EK];
+#pragma unroll
+                for (int t = 0; t < QG; t++)
+#pragma unroll
+                    for (int u = 0; u < EK; u++) y[t][u] = yr[(long)(q + t < WL ? q + t : WL - 1) * M + ent[u]];
+#pragma unroll
+                for (int t = 0; t < QG; t += QT) {
+                    if (q + t + QT <= WL) {
+                        add_cells(std::integral_constant<int, QT>{}, q + t, y + t);
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < QT; r++)
+                            if (q + t + r < WL) add_cells(std::integral_constant<int, 1>{}, q + t + r, y + t + r);
+                    }
+                }
             }
-        for (; q < WL; q++) trip(std::integral_constant<int, 1>{}, q);
+        } else {
+            for (; q + QG <= WL; q += QG) trip(std::integral_constant<int, QG>{}, q);
+            if constexpr (QG == 8)
+                if (q + 4 <= WL) {
+                    trip(std::integral_constant<int, 4>{}, q);
+                    q += 4;
+                }
+            for (; q < WL; q++) trip(std::integral_constant<int, 1>{}, q);
+        }
     }
 #pragma unroll
     for (int kk = 0; kk < KPW; kk++) {
         const bool kin = (long)kf + kk < nk;
 #pragma unroll
         for (int u = 0; u < EK; u++)
-            if (!(kin && krc[u])) acc[kk * EK + u] = mk(0, 0);
+            if (!(kin && krc[u])) acc[at(kk, u)] = mk(0, 0);
     }
     return true;
 }
@@ -1279,7 +1308,8 @@ __device__ __forceinline__ void rhs_stage_body16(const StageArgs &a, const long 
 // entry (r, c) in LDS is at 17 r + c: a lane's entries are one address and constant
 // offsets, and so are those of the transpose; rows and columns walk distinct banks.
 struct Frag16 {
-    static constexpr int N = 16, LR = 4, KPW = 1, RS = 17, MS = 16 * RS;
+    using Acc = CAcc;
+    static constexpr int N = 16, LR = 4, KPW = 1, E = 4, RS = 17, MS = 16 * RS;
     static __device__ __forceinline__ int kk() { return 0; }
     static __device__ __forceinline__ int row(int j) { return cacc_row(j); }
     static __device__ __forceinline__ int col(int) { return cacc_col(); }
@@ -1303,7 +1333,8 @@ struct Frag16 {
 // (l / 4) % 4, no lane idles and no operand is rearranged.  LDS strides: the four
 // k-points and the four rows or columns of a block walk distinct banks.
 struct Frag8 {
-    static constexpr int N = 8, LR = 2, KPW = 4, RS = 9, MS = 76;
+    using Acc = CAcc;
+    static constexpr int N = 8, LR = 2, KPW = 4, E = 4, RS = 9, MS = 76;
     static __device__ __forceinline__ int lane() { return threadIdx.x & 63; }
     static __device__ __forceinline__ int kk() { return (lane() >> 2) & 3; }
     static __device__ __forceinline__ int row(int j) { return 4 * (j >> 1) + (lane() >> 4); }
@@ -1363,6 +1394,93 @@ struct Frag8 {
     }
 };
 
+// 8 bands, one k-point, an entry per lane: the instruction's four 4 x 4 products are
+// the four blocks of one 8 x 8 product, lanes 4 b .. 4 b + 3 of each 16 holding
+// block b = 2 I + J, and two steps of the inner index move the operands' blocks into
+// place within the 16 lanes.  Four times the wavefronts of Frag8, each with a quarter
+// of the matrix instructions and of the arithmetic per entry: for grids that leave most
+// SIMDs idle, where the time is one wavefront's.  An attempt of six stages on 15 x 15 k:
+// 92.5 -> 48.7 us, a propagation of 56 attempts there 6.8 -> 4.2 ms.
+struct Acc1 {
+    double r[1], i[1];
+};
+__device__ __forceinline__ void cacc_zero(Acc1 &c) { c.r[0] = c.i[0] = 0; }
+__device__ __forceinline__ void acc_right(const Acc1 &m, cd *y) { y[0] = mk(m.r[0], m.i[0]); }
+
+struct FragOne {
+    using Acc = Acc1;
+    static constexpr int N = 8, LR = 2, KPW = 1, E = 1, RS = 9, MS = 76;
+    static __device__ __forceinline__ int lane() { return threadIdx.x & 63; }
+    static __device__ __forceinline__ int kk() { return 0; }
+    static __device__ __forceinline__ int row(int) { return 4 * ((lane() >> 3) & 1) + (lane() >> 4); }
+    static __device__ __forceinline__ int col(int) { return 4 * ((lane() >> 2) & 1) + (lane() & 3); }
+    static constexpr int nat_step(int) { return 0; }
+    static constexpr int tr_step(int) { return 0; }
+    // in the order of Frag8
+    static __device__ __forceinline__ double sum(double v)
+    {
+        const int l = lane() & ~12;
+        const double b0 = __shfl(v, l), b1 = __shfl(v, l + 4), b2 = __shfl(v, l + 8), b3 = __shfl(v, l + 12);
+        return Frag8::sum(b0 + b1 + b2 + b3);
+    }
+    static __device__ __forceinline__ double max(double v)
+    {
+        v = fmax(v, __shfl_xor(v, 4));
+        return Frag8::max(fmax(v, __shfl_xor(v, 8)));
+    }
+    // lanes of the 4-lane groups in BANKS take v from the lane CTRL names, others keep old
+    template <int CTRL, int BANKS>
+    static __device__ __forceinline__ double take(double old, double v)
+    {
+        const long long o = __double_as_longlong(old), b = __double_as_longlong(v);
+        const int lo = __builtin_amdgcn_update_dpp((int)o, (int)b, CTRL, 0xF, BANKS, false);
+        const int hi = __builtin_amdgcn_update_dpp((int)(o >> 32), (int)(b >> 32), CTRL, 0xF, BANKS, false);
+        return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+    }
+    static constexpr int UP = 0x100, DOWN = 0x110;  // + d: from lane + d, from lane - d
+    // block 2 K + I of the left operand, 2 K + J of the right one
+    template <int K>
+    static __device__ __forceinline__ double left(double v)
+    {
+        if constexpr (K == 0) return take<DOWN + 8, 0x8>(take<DOWN + 4, 0x6>(v, v), v);
+        else return take<UP + 8, 0x1>(take<UP + 4, 0x6>(v, v), v);
+    }
+    template <int K>
+    static __device__ __forceinline__ double right(double v)
+    {
+        if constexpr (K == 0) return take<DOWN + 8, 0xC>(v, v);
+        else return take<UP + 8, 0x3>(v, v);
+    }
+    template <int K>
+    static __device__ __forceinline__ void step(cd a, cd b, Acc &acc)
+    {
+        const double xr = left<K>(a.x), xi = left<K>(a.y), yr = right<K>(b.x), yi = right<K>(b.y);
+        acc.r[0] = Frag8::fma4(xr, yr, acc.r[0]);
+        acc.i[0] = Frag8::fma4(xr, yi, acc.i[0]);
+        acc.r[0] = Frag8::fms4(xi, yi, acc.r[0]);
+        acc.i[0] = Frag8::fma4(xi, yr, acc.i[0]);
+    }
+    static __device__ __forceinline__ void cmul(const cd *a, const cd *b, Acc &acc)
+    {
+        step<0>(a[0], b[0], acc);
+        step<1>(a[0], b[0], acc);
+    }
+    template <int K>
+    static __device__ __forceinline__ void step_dagger(const Acc &m, cd b, Acc &acc)
+    {
+        const double xr = left<K>(m.r[0]), xi = left<K>(m.i[0]), yr = right<K>(b.x), yi = right<K>(b.y);
+        acc.r[0] = Frag8::fma4(xr, yr, acc.r[0]);
+        acc.i[0] = Frag8::fma4(xr, yi, acc.i[0]);
+        acc.r[0] = Frag8::fma4(xi, yi, acc.r[0]);
+        acc.i[0] = Frag8::fms4(xi, yr, acc.i[0]);
+    }
+    static __device__ __forceinline__ void cmul_dagger(const Acc &m, const cd *b, Acc &acc)
+    {
+        step_dagger<0>(m, b[0], acc);
+        step_dagger<1>(m, b[0], acc);
+    }
+};
+
 // LDS address of the lane's first entry, natural and transposed
 struct AccPos {
     int nat, tr;
@@ -1374,16 +1492,16 @@ __device__ __forceinline__ AccPos acc_pos()
     return AccPos{k + r * F::RS + c, k + c * F::RS + r};
 }
 template <class F>
-__device__ __forceinline__ void acc_put(cd *buf, const AccPos &p, const CAcc &m)
+__device__ __forceinline__ void acc_put(cd *buf, const AccPos &p, const typename F::Acc &m)
 {
 #pragma unroll
-    for (int j = 0; j < 4; j++) buf[p.nat + F::nat_step(j)] = mk(m.r[j], m.i[j]);
+    for (int j = 0; j < F::E; j++) buf[p.nat + F::nat_step(j)] = mk(m.r[j], m.i[j]);
 }
 template <class F>
-__device__ __forceinline__ void acc_get(const cd *buf, const AccPos &p, CAcc &m)
+__device__ __forceinline__ void acc_get(const cd *buf, const AccPos &p, typename F::Acc &m)
 {
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < F::E; j++) {
         const cd v = buf[p.nat + F::nat_step(j)];
         m.r[j] = v.x;
         m.i[j] = v.y;
@@ -1391,10 +1509,10 @@ __device__ __forceinline__ void acc_get(const cd *buf, const AccPos &p, CAcc &m)
 }
 // the adjoint of the matrix in buf
 template <class F>
-__device__ __forceinline__ void acc_get_dagger(const cd *buf, const AccPos &p, CAcc &m)
+__device__ __forceinline__ void acc_get_dagger(const cd *buf, const AccPos &p, typename F::Acc &m)
 {
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < F::E; j++) {
         const cd v = buf[p.tr + F::tr_step(j)];
         m.r[j] = v.x;
         m.i[j] = -v.y;
@@ -1402,7 +1520,7 @@ __device__ __forceinline__ void acc_get_dagger(const cd *buf, const AccPos &p, C
 }
 // M -> M^dagger through the LDS buffer (free on entry and on exit)
 template <class F>
-__device__ __forceinline__ void acc_dagger(cd *buf, const AccPos &p, const CAcc &m, CAcc &out)
+__device__ __forceinline__ void acc_dagger(cd *buf, const AccPos &p, const typename F::Acc &m, typename F::Acc &out)
 {
     acc_put<F>(buf, p, m);
     wsync();
@@ -1412,9 +1530,9 @@ __device__ __forceinline__ void acc_dagger(cd *buf, const AccPos &p, const CAcc 
 
 // acc += A B with A = M^dagger from an accumulator M
 template <class F>
-__device__ __forceinline__ void mul_dagger(const CAcc &m, const CAcc &b, CAcc &acc)
+__device__ __forceinline__ void mul_dagger(const typename F::Acc &m, const typename F::Acc &b, typename F::Acc &acc)
 {
-    cd y[4];
+    cd y[F::E];
     acc_right(b, y);
     F::cmul_dagger(m, y, acc);
 }
@@ -1457,28 +1575,28 @@ __device__ __forceinline__ double rcp_newton(double x)
 // latency counts, 8.1 -> 7.2 ms per propagation against four lanes per row.
 // With every band twofold degenerate: 362 -> 278 us and 46.7 -> 33.2 ms.
 template <class F>
-__device__ __forceinline__ bool refine(cd *buf, const cd *H0, const AccPos &pos, CAcc &U, CAcc &Q, double *Dgs,
+__device__ __forceinline__ bool refine(cd *buf, const cd *H0, const AccPos &pos, typename F::Acc &U, typename F::Acc &Q, double *Dgs,
                                        int sweeps)
 {
     constexpr double XB = 0.1, XF = 4e-6, X2 = 1e-8, RF = 1e-14;
     double *Dg = Dgs + F::kk() * F::N;
     double thr2 = 0;
     for (int it = 0;; it++) {
-        CAcc t, R;
+        typename F::Acc t, R;
         {
-            CAcc h;
+            typename F::Acc h;
             acc_get<F>(H0, pos, h);
             cacc_zero(t);
             mul_dagger<F>(h, Q, t);  // H0 Q
         }
-        CAcc S;
+        typename F::Acc S;
         cacc_zero(S);
         mul_dagger<F>(Q, t, S);  // Q^dagger H0 Q
         cacc_zero(R);
         if (it > 0) {
-            cd x[4], y[4];
+            cd x[F::E], y[F::E];
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
+            for (int j = 0; j < F::E; j++) {
                 R.r[j] = F::row(j) == F::col(j) ? 1.0 : 0.0;
                 x[j] = mk(-Q.r[j], Q.i[j]);
             }
@@ -1486,22 +1604,22 @@ __device__ __forceinline__ bool refine(cd *buf, const cd *H0, const AccPos &pos,
             F::cmul(x, y, R);  // 1 - Q^dagger Q
         }
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int j = 0; j < F::E; j++)
             if (F::row(j) == F::col(j)) Dg[F::col(j)] = S.r[j] / (1.0 - R.r[j]);
         if (it == 0) {
             double s = 0;
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+            for (int j = 0; j < F::E; j++)
                 if (F::row(j) <= F::col(j)) s += fabs(S.r[j]) + fabs(S.i[j]);
             s = F::sum(s);
             const double thr = 1e-15 * (0.5 * s);
             thr2 = thr * thr;
         }
         wsync();
-        CAcc E, X;
-        double rd[4], x2 = 0, r2 = 0;
+        typename F::Acc E, X;
+        double rd[F::E], x2 = 0, r2 = 0;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < F::E; j++) {
             const double lr = Dg[F::row(j)], lc = Dg[F::col(j)];
             const bool off = F::row(j) != F::col(j);
             const double hs = 0.5 * (lr + lc);
@@ -1524,7 +1642,7 @@ __device__ __forceinline__ bool refine(cd *buf, const cd *H0, const AccPos &pos,
             double e2 = 0;
             x2 = 0;
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
+            for (int j = 0; j < F::E; j++) {
                 const double q = fma(X.r[j], X.r[j], X.i[j] * X.i[j]);
                 if (q <= XB * XB) {
                     x2 = fmax(x2, q);
@@ -1533,7 +1651,7 @@ __device__ __forceinline__ bool refine(cd *buf, const cd *H0, const AccPos &pos,
             }
             const double second2 = F::N * F::N * F::max(e2) * F::max(x2);
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+            for (int j = 0; j < F::E; j++)
                 if (fma(X.r[j], X.r[j], X.i[j] * X.i[j]) > XB * XB) {
                     const double m2 = fma(E.r[j], E.r[j], E.i[j] * E.i[j]);
                     X.r[j] = X.i[j] = rd[j] = 0;
@@ -1546,21 +1664,21 @@ __device__ __forceinline__ bool refine(cd *buf, const cd *H0, const AccPos &pos,
             wait = __any(wait);
         }
         const bool second = __any(x2 > X2 * X2);
-        CAcc V;  // the adjoint of the update: 1 - X + R/2 + (X - R) X / 2
+        typename F::Acc V;  // the adjoint of the update: 1 - X + R/2 + (X - R) X / 2
         cacc_zero(V);
         if (second && !bad) {
-            cd x[4], y[4];
-            CAcc W;
+            cd x[F::E], y[F::E];
+            typename F::Acc W;
             cacc_zero(W);
 #pragma unroll
-            for (int j = 0; j < 4; j++) x[j] = mk(R.r[j] - X.r[j], X.i[j] - R.i[j]);  // X1 + R
+            for (int j = 0; j < F::E; j++) x[j] = mk(R.r[j] - X.r[j], X.i[j] - R.i[j]);  // X1 + R
             acc_right(E, y);
             F::cmul(x, y, W);
-            CAcc Wd;
+            typename F::Acc Wd;
             acc_dagger<F>(buf, pos, W, Wd);
             double c2 = 0;
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
+            for (int j = 0; j < F::E; j++) {
                 const double cr = 0.5 * (W.r[j] + Wd.r[j]), ci = 0.5 * (W.i[j] + Wd.i[j]);
                 const bool off = F::row(j) != F::col(j);
                 if (!off) Dg[F::col(j)] += cr;
@@ -1572,7 +1690,7 @@ __device__ __forceinline__ bool refine(cd *buf, const cd *H0, const AccPos &pos,
             }
             bad = __any(c2 > XB * XB);
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
+            for (int j = 0; j < F::E; j++) {
                 // left (X - R) / 2 = (-(X + R) / 2)^dagger
                 x[j] = mk(-0.5 * (X.r[j] + R.r[j]), 0.5 * (X.i[j] + R.i[j]));
                 y[j] = mk(X.r[j], X.i[j]);
@@ -1584,7 +1702,7 @@ __device__ __forceinline__ bool refine(cd *buf, const cd *H0, const AccPos &pos,
             return false;
         }
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < F::E; j++) {
             V.r[j] += fma(0.5, R.r[j], (F::row(j) == F::col(j) ? 1.0 : 0.0) - X.r[j]);
             V.i[j] += fma(0.5, R.i[j], -X.i[j]);
         }
@@ -1596,63 +1714,101 @@ __device__ __forceinline__ bool refine(cd *buf, const cd *H0, const AccPos &pos,
     }
 }
 
-template <class F>
+// AHEAD: everything the stage reads is loaded before the decomposition, H0 and H_E
+// in the same memory trips, for grids of a wavefront per SIMD at most, where a trip is
+// waited for in full and registers are free (246 VGPRs).  Used with FragOne; with
+// four k-points per wavefront, whose time is instructions, it gave nothing (6.8 ms
+// either way on 15 x 15 k).
+template <class F, bool AHEAD>
 __device__ __forceinline__ void rhs_stage_body_acc(const StageArgs &a, const long blk)
 {
     constexpr int N = F::N, LR = F::LR, KPW = F::KPW;
     using G = Geo<N, LR>;
-    static_assert(G::KPW == KPW && KPW * N * N == 256, "four entries per lane");
+    static_assert(KPW * N * N == 64 * F::E, "the wavefront's matrices fill its lanes");
     constexpr int C = G::C;
     __shared__ cd S0[KPW * F::MS];  // transposes, operands
     __shared__ cd S1[KPW * F::MS];  // H0, then rho
-    __shared__ double Dgs[KPW * N];
-    __shared__ cd Ja[KPW * N], Jb[KPW * N];
-    __shared__ int Fa[KPW * N];
+    __shared__ double Dgs[G::KPW * N];
+    __shared__ cd Ja[G::KPW * N], Jb[G::KPW * N];
+    __shared__ int Fa[G::KPW * N];
 
     const AccPos pos = acc_pos<F>();
     const int n = a.n, nn = n * n;
     double *Dg = Dgs + F::kk() * N;
     // the block's first k-point and the addresses of its matrices are wave-uniform;
     // lanes of a k-point beyond the last one work on the last one and store nothing
-    const long k0 = first_k<N, LR>(blk), kst = 8 + k0 * a.P;
+    const long k0 = (long)__builtin_amdgcn_readfirstlane((int)blk) * KPW, kst = 8 + k0 * a.P;
     if (k0 >= a.nk) return;
     const bool kin = k0 + F::kk() < a.nk;
     const int kk = kin ? F::kk() : (int)(a.nk - 1 - k0);
     stage_specials(a, blk);
-    bool own[4];  // the lane's registers that are entries of the n x n matrix
-    int ent[4];   // and their index in it
+    bool own[F::E];  // the lane's registers that are entries of the n x n matrix
+    int ent[F::E];   // and their index in it
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < F::E; j++) {
         own[j] = F::row(j) < n && F::col(j) < n;
         ent[j] = own[j] ? F::row(j) * n + F::col(j) : 0;
     }
     auto load = [&](const double *src, int j) { return reinterpret_cast<const double2 *>(src)[kk * a.P + ent[j]]; };
+    // AHEAD: the stage input's terms (x last) and both operators
+    double2 vin[AHEAD ? 7 : 1][F::E];
+    cd hop[AHEAD ? 2 * F::E : 1];
+    bool formed = false;
+    if constexpr (AHEAD) {
+#pragma unroll
+        for (int j = 0; j < F::E; j++) vin[6][j] = load(a.in.x + 2 * kst, j);
+#pragma unroll
+        for (int d = 0; d < 6; d++)
+            if (d < a.in.nt)
+#pragma unroll
+                for (int j = 0; j < F::E; j++) vin[d][j] = load(a.in.k[d] + 2 * kst, j);
+    }
     // an operator into an LDS buffer (a sync of the caller's later)
     auto phase_put = [&](int op, cd *buf) {
-        cd v[4];
-        if (phase_rows<N, KPW>(v, a.ph, a.nk, n, 2 * nn, op * nn, k0)) {
+        cd v[F::E];
+        if constexpr (AHEAD)
+#pragma unroll
+            for (int q = 0; q < F::E; q++) v[q] = hop[F::E * op + q];
+        if (formed || phase_rows<N, KPW>(v, a.ph, a.nk, n, 2 * nn, op * nn, k0)) {
             // register q of the rows: entry i of k-point q / EK
             constexpr int EK = N * N / 64;
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
+            for (int q = 0; q < F::E; q++) {
                 const int i = threadIdx.x + 64 * (q % EK);
                 buf[q / EK * F::MS + i / N * F::RS + i % N] = v[q];
             }
         } else {
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+            for (int j = 0; j < F::E; j++)
                 buf[pos.nat + F::nat_step(j)] =
                     own[j] && kin ? phase_last(a.ph, k0 + kk, 2 * nn, op * nn + ent[j]) : mk(0, 0);
         }
     };
 
-    CAcc U, Q;  // eigenvector rows, and U^dagger
+    typename F::Acc U, Q;  // eigenvector rows, and U^dagger
+    typename F::Acc rho;   // x + sum_j c_j k_j, left to right
+    if constexpr (AHEAD) {
+        if (a.dephase) formed = phase_rows<N, KPW, 2>(hop, a.ph, a.nk, n, 2 * nn, 0, k0);
+#pragma unroll
+        for (int j = 0; j < F::E; j++) {
+            rho.r[j] = vin[6][j].x;
+            rho.i[j] = vin[6][j].y;
+        }
+#pragma unroll
+        for (int d = 0; d < 6; d++)
+            if (d < a.in.nt)
+#pragma unroll
+                for (int j = 0; j < F::E; j++) {
+                    rho.r[j] += a.in.c[d] * vin[d][j].x;
+                    rho.i[j] += a.in.c[d] * vin[d][j].y;
+                }
+    }
     if (a.dephase) {
         double2 *uc = reinterpret_cast<double2 *>(a.ucache) + k0 * nn;
         // the previous call's eigenvectors; padded rows and columns are the identity
         auto load_prev = [&]() {
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
+            for (int j = 0; j < F::E; j++) {
                 const double2 v = uc[kk * nn + ent[j]];
                 U.r[j] = own[j] ? v.x : (F::row(j) == F::col(j) ? 1.0 : 0.0);
                 U.i[j] = own[j] ? v.y : 0.0;
@@ -1669,19 +1825,21 @@ __device__ __forceinline__ void rhs_stage_body_acc(const StageArgs &a, const lon
         }
         if (rotate) {
             // the layout of the row functions
-            auto put_sw = [&](const CAcc &m) {
+            auto put_sw = [&](const typename F::Acc &m) {
 #pragma unroll
-                for (int j = 0; j < 4; j++)
+                for (int j = 0; j < F::E; j++)
                     S0[F::kk() * G::NN + sw<N>(F::row(j), F::col(j))] = mk(m.r[j], m.i[j]);
             };
-            const Lane L = lane_id<N, LR>(a.nk, blk);
-            cd A[C], V[C], *sk = S0 + L.kk * G::NN;
-            CAcc S;
+            // (one k-point in a layout of several: they all work on it and store the same)
+            constexpr bool SAME = KPW < G::KPW;
+            const Lane L = SAME ? lane_id<N, LR>(G::KPW, 0) : lane_id<N, LR>(a.nk, blk);
+            cd A[C], V[C], *sk = S0 + (SAME ? 0 : L.kk) * G::NN;
+            typename F::Acc S;
             if (a.warm) {
                 // S = U H0 U^dagger of the previous call's U
                 load_prev();
                 acc_dagger<F>(S0, pos, U, Q);
-                CAcc h, t;
+                typename F::Acc h, t;
                 acc_get<F>(S1, pos, h);
                 cacc_zero(t);
                 mul_dagger<F>(h, Q, t);
@@ -1702,7 +1860,7 @@ __device__ __forceinline__ void rhs_stage_body_acc(const StageArgs &a, const lon
             store_u<N, LR>(sk, L, V);
             wsync();
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
+            for (int j = 0; j < F::E; j++) {
                 const cd *s = S0 + F::kk() * G::NN;
                 const cd u = s[sw<N>(F::row(j), F::col(j))], q = s[sw<N>(F::col(j), F::row(j))];
                 U.r[j] = u.x;
@@ -1712,13 +1870,11 @@ __device__ __forceinline__ void rhs_stage_body_acc(const StageArgs &a, const lon
             }
         }
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int j = 0; j < F::E; j++)
             if (own[j] && kin) uc[kk * nn + ent[j]] = make_double2(U.r[j], U.i[j]);
         wsync();
     }
-    // rho = x + sum_j c_j k_j, left to right
-    CAcc rho;
-    {
+    if constexpr (!AHEAD) {
         const StageInput &inp = a.in;
         // two entries per memory trip, all terms
         auto sum = [&](auto terms) {
@@ -1754,15 +1910,15 @@ __device__ __forceinline__ void rhs_stage_body_acc(const StageArgs &a, const lon
         case 5: sum(std::integral_constant<int, 5>{}); break;
         default: sum(std::integral_constant<int, 6>{}); break;
         }
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            if (!own[j]) rho.r[j] = rho.i[j] = 0;
     }
+#pragma unroll
+    for (int j = 0; j < F::E; j++)
+        if (!own[j]) rho.r[j] = rho.i[j] = 0;
     // a matrix of the state from the accumulator, with zero pads
-    auto store = [&](double *dst, const CAcc &m) {
+    auto store = [&](double *dst, const typename F::Acc &m) {
         double2 *d2 = reinterpret_cast<double2 *>(dst) + kst;
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int j = 0; j < F::E; j++)
             if (own[j] && kin) d2[kk * a.P + ent[j]] = make_double2(m.r[j], m.i[j]);
         for (int t = threadIdx.x; t < KPW * (a.P - nn); t += 64) {
             const int q = t / (a.P - nn);
@@ -1771,16 +1927,16 @@ __device__ __forceinline__ void rhs_stage_body_acc(const StageArgs &a, const lon
     };
     if (a.xout) store(a.xout, rho);
     acc_put<F>(S1, pos, rho);
-    CAcc D;
+    typename F::Acc D;
     cacc_zero(D);
     if (a.dephase) {
-        CAcc t, h;
+        typename F::Acc t, h;
         cacc_zero(t);
         mul_dagger<F>(rho, Q, t);  // rho^dagger U^dagger
         cacc_zero(h);
         mul_dagger<F>(Q, t, h);  // (U rho U^dagger)^dagger
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < F::E; j++) {
             double gam;
             if (a.w < 0) {
                 gam = (F::row(j) != F::col(j)) ? 1.0 : 0.0;
@@ -1799,39 +1955,56 @@ __device__ __forceinline__ void rhs_stage_body_acc(const StageArgs &a, const lon
     // coherent part -i (H_E rho - rho H_E): D + (-i) X = D + (X.i, -X.r), so it is
     // accumulated as i (rho H_E - H_E rho) with the accumulators' roles exchanged
     {
-        CAcc he, t;
+        typename F::Acc he, t;
         phase_put(1, S0);
         wsync();
         acc_get<F>(S0, pos, he);
-        cd x[4], y[4];
-        t.r = D.i;
-        t.i = -D.r;
+        cd x[F::E], y[F::E];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < F::E; j++) {
+            t.r[j] = D.i[j];
+            t.i[j] = -D.r[j];
             const cd v = S0[pos.tr + F::tr_step(j)];
             x[j] = mk(-v.x, -v.y);
         }
         acc_right(rho, y);
         F::cmul(x, y, t);  // - H_E rho
 #pragma unroll
-        for (int j = 0; j < 4; j++) x[j] = S1[pos.tr + F::tr_step(j)];
+        for (int j = 0; j < F::E; j++) x[j] = S1[pos.tr + F::tr_step(j)];
         acc_right(he, y);
         F::cmul(x, y, t);  // + rho H_E
-        D.r = -t.i;
-        D.i = t.r;
+#pragma unroll
+        for (int j = 0; j < F::E; j++) {
+            D.r[j] = -t.i[j];
+            D.i[j] = t.r[j];
+        }
     }
     store(a.dxdt, D);
     if (a.err_partial) {
         double v = 0;
-#pragma unroll 2
-        for (int j = 0; j < 4; j++)
-            if (own[j] && kin) {
-                double2 kv[6];
+        if constexpr (AHEAD) {  // all loads in one trip
+            double2 kv[F::E][6], xv[F::E];
 #pragma unroll
-                for (int d = 0; d < 5; d++) kv[d] = load(a.in.k[d] + 2 * kst, j);
-                kv[5] = make_double2(D.r[j], D.i[j]);
-                v = fmax(v, err_entry(load(a.in.x + 2 * kst, j), kv, a.err_e, a.err_ea, a.err_er, a.err_dt));
+            for (int j = 0; j < F::E; j++) {
+                xv[j] = load(a.in.x + 2 * kst, j);
+#pragma unroll
+                for (int d = 0; d < 5; d++) kv[j][d] = load(a.in.k[d] + 2 * kst, j);
+                kv[j][5] = make_double2(D.r[j], D.i[j]);
             }
+#pragma unroll
+            for (int j = 0; j < F::E; j++)
+                if (own[j] && kin) v = fmax(v, err_entry(xv[j], kv[j], a.err_e, a.err_ea, a.err_er, a.err_dt));
+        } else {
+#pragma unroll 2
+            for (int j = 0; j < F::E; j++)
+                if (own[j] && kin) {
+                    double2 kv[6];
+#pragma unroll
+                    for (int d = 0; d < 5; d++) kv[d] = load(a.in.k[d] + 2 * kst, j);
+                    kv[5] = make_double2(D.r[j], D.i[j]);
+                    v = fmax(v, err_entry(load(a.in.x + 2 * kst, j), kv, a.err_e, a.err_ea, a.err_er, a.err_dt));
+                }
+        }
         v = fmax(v, stage_err_specials(a, blk));
         v = seg_max<64>(v);
         if (threadIdx.x == 0) a.err_partial[blk] = v;
@@ -2026,16 +2199,19 @@ __device__ __forceinline__ void rhs_stage_body_r1(const StageArgs &a, const long
 // PAIR: for n <= 4, H_E is formed together with H_0 and held in registers
 // (fewer memory trips; more registers, which a caller through a call
 // boundary may not want)
-template <int N, int LR, bool PAIR = true>
+template <int N, int LR, bool PAIR = true, bool AHEAD = false>
 __device__ __forceinline__ void rhs_stage_body(const StageArgs &a, const long blk)
 {
     using G = Geo<N, LR>;
     constexpr int C = G::C;
-    if constexpr (N == 16 && LR == 4) {
-        rhs_stage_body_acc<Frag16>(a, blk);
+    if constexpr (N == 8 && LR == 8) {
+        rhs_stage_body_acc<FragOne, AHEAD>(a, blk);
+        return;
+    } else if constexpr (N == 16 && LR == 4) {
+        rhs_stage_body_acc<Frag16, AHEAD>(a, blk);
         return;
     } else if constexpr (N == 8 && LR == 2 && PAIR) {
-        rhs_stage_body_acc<Frag8>(a, blk);
+        rhs_stage_body_acc<Frag8, AHEAD>(a, blk);
         return;
     } else if constexpr (N == 16) {
         rhs_stage_body16<LR>(a, blk);
@@ -2185,7 +2361,7 @@ template <int N, int LR>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(stage_min_waves<N, LR>())))
 void rhs_stage_kernel(StageArgs a)
 {
-    rhs_stage_body<N, LR>(a, xcd_block(blockIdx.x, gridDim.x));
+    rhs_stage_body<N, LR, true, N == 8 && LR == 8>(a, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // Several instances in one launch: entry j owns the logical blocks
@@ -2370,7 +2546,7 @@ __global__ __launch_bounds__(64) void rhs_stage_set_kernel(
 {
     const long blk = xcd_block(blockIdx.x, gridDim.x);
     for (int q = 0; q < ss.m; q++) {
-        rhs_stage_body<N, LR>(ss.st[q], blk);
+        rhs_stage_body<N, LR, true, N == 8 && LR == 8>(ss.st[q], blk);
         // the next stage loads, from other lanes, what this one stored
         __threadfence_block();
         wsync();

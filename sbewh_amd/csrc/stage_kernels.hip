@@ -119,6 +119,13 @@ int stage_variants(int N, int *lr_out, int cap)
     return k;
 }
 
+// Grids of 5 to 8 bands with a SIMD of its own for each k-point (256 CUs of four): a
+// k-point per wavefront (FragOne).  Above, four per wavefront (Frag8) run a
+// grid of up to 4096 k-points in one round, where the others take a second one.  Measured on a
+// propagation of 56 attempts, four per wavefront against one, by k-points: 225
+// 6.9 -> 4.6 ms, 900 8.3 -> 6.5 ms, 1296 8.4 -> 9.2 ms, 2025 9.5 -> 11.7 ms.
+constexpr long ONE_K_MOST = 1024;
+
 hipError_t launch_rhs_stage(int N, int LR, const StageArgs &a, hipStream_t s)
 {
     switch (N * 100 + LR) {
@@ -128,7 +135,9 @@ hipError_t launch_rhs_stage(int N, int LR, const StageArgs &a, hipStream_t s)
     case 402: return launch_rhs_NL<4, 2>(a, s);
     case 404: return launch_rhs_NL<4, 4>(a, s);
     case 801: return launch_rhs_stage_r1(8, a, s);
-    case 802: return launch_rhs_NL<8, 2>(a, s);
+    case 802:
+        // (the caller adds up one error partial per block of the layout it named)
+        return a.nk <= ONE_K_MOST && !a.err_partial ? launch_rhs_NL<8, 8>(a, s) : launch_rhs_NL<8, 2>(a, s);
     case 804: return launch_rhs_NL<8, 4>(a, s);
     case 1602: return launch_rhs_NL<16, 2>(a, s);
     case 1604: return launch_rhs_NL<16, 4>(a, s);
@@ -145,7 +154,7 @@ hipError_t launch_rhs_stage_set(int N, int LR, const StageSet &ss, hipStream_t s
     case 402: return launch_rhs_set_NL<4, 2>(ss, s);
     case 404: return launch_rhs_set_NL<4, 4>(ss, s);
     case 801: return launch_rhs_stage_set_r1(8, ss, s);
-    case 802: return launch_rhs_set_NL<8, 2>(ss, s);
+    case 802: return ss.st[0].nk <= ONE_K_MOST ? launch_rhs_set_NL<8, 8>(ss, s) : launch_rhs_set_NL<8, 2>(ss, s);
     case 804: return launch_rhs_set_NL<8, 4>(ss, s);
     case 1602: return launch_rhs_set_NL<16, 2>(ss, s);
     case 1604: return launch_rhs_set_NL<16, 4>(ss, s);

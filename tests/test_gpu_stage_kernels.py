@@ -159,3 +159,29 @@ def test_layout_rule():
             o.close()
             t = g.stage_tuning()
             assert t["lanes_per_row"] == lr if not cold else len(t["timed"]) > 1
+
+
+# 5 to 8 bands take a k-point per wavefront up to 1024 k-points and four above (the
+# last wavefront with two on 42 x 25 k)
+@pytest.mark.parametrize("n,copies,Nk,Nf", [
+    (8, 1, (32, 32), (4, 4)), (5, 1, (41, 25), (1, 5)), (8, 1, (42, 25), (6, 5)), (6, 2, (42, 25), (6, 5)),
+    (7, 1, (1, 1), (1, 1))])
+def test_k_points_per_wavefront_8_bands(n, copies, Nk, Nf):
+    ext = (min(1, (Nf[0] - 1) // 2), min(1, (Nf[1] - 1) // 2))
+    check_sequence(config(n, ext, Nk, Nf, copies=copies), STEPS)
+
+
+@pytest.mark.parametrize("n,Nk,Nf", [(8, (4, 5), (4, 5)), (6, (32, 32), (4, 4)), (8, (42, 25), (6, 5))])
+def test_attempt_in_one_launch_8_bands(n, Nk, Nf):
+    """a propagation whose attempts are one launch each replays the oracle's steps"""
+    cfg = dataclasses.replace(config(n, (1, 1), Nk, Nf, eps_rel=1e-7, T2_fs=10.0, output_count=5),
+                              pulses=model.elliptic_sin2(1.0, 0.4, 3000.0, 0.1))
+    g, o = SBEContext(cfg), Oracle(cfg)
+    a = o.initial_state(0.0)
+    b = a.copy()
+    ro = o.integrate(a, cfg.output_count)
+    rg = g.integrate(b, cfg.output_count, replay=ro["log"])
+    assert np.abs(rg["j"] - ro["j"]).max() < 1e-10 * np.abs(ro["j"]).max()
+    assert np.abs(b - a).max() < 1e-10 * np.abs(a).max()
+    o.close()
+    g.close()
