@@ -140,12 +140,18 @@ struct sbe_scan {
     void partial(const std::vector<sbe_ctx *> &cs, const std::vector<std::array<double, 3>> &E, int ops, bool obs)
     {
         const int m = (int)cs.size();
+        // All instances share a launch, so 2048 blocks, which fill the GPU, are theirs
+        // together: larger row tiles then read the model fewer times.  (24 pulses on
+        // 15 x 15 and 60 x 60 k, 2048 blocks for each one against for all: 27.8 -> 20 us
+        // a launch; 1024 and 4096 for all 22.5 us.)
+        constexpr long MIN_BLOCKS = 2048;
         std::vector<std::vector<ContractStage>> st(2, std::vector<ContractStage>(m));
         for (int j = 0; j < m; j++) {
             ContractStage tmp[2];
             sbe_ctx &c = *cs[j];
             int k = phase_partial_plan(c.geom, c.pbufs(), ops, E[j][0], E[j][1], E[j][2], obs ? c.Yobs : c.Y,
-                                       obs ? nullptr : c.merged(), tmp);
+                                       obs ? nullptr : c.merged(), tmp,
+                                       std::max(1L, MIN_BLOCKS / m));
             if (k != (obs ? ns_obs : ns)) fail(SBE_ERR_ARG, "inconsistent phase-sum plans in the scan");
             for (int d = 0; d < k; d++) st[d][j] = tmp[d];
         }
