@@ -78,3 +78,19 @@ def test_scan_instance_against_oracle_replay():
     ro = o.integrate(xo, cfg.output_count, replay=s["log"])
     assert rel(r["j"][0], ro["j"]) <= 1e-10
     assert rel(sc.final_state(0), xo) <= 1e-10
+
+
+def test_scan_cold_jacobi():
+    """decompositions from the identity: the scan times its layouts between the
+    phase sums and the first right-hand side.  Layouts round differently, so
+    steps may too: within the step tolerance of the single runs."""
+    cfgs = [dataclasses.replace(cases.small_square(Nk=(nk, nk, 1), eps_rel=1e-8, cycles=0.2), cold_jacobi=True,
+                                output_count=4) for nk in (15, 30)]
+    r = Scan(cfgs).run(4)
+    for i, cfg in enumerate(cfgs):
+        g = SBEContext(cfg)
+        x = g.initial_state(g.fermi_level(cfg.occupied_bands))
+        s = g.integrate(x, 4)
+        assert np.array_equal(r["t"][i], s["t"])
+        assert np.abs(r["j"][i] - s["j"]).max() <= 1e-8 * np.abs(s["j"]).max()
+        g.close()
