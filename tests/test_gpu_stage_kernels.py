@@ -185,3 +185,9 @@ def test_attempt_in_one_launch_8_bands(n, Nk, Nf):
     assert np.abs(b - a).max() < 1e-10 * np.abs(a).max()
     o.close()
     g.close()
+
+
+@pytest.mark.parametrize("Nk,Nf", [((4, 5), (4, 5)), ((42, 25), (6, 5))])
+def test_no_dephasing_8_bands(Nk, Nf, monkeypatch):
+    monkeypatch.setenv("SBEWH_STAGE_LR", "2")
+    check_sequence(config(7, (1, 1), Nk, Nf, T2_fs=0.0), [0.0, 0.01])
