@@ -126,6 +126,13 @@ int stage_variants(int N, int *lr_out, int cap)
 // 6.9 -> 4.6 ms, 900 8.3 -> 6.5 ms, 1296 8.4 -> 9.2 ms, 2025 9.5 -> 11.7 ms.
 constexpr long ONE_K_MOST = 1024;
 
+static hipError_t launch_rhs_12(const StageArgs &a, hipStream_t s)
+{
+    if (a.nk <= 0) return hipSuccess;
+    hipLaunchKernelGGL((rhs_stage_acc_kernel<Frag12>), dim3((unsigned)a.nk), dim3(64), 0, s, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_rhs_stage(int N, int LR, const StageArgs &a, hipStream_t s)
 {
     switch (N * 100 + LR) {
@@ -140,7 +147,7 @@ hipError_t launch_rhs_stage(int N, int LR, const StageArgs &a, hipStream_t s)
         return a.nk <= ONE_K_MOST && !a.err_partial ? launch_rhs_NL<8, 8>(a, s) : launch_rhs_NL<8, 2>(a, s);
     case 804: return launch_rhs_NL<8, 4>(a, s);
     case 1602: return launch_rhs_NL<16, 2>(a, s);
-    case 1604: return launch_rhs_NL<16, 4>(a, s);
+    case 1604: return a.n <= 12 ? launch_rhs_12(a, s) : launch_rhs_NL<16, 4>(a, s);
     }
     return hipErrorInvalidValue;
 }
