@@ -205,7 +205,7 @@ int stage_variants(int N, int *lr_out, int cap);
 // k-points per block (one wavefront) of layout (N, LR)
 int stage_k_per_block(int N, int LR);
 // entry j owns the logical blocks [block0[j], block0[j+1]) (ceil(nk_j / k_per_block) each)
-hipError_t launch_rhs_stage_batched(int N, int LR, const StageArgs *d_args, const long *d_block0, int m, long blocks,
+hipError_t launch_rhs_stage_batched(int N, int LR, int n, const StageArgs *d_args, const long *d_block0, int m, long blocks,
                                     hipStream_t s);
 
 struct InitArgs {

@@ -244,7 +244,7 @@ struct sbe_scan {
         long *db = add(b0.data(), m);
         stage_b0 = db;
         stage_blocks = tot;
-        enqueue([=] { HIPCHK(launch_rhs_stage_batched(N, lr, da, db, m, tot, stream)); });
+        enqueue([=] { HIPCHK(launch_rhs_stage_batched(N, lr, n, da, db, m, tot, stream)); });
         for (int j = 0; j < m; j++) {
             if (args[j].dephase) rq[j].c->ucache_valid = true;
             rq[j].c->rhs_calls++;
@@ -288,9 +288,9 @@ struct sbe_scan {
             }
             long *db = add(b0.data(), m);
             flush();
-            HIPCHK(launch_rhs_stage_batched(N, lrs[v], da, db, m, tot, stream));
+            HIPCHK(launch_rhs_stage_batched(N, lrs[v], n, da, db, m, tot, stream));
             HIPCHK(hipEventRecord(ev[0], stream));
-            for (int it = 0; it < 3; it++) HIPCHK(launch_rhs_stage_batched(N, lrs[v], da, db, m, tot, stream));
+            for (int it = 0; it < 3; it++) HIPCHK(launch_rhs_stage_batched(N, lrs[v], n, da, db, m, tot, stream));
             HIPCHK(hipEventRecord(ev[1], stream));
             HIPCHK(hipEventSynchronize(ev[1]));
             float ms = 0;

@@ -1331,7 +1331,8 @@ struct Frag16 {
 // 9 to 12 bands: the same without the last four rows, which are padding, as entries or
 // as steps of the inner index (the columns keep their lanes): a quarter of the matrix
 // instructions and of the arithmetic per entry less.  Four right-hand sides on
-// 63 x 63 k, 11 bands: 212 -> 179 us.
+// 63 x 63 k, 11 bands: 212 -> 179 us; a propagation on 18 x 18 k 8.4 -> 7.6 ms, a scan of
+// 12 pulses on 18 x 18 and 54 x 54 k 46.2 -> 40.3 ms.
 struct Frag12 : Frag16 {
     static constexpr int E = 3;
     static __device__ __forceinline__ void cmul(const cd *a, const cd *b, CAcc &acc) { mfma_cmul<3>(a, b, acc); }
@@ -2228,10 +2229,11 @@ __device__ __forceinline__ void rhs_stage_body_r1(const StageArgs &a, const long
 template <int N, int LR, bool PAIR = true, bool AHEAD = false>
 __device__ __forceinline__ void rhs_stage_body(const StageArgs &a, const long blk)
 {
-    using G = Geo<N, LR>;
-    constexpr int C = G::C;
     if constexpr (N == 8 && LR == 8) {
         rhs_stage_body_acc<FragOne, AHEAD>(a, blk);
+        return;
+    } else if constexpr (N == 16 && LR == 12) {  // (12: a name, not a row layout)
+        rhs_stage_body_acc<Frag12, AHEAD>(a, blk);
         return;
     } else if constexpr (N == 16 && LR == 4) {
         rhs_stage_body_acc<Frag16, AHEAD>(a, blk);
@@ -2246,6 +2248,8 @@ __device__ __forceinline__ void rhs_stage_body(const StageArgs &a, const long bl
         rhs_stage_body_r1<N, PAIR>(a, blk);
         return;
     } else {
+    using G = Geo<N, LR>;
+    constexpr int C = G::C;
     __shared__ cd S0[G::KPW * G::NN];
     __shared__ cd S1[G::KPW * G::NN];
     __shared__ double Dg[G::KPW * N];
@@ -2381,20 +2385,13 @@ __device__ __forceinline__ void rhs_stage_body(const StageArgs &a, const long bl
 // at one and two lanes per row and the 16-band kernel at four fit three (at most 168
 // VGPRs; a fourth wave of the latter costs spills, see refine)
 template <int N, int LR>
-constexpr int stage_min_waves() { return (N == 16 && LR == 4) || (N == 8 && LR <= 2) ? 3 : 1; }
+constexpr int stage_min_waves() { return (N == 16 && LR >= 4) || (N == 8 && LR <= 2) ? 3 : 1; }
 
 template <int N, int LR>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(stage_min_waves<N, LR>())))
 void rhs_stage_kernel(StageArgs a)
 {
     rhs_stage_body<N, LR, true, N == 8 && LR == 8>(a, xcd_block(blockIdx.x, gridDim.x));
-}
-
-template <class F>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
-void rhs_stage_acc_kernel(StageArgs a)
-{
-    rhs_stage_body_acc<F, false>(a, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // Several instances in one launch: entry j owns the logical blocks

@@ -14,11 +14,15 @@ static hipError_t launch_occ_NL(const OccArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
+// k-points of a wavefront
+template <int N, int LR>
+constexpr int k_per_wave() { return N * LR > 64 ? 1 : 64 / (N * LR); }
+
 template <int N, int LR>
 static hipError_t launch_rhs_NL(const StageArgs &a, hipStream_t s)
 {
-    using G = Geo<N, LR>;
-    long blocks = (a.nk + G::KPW - 1) / G::KPW;
+    constexpr int K = k_per_wave<N, LR>();
+    long blocks = (a.nk + K - 1) / K;
     if (blocks <= 0) return hipSuccess;
     hipLaunchKernelGGL((rhs_stage_kernel<N, LR>), dim3((unsigned)blocks), dim3(64), 0, s, a);
     return hipGetLastError();
@@ -27,13 +31,13 @@ static hipError_t launch_rhs_NL(const StageArgs &a, hipStream_t s)
 template <int N, int LR>
 static hipError_t launch_rhs_set_NL(const StageSet &ss, hipStream_t s)
 {
-    using G = Geo<N, LR>;
+    constexpr int K = k_per_wave<N, LR>();
     if (ss.m <= 0) return hipSuccess;
     if (ss.m > SET_MAX) return hipErrorInvalidValue;
     for (int q = 1; q < ss.m; q++)
         if (ss.st[q].nk != ss.st[0].nk) return hipErrorInvalidValue;
     if (ss.ticket && (!ss.err_out || !ss.st[ss.m - 1].err_partial)) return hipErrorInvalidValue;
-    long blocks = (ss.st[0].nk + G::KPW - 1) / G::KPW;
+    long blocks = (ss.st[0].nk + K - 1) / K;
     if (blocks <= 0) return hipSuccess;
     hipLaunchKernelGGL((rhs_stage_set_kernel<N, LR>), dim3((unsigned)blocks), dim3(64), 0, s, ss);
     return hipGetLastError();
@@ -126,13 +130,6 @@ int stage_variants(int N, int *lr_out, int cap)
 // 6.9 -> 4.6 ms, 900 8.3 -> 6.5 ms, 1296 8.4 -> 9.2 ms, 2025 9.5 -> 11.7 ms.
 constexpr long ONE_K_MOST = 1024;
 
-static hipError_t launch_rhs_12(const StageArgs &a, hipStream_t s)
-{
-    if (a.nk <= 0) return hipSuccess;
-    hipLaunchKernelGGL((rhs_stage_acc_kernel<Frag12>), dim3((unsigned)a.nk), dim3(64), 0, s, a);
-    return hipGetLastError();
-}
-
 hipError_t launch_rhs_stage(int N, int LR, const StageArgs &a, hipStream_t s)
 {
     switch (N * 100 + LR) {
@@ -147,7 +144,7 @@ hipError_t launch_rhs_stage(int N, int LR, const StageArgs &a, hipStream_t s)
         return a.nk <= ONE_K_MOST && !a.err_partial ? launch_rhs_NL<8, 8>(a, s) : launch_rhs_NL<8, 2>(a, s);
     case 804: return launch_rhs_NL<8, 4>(a, s);
     case 1602: return launch_rhs_NL<16, 2>(a, s);
-    case 1604: return a.n <= 12 ? launch_rhs_12(a, s) : launch_rhs_NL<16, 4>(a, s);
+    case 1604: return a.n <= 12 ? launch_rhs_NL<16, 12>(a, s) : launch_rhs_NL<16, 4>(a, s);
     }
     return hipErrorInvalidValue;
 }
@@ -164,12 +161,12 @@ hipError_t launch_rhs_stage_set(int N, int LR, const StageSet &ss, hipStream_t s
     case 802: return ss.st[0].nk <= ONE_K_MOST ? launch_rhs_set_NL<8, 8>(ss, s) : launch_rhs_set_NL<8, 2>(ss, s);
     case 804: return launch_rhs_set_NL<8, 4>(ss, s);
     case 1602: return launch_rhs_set_NL<16, 2>(ss, s);
-    case 1604: return launch_rhs_set_NL<16, 4>(ss, s);
+    case 1604: return ss.st[0].n <= 12 ? launch_rhs_set_NL<16, 12>(ss, s) : launch_rhs_set_NL<16, 4>(ss, s);
     }
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_rhs_stage_batched(int N, int LR, const StageArgs *args, const long *block0, int m, long blocks,
+hipError_t launch_rhs_stage_batched(int N, int LR, int n, const StageArgs *args, const long *block0, int m, long blocks,
                                     hipStream_t s)
 {
     switch (N * 100 + LR) {
@@ -182,7 +179,9 @@ hipError_t launch_rhs_stage_batched(int N, int LR, const StageArgs *args, const 
     case 802: return launch_rhs_batched_NL<8, 2>(args, block0, m, blocks, s);
     case 804: return launch_rhs_batched_NL<8, 4>(args, block0, m, blocks, s);
     case 1602: return launch_rhs_batched_NL<16, 2>(args, block0, m, blocks, s);
-    case 1604: return launch_rhs_batched_NL<16, 4>(args, block0, m, blocks, s);
+    case 1604:
+        return n <= 12 ? launch_rhs_batched_NL<16, 12>(args, block0, m, blocks, s)
+                       : launch_rhs_batched_NL<16, 4>(args, block0, m, blocks, s);
     }
     return hipErrorInvalidValue;
 }

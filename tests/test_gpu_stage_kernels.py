@@ -8,6 +8,7 @@ import pytest
 
 from sbewh_amd import model
 from sbewh_amd.propagator import SBEContext
+from sbewh_amd.scan import Scan
 from oracle.oracle_py import Oracle
 from tests import cases
 
@@ -171,8 +172,9 @@ def test_k_points_per_wavefront_8_bands(n, copies, Nk, Nf):
     check_sequence(config(n, ext, Nk, Nf, copies=copies), STEPS)
 
 
-@pytest.mark.parametrize("n,Nk,Nf", [(8, (4, 5), (4, 5)), (6, (32, 32), (4, 4)), (8, (42, 25), (6, 5))])
-def test_attempt_in_one_launch_8_bands(n, Nk, Nf):
+@pytest.mark.parametrize("n,Nk,Nf", [(8, (4, 5), (4, 5)), (6, (32, 32), (4, 4)), (8, (42, 25), (6, 5)), (12, (4, 5), (4, 5)),
+                                      (9, (4, 5), (4, 5))])
+def test_attempt_in_one_launch(n, Nk, Nf):
     """a propagation whose attempts are one launch each replays the oracle's steps"""
     cfg = dataclasses.replace(config(n, (1, 1), Nk, Nf, eps_rel=1e-7, T2_fs=10.0, output_count=5),
                               pulses=model.elliptic_sin2(1.0, 0.4, 3000.0, 0.1))
@@ -191,3 +193,22 @@ def test_attempt_in_one_launch_8_bands(n, Nk, Nf):
 def test_no_dephasing_8_bands(Nk, Nf, monkeypatch):
     monkeypatch.setenv("SBEWH_STAGE_LR", "2")
     check_sequence(config(7, (1, 1), Nk, Nf, T2_fs=0.0), [0.0, 0.01])
+
+
+@pytest.mark.parametrize("n", [9, 12])
+def test_scan_9_to_12_bands(n):
+    """two pulses in a scan against single runs: the same kernels and steps"""
+    base = dataclasses.replace(config(n, (1, 1), (4, 5), (4, 5), eps_rel=1e-7, T2_fs=10.0, output_count=4),
+                               pulses=model.elliptic_sin2(1.0, 0.4, 3000.0, 0.1))
+    half = n // 2   # a gap between the halves
+    base.model.H[len(base.model.cells) // 2] += np.diag(np.where(np.arange(n) < half, -2.0, 2.0))
+    base = dataclasses.replace(base, occupied_bands=half)
+    cfgs = [base, dataclasses.replace(base, Nk=(8, 10, 1))]
+    r = Scan(cfgs).run(4)
+    for i, cfg in enumerate(cfgs):
+        g = SBEContext(cfg)
+        x = g.initial_state(g.fermi_level(cfg.occupied_bands))
+        s = g.integrate(x, 4)
+        assert r["steps"][i] == s["steps"]
+        assert np.abs(r["j"][i] - s["j"]).max() <= 1e-12 * np.abs(s["j"]).max()
+        g.close()
