@@ -94,7 +94,8 @@ int sbe_initial_state(sbe_ctx *ctx, double mu, double *state);
 int sbe_rhs(sbe_ctx *ctx, const double *state, double *dsdt, double t);
 
 /* The same on device buffers, enqueued on `stream` (a hipStream_t; NULL = the
- * context's stream) and returning without synchronising.  Replaces
+ * context's stream) and returning without synchronising.  d_dsdt may be d_state
+ * itself.  Replaces
  * CuPropagator::operator()(const GPUstate&, GPUstate&, double)
  * (code/src/CuPropagator.h:34). */
 int sbe_rhs_device(sbe_ctx *ctx, const double *d_state, double *d_dsdt, double t, void *stream);

@@ -203,11 +203,18 @@ __device__ __forceinline__ void store_entry(double *s, const Site &p, int P, cd 
 // d/dt of special slot t: dA_0/dt = -E, the rest 0
 __device__ __forceinline__ double2 special_rate(int t, double E) { return make_double2(t == 0 ? -E : 0.0, 0.0); }
 
+// the special slots of dxdt; they are read as A by every block of
+// chain_rhs_kernel, so with dxdt == x they are written behind it
+__global__ void chain_specials_kernel(double *dxdt, double E)
+{
+    reinterpret_cast<double2 *>(dxdt)[threadIdx.x] = special_rate(threadIdx.x, E);
+}
+
 template <int MW>
 __global__ __launch_bounds__(64) void chain_rhs_kernel(ChainArgs c, const double *x, double *dxdt, double E)
 {
     const Site p = site(c);
-    if (blockIdx.x == 0 && threadIdx.x < 8)
+    if (dxdt != x && blockIdx.x == 0 && threadIdx.x < 8)
         reinterpret_cast<double2 *>(dxdt)[threadIdx.x] = special_rate(threadIdx.x, E);
     const double *const op[2] = {c.Hb, c.Db};
     Cells<MW> cell[2];
@@ -361,9 +368,12 @@ static hipError_t by_extent(const ChainArgs &c, F &&launch)
 
 hipError_t launch_chain_rhs(const ChainArgs &c, const double *x, double *dxdt, double E, hipStream_t s)
 {
-    return by_extent(c, [&](auto mw, dim3 grid, dim3 blk) {
+    const hipError_t e = by_extent(c, [&](auto mw, dim3 grid, dim3 blk) {
         hipLaunchKernelGGL(chain_rhs_kernel<decltype(mw)::value>, grid, blk, 0, s, c, x, dxdt, E);
     });
+    if (e != hipSuccess || dxdt != x) return e;
+    hipLaunchKernelGGL(chain_specials_kernel, dim3(1), dim3(8), 0, s, dxdt, E);
+    return hipGetLastError();
 }
 
 hipError_t launch_chain_output(const ChainArgs &c, const double *x, double *j, double *partial, double *k1, double E,

@@ -112,6 +112,37 @@ def test_rhs_device_gpu_layout_on_device_buffers():
     cg.close()
 
 
+def in_place_equals_out_of_place(cfg, seed=7):
+    """on a fresh context each, so that both are the context's first evaluation"""
+    out = []
+    for in_place in (False, True):
+        g = SBEContext(cfg)
+        rng = np.random.default_rng(seed)
+        x = np.zeros(g.state_size, complex)
+        x[8:].reshape(g.num_k, g.P)[:, :g.n ** 2] = cases.random_hermitian(rng, g.num_k, g.n, 0.3).reshape(g.num_k, -1)
+        x[:cfg.dim] = [0.2, -0.1, 0.05][:cfg.dim]
+        d_in = hip_mem.DeviceBuffer.from_array(x.view(np.float64))
+        d_out = d_in if in_place else hip_mem.DeviceBuffer.from_array(np.full(2 * x.size, 7.0))
+        s = hip_mem.Stream()
+        print(f"[gpu] rhs in place={in_place} n={g.n} k={g.num_k}", flush=True)
+        g.rhs_device(d_in.ptr, d_out.ptr, 0.3, s.handle)
+        s.synchronize()
+        out.append(d_out.download(np.float64, 2 * x.size))
+        s.destroy()
+        g.close()
+    assert np.array_equal(*out)
+
+
+# one wavefront and many, cells kept in registers and read from memory
+@pytest.mark.parametrize("reach,nk,nf", [(2, 10, 5), (4, 256, 16), (6, 160, 16)])
+@pytest.mark.parametrize("gpu_layout", [False, True])
+def test_rhs_in_place_two_band_chain(reach, nk, nf, gpu_layout):
+    """the derivative over the state itself: every k-point reads the vector
+    potential before the special slots are overwritten"""
+    from tests.test_gpu_chain import chain
+    in_place_equals_out_of_place(chain(reach, nk, nf, gpu_layout=gpu_layout))
+
+
 def test_integrate_gpu_layout_equals_cpu_layout(monkeypatch):
     cc, cg = SBEContext(chain_short(False)), SBEContext(chain_short(True))
     n, nk = cc.n, cc.num_k
