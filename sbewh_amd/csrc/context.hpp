@@ -165,8 +165,11 @@ struct sbe_ctx {
     // Unless warm_layout() decides, time every compiled layout variant of the stage
     // kernel on the current inputs (3 timed launches after one warm-up each) and keep the fastest.
     // SBEWH_STAGE_LR in the environment forces a variant.
-    void tune_stage(const StageArgs &a, hipStream_t s)
+    void tune_stage(StageArgs a, hipStream_t s)
     {
+        // a caller's right-hand side in place: the timed launches must leave its
+        // input as it is (the context's own calls never name st[9] as an input)
+        if (a.dxdt == a.in.x) a.dxdt = st[9];
         int lrs[8];
         int nv = stage_variants(N, lrs, 8);
         if (const char *env = std::getenv("SBEWH_STAGE_LR")) {
