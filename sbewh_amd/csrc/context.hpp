@@ -140,10 +140,12 @@ struct sbe_ctx {
     // lanes per row 299 / 254 / 344 us per four right-hand sides on 150 x 150 k and
     // 14.2 / 6.7 / 7.2 ms per propagation on 15 x 15 k (now 4.2 at two: small grids take
     // a k-point per wavefront, stage_kernels.hip).  So only calls that
-    // diagonalise from the identity each time, or not at all, are timed: a new
+    // diagonalise from the identity each time, or not at all, or are bound to one
+    // sweep, which is one of rotations, are timed: a new
     // state's first right-hand side then takes 0.35 instead of 1.9 ms on that
     // grid and 7.5 instead of 38 ms with 16 bands on 48^3 k.
     static int warm_layout(int N) { return N == 8 ? 2 : N == 16 ? 4 : 0; }
+    bool refines() const { return prm.relaxation_F2 > 0 && !(prm.flags & SBE_FLAG_COLD_JACOBI) && prm.sweep_count != 1; }
     bool lr_forced = false;
 
     // Jacobi sweep bound of one diagonalisation.  A call that starts from the
@@ -179,7 +181,7 @@ struct sbe_ctx {
             lr_forced = lr != 0;
             if (lr) return;
         }
-        if (a.dephase && !(prm.flags & SBE_FLAG_COLD_JACOBI)) lr = warm_layout(N);
+        if (refines()) lr = warm_layout(N);
         if (lr) return;
         if (nv == 1) {
             lr = lrs[0];

@@ -264,8 +264,7 @@ struct sbe_scan {
             if (lr) return;
         }
         bool warm = true;
-        for (int j = 0; j < (int)rq.size(); j++)
-            warm = warm && args[j].dephase && !(rq[j].c->prm.flags & SBE_FLAG_COLD_JACOBI);
+        for (const RhsReq &r : rq) warm = warm && r.c->refines();
         if (warm) lr = sbe_ctx::warm_layout(N);
         if (lr) return;
         if (nv == 1) {

@@ -133,6 +133,31 @@ def test_warm_start_long_chain(monkeypatch):
     assert np.abs(a - b).max() / np.abs(b).max() < 1e-12
 
 
+@pytest.mark.parametrize("sweeps", [1, 2])
+@pytest.mark.parametrize("n,lr,rotations", [(8, 2, 1), (6, 2, 4), (16, 4, 2), (11, 4, 2), (14, 4, 2)])
+def test_warm_chain_small_sweep_bounds(n, lr, rotations, sweeps, monkeypatch):
+    """1500 warm starts under a small sweep bound: the decomposition stays unitary (the
+    dephasing term then has no trace) and is as good as the rotations' with that bound"""
+    cfg = config(n, (2, 2), (6, 5), (6, 5), sweeps=sweeps)
+    o = Oracle(dataclasses.replace(cfg, sweeps=12))
+    err = []
+    for layout in (rotations, lr):
+        monkeypatch.setenv("SBEWH_STAGE_LR", str(layout))
+        g = SBEContext(cfg)
+        x = states(o, 1, [0.0])[0]
+        for q in range(1500):
+            x[0] += 0.004 * np.cos(0.1 * q)
+            a = g.rhs(x, 3.0)
+        g.close()
+        b = o.rhs(x, 3.0)
+        tr = np.trace(a[8:].reshape(o.num_k, o.P)[:, :n * n].reshape(-1, n, n), axis1=1, axis2=2)
+        err.append(np.abs(a - b).max() / np.abs(b).max())
+        print(f"[gpu] n={n} lanes {layout} sweeps {sweeps}: trace {np.abs(tr).max():.1e} error {err[-1]:.1e}", flush=True)
+        assert np.abs(tr).max() < 1e-12 * np.abs(b).max()
+    assert err[1] <= max(1e-12, 2 * err[0])
+    o.close()
+
+
 # the grid leaves the last of the four-k wavefronts with two k-points
 @pytest.mark.parametrize("n,copies", [(5, 1), (7, 1), (8, 1), (6, 2), (8, 2), (8, 4)])
 def test_warm_start_steps_8_bands(n, copies, monkeypatch):
