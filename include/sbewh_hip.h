@@ -33,7 +33,7 @@ enum sbe_status {
     SBE_OK = 0,
     SBE_ERR_ARG = -1,        /* invalid argument / unsupported configuration */
     SBE_ERR_HIP = -2,        /* HIP runtime or launch failure */
-    SBE_ERR_STEP = -3,       /* step-size control failed (500 rejected tries) */
+    SBE_ERR_STEP = -3,       /* step-size control failed (500 rejected tries, an error norm that is NaN) */
     SBE_ERR_PHYSICS = -4,    /* e.g. no unique band gap for the Fermi level */
     SBE_ERR_REPLAY = -5      /* replay log exhausted / inconsistent */
 };

@@ -323,7 +323,8 @@ __global__ __launch_bounds__(64) void chain_attempt_kernel(ChainArgs c, ChainAtt
     double2 kv[6];
 #pragma unroll
     for (int j = 0; j < 6; j++) kv[j] = make_double2(kd[idx[j]].x, kd[idx[j]].y);
-    double err = p.ok ? err_entry(make_double2(x.x, x.y), kv, s.err_e, s.ea, s.er, s.dt) : 0.0;
+    ErrMax err;
+    if (p.ok) err.add(err_entry(make_double2(x.x, x.y), kv, s.err_e, s.ea, s.er, s.dt));
     if (blockIdx.x == 0 && threadIdx.x < 8) {
         // the special slots
         const int t = threadIdx.x;
@@ -339,18 +340,16 @@ __global__ __launch_bounds__(64) void chain_attempt_kernel(ChainArgs c, ChainAtt
         }
         reinterpret_cast<double2 *>(s.xn)[t] = make_double2(re, im);
         reinterpret_cast<double2 *>(s.k7)[t] = kv[5];
-        err = fmax(err, err_entry(xv, kv, s.err_e, s.ea, s.er, s.dt));
+        err.add(err_entry(xv, kv, s.err_e, s.ea, s.er, s.dt));
     }
-    err = seg_max<64>(err);
-    if (threadIdx.x == 0) s.partial[blockIdx.x] = err;
+    const double mine = err.wave();
+    if (threadIdx.x == 0) s.partial[blockIdx.x] = mine;
     if (!last_block(s.ticket)) return;
-    double v = 0;
+    ErrMax all;
     for (unsigned b = threadIdx.x; b < gridDim.x; b += 64)
-        v = fmax(v, __hip_atomic_load(s.partial + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    v = seg_max<64>(v);
-    if (threadIdx.x == 0)
-        __hip_atomic_store(s.err_out, (unsigned long long)__double_as_longlong(v), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_SYSTEM);
+        all.add(__hip_atomic_load(s.partial + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    const double v = all.wave();
+    if (threadIdx.x == 0) store_error(s.err_out, v);
 }
 
 // The cells a lane keeps: 4 VGPRs per cell and operator, so up to nine (the

@@ -529,7 +529,7 @@ struct sbe_ctx {
     // poll it instead of waiting for the stream to drain (the next attempt's
     // launches then queue behind the retiring kernel).  A stream that has
     // completed, or failed, without the value arriving is an error.
-    static constexpr unsigned long long ERR_PENDING = ~0ull;  // a negative NaN: never a max of |.| terms
+    static constexpr unsigned long long ERR_PENDING = ~0ull;  // a NaN that store_error() never stores
     double wait_error(hipStream_t s)
     {
         const volatile unsigned long long *p = err_host;

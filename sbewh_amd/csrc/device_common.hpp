@@ -56,7 +56,31 @@ __device__ __forceinline__ double err_entry(double2 xv, const double2 (&kv)[6], 
     }
     const double num = sqrt(fma(re, re, im * im));
     const double ax = sqrt(fma(xv.x, xv.x, xv.y * xv.y)), ak = sqrt(fma(kv[0].x, kv[0].x, kv[0].y * kv[0].y));
-    return num / fma(er, fma(dt, ak, ax), ea);
+    // (a zero under a relative bound alone has no error)
+    return num / fmax(fma(er, fma(dt, ak, ax), ea), 2.2250738585072014e-308);
+}
+
+// A maximum of error terms (none is negative) that keeps a NaN, which fmax drops: a
+// state with a NaN had norm 0, and its steps were accepted.  The sum of the terms is
+// NaN if one of them is.
+struct ErrMax {
+    double v = 0, sum = 0;
+    __device__ __forceinline__ void add(double t)
+    {
+        v = fmax(v, t);
+        sum += t;
+    }
+    // the lane's
+    __device__ __forceinline__ double value() const { return sum != sum ? sum : v; }
+    // over the wavefront
+    __device__ __forceinline__ double wave() const;
+};
+// The norm's bits for a host that polls them: one NaN for all, as another one's may
+// be the pattern that stands for "not there yet".
+__device__ __forceinline__ void store_error(unsigned long long *out, double v)
+{
+    const unsigned long long b = v != v ? 0x7ff8000000000000ull : (unsigned long long)__double_as_longlong(v);
+    __hip_atomic_store(out, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Last-axis contraction of a partial phase sum (see PhaseLast in kernels.hpp)
@@ -188,6 +212,12 @@ __device__ __forceinline__ double seg_max(double v)
 #pragma unroll
     for (int m = 1; m < seg; m <<= 1) v = fmax(v, __shfl_xor(v, m));
     return v;
+}
+
+__device__ __forceinline__ double ErrMax::wave() const
+{
+    const double m = seg_max<64>(v);
+    return __any(sum != sum) ? __builtin_nan("") : m;
 }
 
 // k index (state / Fourier-block order) <-> global grid indices.

@@ -366,9 +366,9 @@ __global__ __launch_bounds__(64) void resident_kernel(ResidentArgs r)
             run_stage(Si[q], q < 5 ? r.k[q + 2] : s.k7, Es[q], q, q == 5 ? s.xn : nullptr, dt);
         rhs += 6;
         grid_sync(grid);
-        double err = 0;
-        for (long b = 0; b < nblk; b++) err = fmax(err, r.err_partial[b]);
-        return err;
+        ErrMax err;
+        for (long b = 0; b < nblk; b++) err.add(r.err_partial[b]);
+        return err.value();
     };
 
     {

@@ -15,14 +15,17 @@
 
 namespace sbe {
 
-// max over the 256 threads of a block (result valid in thread 0)
-__device__ __forceinline__ double block_max(double v)
+// the maximum over a block's wavefronts (result valid in thread 0)
+template <int WAVES>
+__device__ __forceinline__ double block_max(const ErrMax &e)
 {
-    __shared__ double red[4];
-    v = seg_max<64>(v);
+    __shared__ double red[WAVES];
+    const double v = e.wave();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    return fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+    ErrMax m;
+    for (int k = 0; k < WAVES; k++) m.add(red[k]);
+    return m.value();
 }
 
 // Final reduction of per-block maxima (the last stage kernel of an attempt
@@ -35,30 +38,20 @@ __device__ __forceinline__ double block_max(double v)
 __global__ __launch_bounds__(1024) void error_final_kernel(const double *partial, int nb, unsigned long long *out)
 {
     constexpr int U = 8;
-    double v[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) v[u] = 0;
+    ErrMax v[U];
     int i = threadIdx.x;
     for (; i + (U - 1) * 1024 < nb; i += U * 1024) {
         double x[U];
 #pragma unroll
         for (int u = 0; u < U; u++) x[u] = partial[i + u * 1024];
 #pragma unroll
-        for (int u = 0; u < U; u++) v[u] = fmax(v[u], x[u]);
+        for (int u = 0; u < U; u++) v[u].add(x[u]);
     }
-    for (; i < nb; i += 1024) v[0] = fmax(v[0], partial[i]);
+    for (; i < nb; i += 1024) v[0].add(partial[i]);
 #pragma unroll
-    for (int u = 1; u < U; u++) v[0] = fmax(v[0], v[u]);
-    __shared__ double red[16];
-    double w = seg_max<64>(v[0]);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = w;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double m = red[0];
-        for (int k = 1; k < 16; k++) m = fmax(m, red[k]);
-        __hip_atomic_store(out, (unsigned long long)__double_as_longlong(m), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    for (int u = 1; u < U; u++) v[0].add(v[u].value());
+    const double m = block_max<16>(v[0]);
+    if (threadIdx.x == 0) store_error(out, m);
 }
 
 // per-instance final reduction of a batched last stage's per-block maxima:
@@ -69,10 +62,10 @@ __global__ __launch_bounds__(256) void error_final_batched_kernel(const long *bl
 {
     const int j = blockIdx.x;
     const long b1 = j + 1 < m ? block0[j + 1] : blocks;
-    double v = 0;
-    for (long b = block0[j] + threadIdx.x; b < b1; b += 256) v = fmax(v, partial[b]);
-    v = block_max(v);
-    if (threadIdx.x == 0) out[j] = v;
+    ErrMax v;
+    for (long b = block0[j] + threadIdx.x; b < b1; b += 256) v.add(partial[b]);
+    const double e = block_max<4>(v);
+    if (threadIdx.x == 0) out[j] = e;
 }
 
 hipError_t launch_error_final(const double *partial, long nb, unsigned long long *out, hipStream_t s)

@@ -1105,12 +1105,12 @@ __device__ __forceinline__ double stage_err_specials(const StageArgs &a, long bl
 // leaves idle), k7 = d rho/dt comes from LDS natural layout; same lane ->
 // entry mapping as load_rho, two entries' loads in flight at a time.
 template <int N, int LR, class Lay = SwLay<N>>
-__device__ __forceinline__ double stage_err(const StageArgs &a, const cd *lds, long blk)
+__device__ __forceinline__ ErrMax stage_err(const StageArgs &a, const cd *lds, long blk)
 {
     using G = Geo<N, LR>;
     const int n = a.n;
     const long k0 = first_k<N, LR>(blk);
-    double v = 0;
+    ErrMax v;
     constexpr int IT = G::KPW * G::NN / 64;
 #pragma unroll 2
     for (int u = 0; u < IT; u++) {
@@ -1125,10 +1125,11 @@ __device__ __forceinline__ double stage_err(const StageArgs &a, const cd *lds, l
             for (int j = 0; j < 5; j++) kv[j] = load(a.in.k[j]);
             const cd d = lds[e.kk * Lay::MS + Lay::at(e.r, e.c)];
             kv[5] = make_double2(d.x, d.y);
-            v = fmax(v, err_entry(load(a.in.x), kv, a.err_e, a.err_ea, a.err_er, a.err_dt));
+            v.add(err_entry(load(a.in.x), kv, a.err_e, a.err_ea, a.err_er, a.err_dt));
         }
     }
-    return fmax(v, stage_err_specials(a, blk));
+    v.add(stage_err_specials(a, blk));
+    return v;
 }
 
 // special slots of the stage: d A_t/dt = -E_t (t < dim), and the stage input
@@ -1286,7 +1287,7 @@ __device__ __forceinline__ void rhs_stage_body16(const StageArgs &a, const long 
     wsync();
     store_state<N, LR>(a.dxdt, S0, n, a.P, a.nk, blk);
     if (a.err_partial) {
-        const double v = seg_max<64>(stage_err<N, LR>(a, S0, blk));
+        const double v = stage_err<N, LR>(a, S0, blk).wave();
         if (threadIdx.x == 0) a.err_partial[blk] = v;
     }
 }
@@ -2014,7 +2015,7 @@ __device__ __forceinline__ void rhs_stage_body_acc(const StageArgs &a, const lon
     }
     store(a.dxdt, D);
     if (a.err_partial) {
-        double v = 0;
+        ErrMax err;
         if constexpr (AHEAD) {  // all loads in one trip
             double2 kv[F::E][6], xv[F::E];
 #pragma unroll
@@ -2026,7 +2027,7 @@ __device__ __forceinline__ void rhs_stage_body_acc(const StageArgs &a, const lon
             }
 #pragma unroll
             for (int j = 0; j < F::E; j++)
-                if (own[j] && kin) v = fmax(v, err_entry(xv[j], kv[j], a.err_e, a.err_ea, a.err_er, a.err_dt));
+                if (own[j] && kin) err.add(err_entry(xv[j], kv[j], a.err_e, a.err_ea, a.err_er, a.err_dt));
         } else {
 #pragma unroll 2
             for (int j = 0; j < F::E; j++)
@@ -2035,11 +2036,11 @@ __device__ __forceinline__ void rhs_stage_body_acc(const StageArgs &a, const lon
 #pragma unroll
                     for (int d = 0; d < 5; d++) kv[d] = load(a.in.k[d] + 2 * kst, j);
                     kv[5] = make_double2(D.r[j], D.i[j]);
-                    v = fmax(v, err_entry(load(a.in.x + 2 * kst, j), kv, a.err_e, a.err_ea, a.err_er, a.err_dt));
+                    err.add(err_entry(load(a.in.x + 2 * kst, j), kv, a.err_e, a.err_ea, a.err_er, a.err_dt));
                 }
         }
-        v = fmax(v, stage_err_specials(a, blk));
-        v = seg_max<64>(v);
+        err.add(stage_err_specials(a, blk));
+        const double v = err.wave();
         if (threadIdx.x == 0) a.err_partial[blk] = v;
     }
 }
@@ -2223,7 +2224,7 @@ __device__ __forceinline__ void rhs_stage_body_r1(const StageArgs &a, const long
     wsync();
     store_state<N, 1, Lay>(a.dxdt, S, n, a.P, a.nk, blk);
     if (a.err_partial) {
-        const double v = seg_max<64>(stage_err<N, 1, Lay>(a, S, blk));
+        const double v = stage_err<N, 1, Lay>(a, S, blk).wave();
         if (threadIdx.x == 0) a.err_partial[blk] = v;
     }
 }
@@ -2381,7 +2382,7 @@ __device__ __forceinline__ void rhs_stage_body(const StageArgs &a, const long bl
     wsync();
     store_state<N, LR>(a.dxdt, S0, n, a.P, a.nk, blk);
     if (a.err_partial) {
-        const double v = seg_max<64>(stage_err<N, LR>(a, S0, blk));
+        const double v = stage_err<N, LR>(a, S0, blk).wave();
         if (threadIdx.x == 0) a.err_partial[blk] = v;
     }
     }
@@ -2598,14 +2599,13 @@ __global__ __launch_bounds__(64) void rhs_stage_set_kernel(
         if (t + 1 == gridDim.x) {
             __threadfence();
             const double *part = ss.st[ss.m - 1].err_partial;
-            double v = 0;
+            ErrMax all;
             for (unsigned i = threadIdx.x; i < gridDim.x; i += 64)
-                v = fmax(v, __hip_atomic_load(part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-            v = seg_max<64>(v);
+                all.add(__hip_atomic_load(part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            const double v = all.wave();
             if (threadIdx.x == 0) {
                 __hip_atomic_store(ss.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(ss.err_out, (unsigned long long)__double_as_longlong(v), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_SYSTEM);
+                store_error(ss.err_out, v);
             }
         }
     }
