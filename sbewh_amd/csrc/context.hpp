@@ -241,13 +241,14 @@ struct sbe_ctx {
     // (chain_kernels.hip), with no layout to tune and no eigenvector cache: a
     // quarter to half of the general path's time on 256 k, and a smaller share of
     // it the larger the grid.  A sweep bound of 0 (no rotation after the first
-    // call) and a layout forced through SBEWH_STAGE_LR keep the general path;
-    // decided at the first use, as the layout is.
+    // call) and a layout forced through SBEWH_STAGE_LR keep the general path.  A
+    // layout that the resident integrator had timed for itself is no reason: what
+    // ran before on a context must not change its results.
     int chain_mode = -1;
     bool chain()
     {
         if (chain_mode < 0) {
-            chain_mode = dim == 1 && n == 2 && prm.sweep_count > 0 && !lr;
+            chain_mode = dim == 1 && n == 2 && prm.sweep_count > 0 && !lr_forced;
             int lrs[8];
             if (const char *env = std::getenv("SBEWH_STAGE_LR"))
                 for (int v = 0, nv = stage_variants(N, lrs, 8); v < nv; v++)

@@ -85,3 +85,36 @@ def test_resident_not_taken_for_2d_or_with_step_log():
     assert not r["device_controller"]
     g.close()
     o.close()
+
+
+def test_resident_leaves_the_chain_path_alone():
+    """a two-band chain gives the same bits whether or not its context ran the resident
+    integrator before, and where that one declines a grid too large for it"""
+    from tests.test_gpu_chain import chain, state
+    cfg = chain(4, 256, 16, device_controller=True)
+    o = Oracle(dataclasses.replace(cfg, device_controller=False))
+    x0 = state(o)
+    o.close()
+    out = []
+    for first in (False, True):
+        g = SBEContext(cfg)
+        if first:
+            assert g.integrate(x0.copy(), 9, log_capacity=0)["device_controller"]
+        x = x0.copy()
+        r = g.integrate(x, 9)
+        assert not r["device_controller"]
+        out.append((g.rhs(x0, 0.5), g.observe(x0), r["j"], x))
+        g.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    say("[gpu] resident integrator: a chain of 2^19 k")
+    out = []
+    for device in (False, True):
+        g = SBEContext(chain(1, 2 ** 19, 4, device_controller=device, output_count=3))
+        x = g.initial_state(0.0)
+        r = g.integrate(x, 3, log_capacity=0)
+        assert not r["device_controller"]
+        out.append((r["j"], x))
+        g.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
