@@ -181,6 +181,8 @@ struct StageArgs {
     double *err_partial;
     double err_e[6];
     double err_ea, err_er, err_dt;
+    // false: a decomposition by rotations alone
+    __host__ __device__ bool refines() const { return !dephase || (warm && sweeps != 1); }
 };
 // N: padded band count (2, 4, 8, 16); LR: lanes per matrix row (layout variant)
 hipError_t launch_rhs_stage(int N, int LR, const StageArgs &a, hipStream_t s);
@@ -205,8 +207,9 @@ int stage_variants(int N, int *lr_out, int cap);
 // k-points per block (one wavefront) of layout (N, LR)
 int stage_k_per_block(int N, int LR);
 // entry j owns the logical blocks [block0[j], block0[j+1]) (ceil(nk_j / k_per_block) each)
-hipError_t launch_rhs_stage_batched(int N, int LR, int n, const StageArgs *d_args, const long *d_block0, int m, long blocks,
-                                    hipStream_t s);
+// (refines: some entry's StageArgs::refines())
+hipError_t launch_rhs_stage_batched(int N, int LR, int n, bool refines, const StageArgs *d_args, const long *d_block0, int m,
+                                    long blocks, hipStream_t s);
 
 struct InitArgs {
     const double *mesh;    // [k][ops][n*n], H0 = op 0

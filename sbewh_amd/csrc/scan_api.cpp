@@ -184,6 +184,11 @@ struct sbe_scan {
         }
     }
 
+    static bool any_refines(const std::vector<StageArgs> &args)
+    {
+        return std::any_of(args.begin(), args.end(), [](const StageArgs &a) { return a.refines(); });
+    }
+
     // dxdt = f(rho_in, t) for every request (queued)
     void rhs(const std::vector<RhsReq> &rq)
     {
@@ -244,7 +249,8 @@ struct sbe_scan {
         long *db = add(b0.data(), m);
         stage_b0 = db;
         stage_blocks = tot;
-        enqueue([=] { HIPCHK(launch_rhs_stage_batched(N, lr, n, da, db, m, tot, stream)); });
+        const bool refines = any_refines(args);
+        enqueue([=] { HIPCHK(launch_rhs_stage_batched(N, lr, n, refines, da, db, m, tot, stream)); });
         for (int j = 0; j < m; j++) {
             if (args[j].dephase) rq[j].c->ucache_valid = true;
             rq[j].c->rhs_calls++;
@@ -273,6 +279,7 @@ struct sbe_scan {
         }
         const int m = (int)args.size();
         for (auto &a : args) a.warm = 0;
+        const bool refines = any_refines(args);
         StageArgs *da = add(args.data(), m);
         run();  // the phase sums that the timed launches read
         float best = 1e30f;
@@ -287,9 +294,9 @@ struct sbe_scan {
             }
             long *db = add(b0.data(), m);
             flush();
-            HIPCHK(launch_rhs_stage_batched(N, lrs[v], n, da, db, m, tot, stream));
+            HIPCHK(launch_rhs_stage_batched(N, lrs[v], n, refines, da, db, m, tot, stream));
             HIPCHK(hipEventRecord(ev[0], stream));
-            for (int it = 0; it < 3; it++) HIPCHK(launch_rhs_stage_batched(N, lrs[v], n, da, db, m, tot, stream));
+            for (int it = 0; it < 3; it++) HIPCHK(launch_rhs_stage_batched(N, lrs[v], n, refines, da, db, m, tot, stream));
             HIPCHK(hipEventRecord(ev[1], stream));
             HIPCHK(hipEventSynchronize(ev[1]));
             float ms = 0;

@@ -1155,8 +1155,8 @@ __device__ __forceinline__ void stage_specials(const StageArgs &a, const long bl
     }
 }
 
-// The stage for 16 bands at two lanes per row: the Jacobi in the XOR-wrapped
-// register layout, every matrix product on the matrix cores, one k-point of the block
+// The stage for 16 bands by rotations, at two or four lanes per row: the Jacobi in
+// the XOR-wrapped register layout, every matrix product on the matrix cores, one k-point of the block
 // at a time with all 64 lanes.  A product's result stays in its accumulator
 // and feeds the next product as an operand (acc_right, acc_left_dagger), so
 // two LDS matrices per k-point suffice (8.9 KB for one k-point per block:
@@ -2239,10 +2239,10 @@ __device__ __forceinline__ void rhs_stage_body(const StageArgs &a, const long bl
     if constexpr (N == 8 && LR == 8) {
         rhs_stage_body_acc<FragOne, AHEAD>(a, blk);
         return;
-    } else if constexpr (N == 16 && LR == 12) {  // (12: a name, not a row layout)
+    } else if constexpr (N == 16 && LR == 12) {  // (12 and 16: names, not row layouts)
         rhs_stage_body_acc<Frag12, AHEAD>(a, blk);
         return;
-    } else if constexpr (N == 16 && LR == 4) {
+    } else if constexpr (N == 16 && LR == 16) {
         rhs_stage_body_acc<Frag16, AHEAD>(a, blk);
         return;
     } else if constexpr (N == 8 && LR == 2 && PAIR) {
@@ -2388,11 +2388,12 @@ __device__ __forceinline__ void rhs_stage_body(const StageArgs &a, const long bl
     }
 }
 
-// minimum waves per SIMD the register allocation must allow: the 8-band kernels
-// at one and two lanes per row and the 16-band kernel at four fit three (at most 168
-// VGPRs; a fourth wave of the latter costs spills, see refine)
+// minimum waves per SIMD the register allocation must allow: the 16-band rotations
+// at four lanes per row fit four (128 VGPRs); the refined 16-band kernels (a fourth
+// wave costs spills, see refine) and the 8-band ones at one and two lanes per row three
+// (at most 168)
 template <int N, int LR>
-constexpr int stage_min_waves() { return (N == 16 && LR >= 4) || (N == 8 && LR <= 2) ? 3 : 1; }
+constexpr int stage_min_waves() { return N == 16 && LR == 4 ? 4 : (N == 16 && LR > 4) || (N == 8 && LR <= 2) ? 3 : 1; }
 
 template <int N, int LR>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(stage_min_waves<N, LR>())))

@@ -130,6 +130,12 @@ int stage_variants(int N, int *lr_out, int cap)
 // 6.9 -> 4.6 ms, 900 8.3 -> 6.5 ms, 1296 8.4 -> 9.2 ms, 2025 9.5 -> 11.7 ms.
 constexpr long ONE_K_MOST = 1024;
 
+// 16 bands at four lanes per row: a launch of decompositions that rotations make alone
+// (from the identity, or under a bound of one) takes the kernel that does nothing else,
+// at four waves per SIMD; without a decomposition the refined kernel is the faster one.
+// Four right-hand sides, rotations inside the refined kernel -> by themselves: from the
+// identity 12.86 -> 12.31 ms on 48^3 k, 16 bands, and 627 -> 590 us on 63 x 63 k, 13 bands;
+// under a bound of one 5.71 -> 5.46 ms and 263 -> 248 us.
 hipError_t launch_rhs_stage(int N, int LR, const StageArgs &a, hipStream_t s)
 {
     switch (N * 100 + LR) {
@@ -144,7 +150,9 @@ hipError_t launch_rhs_stage(int N, int LR, const StageArgs &a, hipStream_t s)
         return a.nk <= ONE_K_MOST && !a.err_partial ? launch_rhs_NL<8, 8>(a, s) : launch_rhs_NL<8, 2>(a, s);
     case 804: return launch_rhs_NL<8, 4>(a, s);
     case 1602: return launch_rhs_NL<16, 2>(a, s);
-    case 1604: return a.n <= 12 ? launch_rhs_NL<16, 12>(a, s) : launch_rhs_NL<16, 4>(a, s);
+    case 1604:
+        if (!a.refines()) return launch_rhs_NL<16, 4>(a, s);
+        return a.n <= 12 ? launch_rhs_NL<16, 12>(a, s) : launch_rhs_NL<16, 16>(a, s);
     }
     return hipErrorInvalidValue;
 }
@@ -161,13 +169,15 @@ hipError_t launch_rhs_stage_set(int N, int LR, const StageSet &ss, hipStream_t s
     case 802: return ss.st[0].nk <= ONE_K_MOST ? launch_rhs_set_NL<8, 8>(ss, s) : launch_rhs_set_NL<8, 2>(ss, s);
     case 804: return launch_rhs_set_NL<8, 4>(ss, s);
     case 1602: return launch_rhs_set_NL<16, 2>(ss, s);
-    case 1604: return ss.st[0].n <= 12 ? launch_rhs_set_NL<16, 12>(ss, s) : launch_rhs_set_NL<16, 4>(ss, s);
+    case 1604:
+        if (!ss.st[ss.m - 1].refines()) return launch_rhs_set_NL<16, 4>(ss, s);
+        return ss.st[0].n <= 12 ? launch_rhs_set_NL<16, 12>(ss, s) : launch_rhs_set_NL<16, 16>(ss, s);
     }
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_rhs_stage_batched(int N, int LR, int n, const StageArgs *args, const long *block0, int m, long blocks,
-                                    hipStream_t s)
+hipError_t launch_rhs_stage_batched(int N, int LR, int n, bool refines, const StageArgs *args, const long *block0, int m,
+                                    long blocks, hipStream_t s)
 {
     switch (N * 100 + LR) {
     case 201: return launch_rhs_stage_batched_r1(2, args, block0, m, blocks, s);
@@ -180,8 +190,9 @@ hipError_t launch_rhs_stage_batched(int N, int LR, int n, const StageArgs *args,
     case 804: return launch_rhs_batched_NL<8, 4>(args, block0, m, blocks, s);
     case 1602: return launch_rhs_batched_NL<16, 2>(args, block0, m, blocks, s);
     case 1604:
+        if (!refines) return launch_rhs_batched_NL<16, 4>(args, block0, m, blocks, s);
         return n <= 12 ? launch_rhs_batched_NL<16, 12>(args, block0, m, blocks, s)
-                       : launch_rhs_batched_NL<16, 4>(args, block0, m, blocks, s);
+                       : launch_rhs_batched_NL<16, 16>(args, block0, m, blocks, s);
     }
     return hipErrorInvalidValue;
 }

@@ -237,3 +237,28 @@ def test_scan_9_to_12_bands(n):
         assert r["steps"][i] == s["steps"]
         assert np.abs(r["j"][i] - s["j"]).max() <= 1e-12 * np.abs(s["j"]).max()
         g.close()
+
+
+@pytest.mark.parametrize("n", [9, 13, 16])
+def test_from_the_identity_16_bands(n, monkeypatch):
+    """decompositions by rotations alone at four lanes per row: single right-hand sides,
+    attempts in one launch and batched ones"""
+    monkeypatch.setenv("SBEWH_STAGE_LR", "4")
+    cfg = dataclasses.replace(config(n, (1, 1), (5, 4), (5, 4), eps_rel=1e-7, T2_fs=10.0, output_count=4, cold_jacobi=True),
+                              pulses=model.elliptic_sin2(1.0, 0.4, 3000.0, 0.1))
+    half = n // 2   # a gap between the halves
+    cfg.model.H[len(cfg.model.cells) // 2] += np.diag(np.where(np.arange(n) < half, -2.0, 2.0))
+    cfg = dataclasses.replace(cfg, occupied_bands=half)
+    check_sequence(cfg, [0.0, 0.01, 0.6])
+    g, o = SBEContext(cfg), Oracle(cfg)
+    a = o.initial_state(o.fermi_level(half))
+    b, c = a.copy(), a.copy()
+    ro = o.integrate(a, 4)
+    rg = g.integrate(b, 4, replay=ro["log"])
+    assert np.abs(rg["j"] - ro["j"]).max() < 1e-10 * np.abs(ro["j"]).max()
+    assert np.abs(b - a).max() < 1e-10 * np.abs(a).max()
+    s, r = g.integrate(c, 4), Scan([cfg, dataclasses.replace(cfg, Nk=(10, 8, 1))]).run(4)
+    assert r["steps"][0] == s["steps"]
+    assert np.abs(r["j"][0] - s["j"]).max() <= 1e-10 * np.abs(s["j"]).max()
+    o.close()
+    g.close()
