@@ -1579,9 +1579,15 @@ __device__ __forceinline__ double rcp_newton(double x)
 // bands: their block only looks coupled until the others are gone) it waits for the
 // next iteration, and up to 4 thr, the rounding of the products, it stays;
 // otherwise (a near crossing) the wavefront is left to the Jacobi rotations: the
-// result is false.  So it is when the bound on the iterations ends the last one with
-// x > XR, where the non-orthonormality left, x^4 / 4 an element, adds up to more than
-// rounding: the rotations leave U unitary whatever their bound.  A bound of one is
+// result is false, and as_came whether U is still the previous call's and H0 now
+// U H0 U^dagger.  It does not wait for others with x > XW either: with steps that
+// large nearly every k-point ended at the rotations all the same, an iteration or two
+// later (four right-hand sides, A moved by 0.02 a.u. a call: 14.0 -> 12.3 ms on 48^3 k,
+// 16 bands, 569 -> 509 us on 63 x 63 k, 11 bands; rotations alone from the same warm
+// start, at four waves per SIMD, 11.4 ms and 496 us).  It is false as well when the
+// bound on the iterations ends the last one with x > XR, where the non-orthonormality
+// left, x^4 / 4 an element, adds up to more than rounding: the rotations leave U
+// unitary whatever their bound.  A bound of one is
 // theirs altogether (the caller's rule): a single iteration never sees the
 // non-orthonormality it made, and 1500 warm calls in a row left a trace of 2e-6
 // (8 bands) to 4e-5 (14) in the dephasing term, now 1e-15.
@@ -1598,10 +1604,10 @@ __device__ __forceinline__ double rcp_newton(double x)
 // latency counts, 8.1 -> 7.2 ms per propagation against four lanes per row.
 // With every band twofold degenerate: 362 -> 278 us and 46.7 -> 33.2 ms.
 template <class F>
-__device__ __forceinline__ bool refine(cd *buf, const cd *H0, const AccPos &pos, typename F::Acc &U, typename F::Acc &Q, double *Dgs,
-                                       int sweeps)
+__device__ __forceinline__ bool refine(cd *buf, cd *H0, const AccPos &pos, typename F::Acc &U, typename F::Acc &Q, double *Dgs,
+                                       int sweeps, bool &as_came)
 {
-    constexpr double XB = 0.1, XF = 4e-6, XR = 1e-4, X2 = 1e-8, RF = 1e-14;
+    constexpr double XB = 0.1, XW = 0.03, XF = 4e-6, XR = 1e-4, X2 = 1e-8, RF = 1e-14;
     double *Dg = Dgs + F::kk() * F::N;
     double thr2 = 0;
     for (int it = 0;; it++) {
@@ -1672,7 +1678,7 @@ __device__ __forceinline__ bool refine(cd *buf, const cd *H0, const AccPos &pos,
                     e2 = fmax(e2, fma(E.r[j], E.r[j], E.i[j] * E.i[j]));
                 }
             }
-            const double second2 = F::N * F::N * F::max(e2) * F::max(x2);
+            const double xk = F::max(x2), second2 = F::N * F::N * F::max(e2) * xk;
 #pragma unroll
             for (int j = 0; j < F::E; j++)
                 if (fma(X.r[j], X.r[j], X.i[j] * X.i[j]) > XB * XB) {
@@ -1680,12 +1686,13 @@ __device__ __forceinline__ bool refine(cd *buf, const cd *H0, const AccPos &pos,
                     X.r[j] = X.i[j] = rd[j] = 0;
                     if (m2 > 16 * thr2) {
                         wait = true;
-                        bad = bad || !(m2 <= second2);
+                        bad = bad || !(m2 <= second2) || xk > XW * XW;
                     }
                 }
             bad = __any(bad);
             wait = __any(wait);
         }
+        as_came = bad && it == 0;
         const bool second = __any(x2 > X2 * X2);
         typename F::Acc V;  // the adjoint of the update: 1 - X + R/2 + (X - R) X / 2
         cacc_zero(V);
@@ -1721,6 +1728,12 @@ __device__ __forceinline__ bool refine(cd *buf, const cd *H0, const AccPos &pos,
             F::cmul(x, y, V);
         }
         if (bad) {
+            if (as_came) {
+                // S: its off-diagonal is E, its diagonal Dg
+#pragma unroll
+                for (int j = 0; j < F::E; j++)
+                    H0[pos.nat + F::nat_step(j)] = mk(F::row(j) != F::col(j) ? E.r[j] : Dg[F::col(j)], E.i[j]);
+            }
             wsync();
             return false;
         }
@@ -1844,12 +1857,12 @@ __device__ __forceinline__ void rhs_stage_body_acc(const StageArgs &a, const lon
                 U.i[j] = own[j] ? v.y : 0.0;
             }
         };
-        bool rotate = true;
+        bool rotate = true, as_came = false;
         if (a.warm) load_prev();
         phase_put(0, S1);
         if (a.warm) {
             acc_dagger<F>(S0, pos, U, Q);  // (its sync orders the store of H0 too)
-            rotate = a.sweeps == 1 || !refine<F>(S0, S1, pos, U, Q, Dgs, a.sweeps);
+            rotate = a.sweeps == 1 || !refine<F>(S0, S1, pos, U, Q, Dgs, a.sweeps, as_came);
         } else {
             wsync();
         }
@@ -1868,24 +1881,26 @@ __device__ __forceinline__ void rhs_stage_body_acc(const StageArgs &a, const lon
             constexpr bool SAME = KPW < G::KPW;
             const Lane L = SAME ? lane_id<N, LR>(G::KPW, 0) : lane_id<N, LR>(a.nk, blk);
             cd A[C], V[C], *sk = S0 + (SAME ? 0 : L.kk) * G::NN;
-            typename F::Acc S;
             if (a.warm) {
-                // S = U H0 U^dagger of the previous call's U
                 load_prev();
-                acc_dagger<F>(S0, pos, U, Q);
-                typename F::Acc h, t;
-                acc_get<F>(S1, pos, h);
-                cacc_zero(t);
-                mul_dagger<F>(h, Q, t);
-                cacc_zero(S);
-                mul_dagger<F>(Q, t, S);
+                if (!as_came) {
+                    // H0 -> U H0 U^dagger of the previous call's U
+                    acc_dagger<F>(S0, pos, U, Q);
+                    typename F::Acc h, t;
+                    acc_get<F>(S1, pos, h);
+                    cacc_zero(t);
+                    mul_dagger<F>(h, Q, t);
+                    cacc_zero(h);
+                    mul_dagger<F>(Q, t, h);
+                    acc_put<F>(S1, pos, h);
+                }
                 put_sw(U, 1);
                 wsync();
                 load_u<N, LR>(sk, L, V);
                 wsync();
-            } else {
-                acc_get<F>(S1, pos, S);
             }
+            typename F::Acc S;
+            acc_get<F>(S1, pos, S);
             put_sw(S, 0);
             wsync();
             load_xrow<N, LR>(sk, L, A);
