@@ -1320,6 +1320,12 @@ struct Frag16 {
     static __device__ __forceinline__ double sum(double v) { return seg_sum<64>(v); }
     static __device__ __forceinline__ double max(double v) { return __shfl(seg_max<64>(v), 0); }
     static __device__ __forceinline__ void cmul(const cd *a, const cd *b, CAcc &acc) { mfma_cmul(a, b, acc); }
+    // acc += a b + c d
+    static __device__ __forceinline__ void cmul2(const cd *a, const cd *b, const cd *c, const cd *d, CAcc &acc)
+    {
+        mfma_cmul(a, b, acc);
+        mfma_cmul(c, d, acc);
+    }
     // left operand M^dagger
     static __device__ __forceinline__ void cmul_dagger(const CAcc &m, const cd *b, CAcc &acc)
     {
@@ -1337,6 +1343,11 @@ struct Frag16 {
 struct Frag12 : Frag16 {
     static constexpr int E = 3;
     static __device__ __forceinline__ void cmul(const cd *a, const cd *b, CAcc &acc) { mfma_cmul<3>(a, b, acc); }
+    static __device__ __forceinline__ void cmul2(const cd *a, const cd *b, const cd *c, const cd *d, CAcc &acc)
+    {
+        mfma_cmul<3>(a, b, acc);
+        mfma_cmul<3>(c, d, acc);
+    }
     static __device__ __forceinline__ void cmul_dagger(const CAcc &m, const cd *b, CAcc &acc)
     {
         cd x[4];
@@ -1395,6 +1406,22 @@ struct Frag8 {
                 acc.r[j] = fms4(x.y, y.y, acc.r[j]);
                 acc.i[j] = fma4(x.y, y.x, acc.i[j]);
             }
+    }
+    // Each product by itself: summed on top of the first, the second's terms all round
+    // at the first's size (a commutator's error 9.4e-16 of its rms on 30 x 30 and 60 x 60 k,
+    // by itself 8.6e-16; no time).
+    static __device__ __forceinline__ void cmul2(const cd *a, const cd *b, const cd *c, const cd *d, CAcc &acc)
+    {
+        CAcc p, q;
+        cacc_zero(p);
+        cacc_zero(q);
+        cmul(a, b, p);
+        cmul(c, d, q);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            acc.r[j] += p.r[j] + q.r[j];
+            acc.i[j] += p.i[j] + q.i[j];
+        }
     }
     static __device__ __forceinline__ void cmul_dagger(const CAcc &m, const cd *b, CAcc &acc)
     {
@@ -1482,6 +1509,17 @@ struct FragOne {
     {
         step<0>(a[0], b[0], acc);
         step<1>(a[0], b[0], acc);
+    }
+    // as Frag8
+    static __device__ __forceinline__ void cmul2(const cd *a, const cd *b, const cd *c, const cd *d, Acc &acc)
+    {
+        Acc p, q;
+        cacc_zero(p);
+        cacc_zero(q);
+        cmul(a, b, p);
+        cmul(c, d, q);
+        acc.r[0] += p.r[0] + q.r[0];
+        acc.i[0] += p.i[0] + q.i[0];
     }
     template <int K>
     static __device__ __forceinline__ void step_dagger(const Acc &m, cd b, Acc &acc)
@@ -2008,20 +2046,18 @@ __device__ __forceinline__ void rhs_stage_body_acc(const StageArgs &a, const lon
         phase_put(1, S0);
         wsync();
         acc_get<F>(S0, pos, he);
-        cd x[F::REGS], y[F::REGS];
+        cd x[F::REGS], y[F::REGS], u[F::REGS], v[F::REGS];
 #pragma unroll
         for (int j = 0; j < F::E; j++) {
             t.r[j] = D.i[j];
             t.i[j] = -D.r[j];
-            const cd v = S0[pos.tr + F::tr_step(j)];
-            x[j] = mk(-v.x, -v.y);
+            const cd h = S0[pos.tr + F::tr_step(j)];
+            x[j] = mk(-h.x, -h.y);
+            u[j] = S1[pos.tr + F::tr_step(j)];
         }
         acc_right(rho, y);
-        F::cmul(x, y, t);  // - H_E rho
-#pragma unroll
-        for (int j = 0; j < F::E; j++) x[j] = S1[pos.tr + F::tr_step(j)];
-        acc_right(he, y);
-        F::cmul(x, y, t);  // + rho H_E
+        acc_right(he, v);
+        F::cmul2(x, y, u, v, t);  // - H_E rho + rho H_E
 #pragma unroll
         for (int j = 0; j < F::E; j++) {
             D.r[j] = -t.i[j];

@@ -220,6 +220,28 @@ def test_no_dephasing_8_bands(Nk, Nf, monkeypatch):
     check_sequence(config(7, (1, 1), Nk, Nf, T2_fs=0.0), [0.0, 0.01])
 
 
+@pytest.mark.parametrize("Nk", [(30, 30), (42, 30)])   # one and four k-points per wavefront
+def test_commutator_rounding_8_bands(Nk, monkeypatch):
+    """the matrix instructions' commutator is no further from one in long double than that
+    of the kernel at four lanes per row, which sums its two products apart (5 % for the
+    spread of the mean over some 60000 entries)"""
+    cfg = config(8, (2, 2), Nk, (6, 6), T2_fs=0.0)
+    cfg.model.H[len(cfg.model.cells) // 2] += np.diag([-1.0] * 4 + [1.0] * 4)
+    rms = []
+    for lr in ("4", "2"):
+        monkeypatch.setenv("SBEWH_STAGE_LR", lr)
+        g = SBEContext(cfg)
+        x = cases.perturbed_state(g.initial_state(0.0), 8, g.P, g.num_k, seed=3, amp=0.05)
+        H = g.hk_mesh(x[:3].real, g.E(3.0))[:, 1].astype(np.clongdouble)
+        rho = g.rho(x).astype(np.clongdouble)
+        ref = -1j * (np.einsum("kab,kbc->kac", H, rho) - np.einsum("kab,kbc->kac", rho, H))
+        err = np.abs(g.rho(g.rhs(x, 3.0)) - ref)
+        rms.append(float(np.sqrt((err ** 2).mean() / (np.abs(ref) ** 2).mean())))
+        g.close()
+    print(f"[gpu] commutator {Nk}: four lanes {rms[0]:.3e}, matrix instructions {rms[1]:.3e}", flush=True)
+    assert rms[1] <= 1.05 * rms[0]
+
+
 @pytest.mark.parametrize("n", [9, 12])
 def test_scan_9_to_12_bands(n):
     """two pulses in a scan against single runs: the same kernels and steps"""
