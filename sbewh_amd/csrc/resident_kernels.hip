@@ -9,13 +9,14 @@
 // the first factor formed once, the second per set from the stage input's A)
 // and its own copy of the six merged model boxes, so the grid meets only once
 // per attempt: after the last stage has left one error maximum per block.
-// Every block then reads
-// all maxima in the same order and runs the same step-size control on the
-// same bits, so all blocks take the same decisions and reach the same
-// barriers.  Per output interval: the current j(t) and the fresh stepper's
-// first derivative at its start, as the host controller does.  No host round
-// trip per attempt; the launch ends after the last output, after an error
-// norm that is NaN, 500 failed step sizes in a row, or an attempt limit.
+// Every block then reads all maxima, the lanes side by side (one load after the
+// other for all lanes took a fifth of an integration of 4 bands on 2048 k, 128
+// blocks: 6.4 -> 5.2 ms), and runs the same step-size control on the same bits, so
+// all blocks take the same decisions and reach the same barriers.  Per output
+// interval: the current j(t) and the fresh stepper's first derivative at its start,
+// as the host controller does.  No host round trip per attempt; the launch ends
+// after the last output, after an error norm that is NaN, 500 failed step sizes in
+// a row, or an attempt limit.
 #include <hip/hip_cooperative_groups.h>
 
 #include "dopri5.hpp"
@@ -367,8 +368,12 @@ __global__ __launch_bounds__(64) void resident_kernel(ResidentArgs r)
         rhs += 6;
         grid_sync(grid);
         ErrMax err;
-        for (long b = 0; b < nblk; b++) err.add(r.err_partial[b]);
-        return err.value();
+        for (long b = threadIdx.x; b < nblk; b += 64) err.add(r.err_partial[b]);
+        // (the same in all lanes; through scalar registers, so that the control flow that
+        // hangs on it stays wave-uniform)
+        const long long bits = __double_as_longlong(err.wave());
+        const int lo = __builtin_amdgcn_readfirstlane((int)bits), hi = __builtin_amdgcn_readfirstlane((int)(bits >> 32));
+        return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
     };
 
     {
