@@ -221,7 +221,8 @@ struct sbe_ctx {
     }
 
     PhaseBuffers pbufs() const { return PhaseBuffers{Hb, Db, dHb, kmap, tw, y1, y2}; }
-    PhaseLast last(const double *Yp) const { return PhaseLast{Yp, tw + 2 * twL_off, kphase, WL}; }
+    PhaseLast last(const double *Yp) const { return PhaseLast{Yp, tw + 2 * twL_off, kphase, WL, row_cells()}; }
+    int row_cells() const { return (long)geom.Nk[dim - 1] * WL <= 1L << 28 ? WL : NO_ROWS; }
     // the merged model box of the RHS (for dim == 1 it is the partial phase sum itself)
     double *merged() const { return dim == 1 ? Y : hm; }
     ModelMerge merge_of(const double E[3]) const
@@ -383,7 +384,7 @@ struct sbe_ctx {
     }
     PhaseLast last_set(int q) const
     {
-        return PhaseLast{Y6 + q * Y_stride, tw6 + q * tw_stride + 2 * twL_off, kphase, WL};
+        return PhaseLast{Y6 + q * Y_stride, tw6 + q * tw_stride + 2 * twL_off, kphase, WL, row_cells()};
     }
 
     void rhs_dev(const double *x_in, double *dxdt, double t, hipStream_t s)

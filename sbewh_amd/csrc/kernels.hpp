@@ -106,6 +106,8 @@ long phase_partial_scratch(const PhaseGeom &g, int ops);
 // twiddle offset (complex entries) of dimension d inside tw
 long twiddle_offset(const PhaseGeom &g, int d);
 
+constexpr int NO_ROWS = 17;  // PhaseLast::row_cells where phase_rows may not be used
+
 // Last-axis contraction of a partial phase sum for one k-point:
 //   X(k)[e] = sum_r twL[kphase[k].y + r] Y[(kphase[k].x + r) M + op nn + e]
 // with kphase[k] = (rest(k) W_L, i_L(k) W_L).
@@ -114,6 +116,9 @@ struct PhaseLast {
     const double *twL;     // [Nk_L][W_L]
     const int *kphase;     // int2 per k
     int WL;
+    // W_L for phase_rows (at most 16 cells), or NO_ROWS: twL beyond 4 GB (its offsets have
+    // 32 bits), or made in the same launch (its loads are scalar ones)
+    int row_cells;
 };
 
 // ---- batched forms: several instances (own grid, pulse, buffers) per launch

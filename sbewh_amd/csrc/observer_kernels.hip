@@ -106,7 +106,7 @@ __device__ __forceinline__ void jk_rows_body(const ObsArgs &a, const long blk)
         for (int q = 0; q < WL; q++) {
             sd2 tw[KB];
 #pragma unroll
-            for (int kk = 0; kk < KB; kk++) tw[kk] = load_const<sd2>(a.ph.twL, tp[kk] + q);
+            for (int kk = 0; kk < KB; kk++) tw[kk] = load_const<sd2>(reinterpret_cast<const sd2 *>(a.ph.twL) + tp[kk], q);
 #pragma unroll
             for (int d = 0; d < 3; d++)
                 if (d < a.dim) {

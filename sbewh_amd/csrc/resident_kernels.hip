@@ -117,7 +117,7 @@ __device__ __forceinline__ StageArgs stage_args(const ResidentArgs &r, const Sta
     StageArgs a{};
     a.in = in;
     a.dxdt = dxdt;
-    a.ph = PhaseLast{box_of(r, blockIdx.x, set), r.tw6 + set * r.tw_stride + 2 * r.twL_off, r.kphase, r.WL};
+    a.ph = PhaseLast{box_of(r, blockIdx.x, set), r.tw6 + set * r.tw_stride + 2 * r.twL_off, r.kphase, r.WL, NO_ROWS};
     a.nk = r.nk;
     a.n = r.n;
     a.P = r.P;
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(64) void resident_kernel(ResidentArgs r)
         if (out < r.output_count) {
             ObsArgs o{};
             o.x = s.x;
-            o.ph = PhaseLast{r.Yobs, r.tw6 + 2 * r.twL_off, r.kphase, r.WL};
+            o.ph = PhaseLast{r.Yobs, r.tw6 + 2 * r.twL_off, r.kphase, r.WL, NO_ROWS};
             o.nk = r.nk;
             o.n = r.n;
             o.P = r.P;

@@ -177,7 +177,9 @@ __device__ __forceinline__ void load_mats(cd *lds, const double *src, long strid
 }
 
 // loads through the constant address space: with a wave-uniform address they
-// are scalar loads.  Only for memory that no kernel of the same launch writes.
+// are scalar loads.  Only for memory that no kernel of the same launch writes, and
+// within 4 GB of p (64-bit offsets cost 3 to 4 % of four right-hand sides on 150 x 150 k,
+// 8 bands, in scalar instructions).  The phase map of a state that fits the GPU is.
 typedef double sd2 __attribute__((ext_vector_type(2)));
 typedef int si2 __attribute__((ext_vector_type(2)));
 template <class V>
@@ -227,8 +229,7 @@ __device__ __forceinline__ void phase_map(const PhaseLast &ph, long nk, int k0, 
 // it, QG cells in one memory trip.  Consecutive k-points share rest(k) along a
 // Fourier block's last axis, so a wavefront has one or two distinct rows; each gets
 // a pass.
-// false, with nothing done, for an R box wider than 16 cells along the last
-// axis.  Sums in the order of phase_mats.
+// false, with nothing done, for more than 16 row cells (PhaseLast).  Sums in the order of phase_mats.
 // Why: one wave-uniform branch and one memory trip per cell and pair of entries
 // (104 in series for 8 bands and 13 cells) kept the 8-band kernel waiting; four
 // right-hand sides on 150 x 150 k, 8 bands: 362 -> 316 us, an integration there
@@ -248,7 +249,7 @@ __device__ __forceinline__ bool phase_rows(cd *acc, const PhaseLast &ph, long nk
     // cells whose twiddles are fetched together (SGPRs), cells per memory trip (VGPRs)
     constexpr int QT = KPW >= 8 ? 1 : EO == 1 ? 4 : 2;
     constexpr int QG = NOP > 1 ? 32 / EK : KPW >= 8 ? 4 : KPW == 4 ? 8 : QT;
-    const int WL = ph.WL;
+    const int WL = ph.row_cells;
     if (WL > 16) return false;
     const int kf = __builtin_amdgcn_readfirstlane((int)k0);
     const double2 *Yb = reinterpret_cast<const double2 *>(ph.Y) + off;

@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 from oracle.oracle_py import Oracle
-from sbewh_amd import model
+from sbewh_amd import hiprt, model
 from sbewh_amd.propagator import SBEContext
 from tests import cases
 
@@ -87,4 +87,49 @@ def test_full_size_propagation_invariants():
     say(f"  A(t_end) {A}, -int E {-integral}, peak |A| {peak:.3e}")
     assert peak > 0.1
     assert np.abs(A + integral).max() < 1e-8 * peak
+    g.close()
+
+
+def test_twiddle_table_beyond_4_gb():
+    """a 1-D grid whose 16 twiddles a k-point take more than 4 GB (17 million k, 5 bands): the
+    last k-points' right-hand side against direct sums over R.  No dephasing: the commutator
+    alone shows H_E(k)."""
+    n, W, nk = 5, 16, 17_000_000
+    rng = np.random.default_rng(8)
+    cells = np.array([(r, 0, 0) for r in range(-8, 8)], np.int32)
+    f = np.exp(-np.abs(cells[:, 0]) / 4)[:, None, None] * 0.1
+    H = f * (rng.normal(size=(W, n, n)) + 1j * rng.normal(size=(W, n, n)))
+    D = np.zeros((W, 3, n, n), complex)
+    D[:, 0] = f * (rng.normal(size=(W, n, n)) + 1j * rng.normal(size=(W, n, n)))
+    m = model.TBModel(cells, H, D, np.eye(3) * 5.0)
+    cfg = model.Config("long", m, 1, (nk, 1, 1), (16, 1, 1), model.elliptic_sin2(1.0, 0.0, 3000.0, 4.0), T2_fs=0.0,
+                       gpu_layout=True)
+    say(f"[gpu] 1-D, {n} bands, {nk} k-points")
+    g = SBEContext(cfg)
+    rho = cases.random_hermitian(rng, 1, n, 0.3)[0]
+    x = np.empty(g.state_size, complex)
+    x[:8] = 0
+    x[0] = 0.2
+    x[8:].reshape(nk, n * n)[:] = rho.reshape(-1)
+    d = hiprt.DeviceBuffer.from_array(x.view(np.float64))
+    size = x.nbytes
+    del x
+    y, s = hiprt.DeviceBuffer(size), hiprt.Stream()
+    g.rhs_device(d.ptr, y.ptr, 3.0, s.handle)
+    s.synchronize()
+    count = 1000
+    out = np.empty(count * n * n, complex)
+    hiprt.check(hiprt.hip().hipMemcpy(out.ctypes.data, y.ptr + size - out.nbytes, out.nbytes, hiprt.D2H), "hipMemcpy")
+    # state order: blocks of 16 consecutive states, each 16 grid points nk / 16 apart
+    idx = np.arange(nk - count, nk)
+    grid = idx % 16 * (nk // 16) + idx // 16
+    k = grid / nk + 0.2 * 5.0 / (2 * np.pi)
+    ph = np.exp(2j * np.pi * k[:, None] * cells[:, 0])
+    HE = np.einsum("kr,rab->kab", ph, H + g.E(3.0)[0] * D[:, 0])
+    ref = -1j * (HE @ rho - rho @ HE)
+    assert (grid * W).max() >= 2 ** 28
+    assert rel(out.reshape(-1, n, n), ref) < 1e-12
+    s.destroy()
+    y.free()
+    d.free()
     g.close()
