@@ -36,9 +36,9 @@ hipError_t launch_gemm(const GemmArgs &g, int ta, int tb, int members, hipStream
 
 // X[e][b][:] = bf16(Xall[perm[e][(step % spe) * batch + b]]), T likewise (fp32);
 // step = *counter.  perm: [members][n_perm]; member e's rows start at row e * cap.
-// perm null: X[e][b][:] = bf16(Xall[first + b]) for every member.
+// perm null: X[e][b][:] = bf16(Xall[b]) for every member.
 hipError_t launch_gather(const float *Xall, const float *Tall, int din, int dout, const int *perm, long n_perm,
-                         const int *counter, int spe, int batch, int cap, int members, long first, bf16 *X, float *T,
+                         const int *counter, int spe, int batch, int cap, int members, bf16 *X, float *T,
                          hipStream_t s);
 // dY = 2 (Y - T) / (batch dout) in bf16; loss[e][*counter] = mean (Y - T)^2 (if loss != null;
 // slot 0 without a counter);

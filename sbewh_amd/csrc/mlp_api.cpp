@@ -338,7 +338,7 @@ int sbe_mlp_forward(sbe_mlp *mlp, int count, const float *x, float *y)
             const int rows = std::min(n.cap, count - s0);
             MCHK(hipMemcpyAsync(n.io_x, x + (size_t)s0 * din, (size_t)rows * din * sizeof(float),
                                 hipMemcpyHostToDevice, n.stream));
-            MCHK(launch_gather(n.io_x, n.io_x, din, 0, nullptr, 0, nullptr, 1, rows, n.cap, n.E, 0, n.X, n.T,
+            MCHK(launch_gather(n.io_x, n.io_x, din, 0, nullptr, 0, nullptr, 1, rows, n.cap, n.E, n.X, n.T,
                                n.stream));
             n.forward(rows);
             for (int e = 0; e < n.E; e++)
@@ -359,7 +359,7 @@ int sbe_mlp_gradient(sbe_mlp *mlp, int count, const float *x, const float *t, fl
         n.ensure_io(count);
         MCHK(hipMemcpyAsync(n.io_x, x, (size_t)count * din * sizeof(float), hipMemcpyHostToDevice, n.stream));
         MCHK(hipMemcpyAsync(n.io_t, t, (size_t)count * dout * sizeof(float), hipMemcpyHostToDevice, n.stream));
-        MCHK(launch_gather(n.io_x, n.io_t, din, dout, nullptr, 0, nullptr, 1, count, n.cap, n.E, 0, n.X, n.T,
+        MCHK(launch_gather(n.io_x, n.io_t, din, dout, nullptr, 0, nullptr, 1, count, n.cap, n.E, n.X, n.T,
                            n.stream));
         n.forward(count);
         MCHK(launch_loss_grad(n.Y, n.T, count, n.cap, dout, n.E, n.dY, n.io_loss, 1, nullptr, n.stream));
@@ -401,7 +401,7 @@ int sbe_mlp_train(sbe_mlp *mlp, int count, const float *x, const float *t, int b
             MCHK(hipStreamSynchronize(n.stream));
             // one training step of every member, captured once and replayed
             MCHK(hipStreamBeginCapture(n.stream, hipStreamCaptureModeThreadLocal));
-            MCHK(launch_gather(dx, dt, din, dout, dperm, count, n.counter, spe, batch, n.cap, n.E, 0, n.X, n.T, n.stream));
+            MCHK(launch_gather(dx, dt, din, dout, dperm, count, n.counter, spe, batch, n.cap, n.E, n.X, n.T, n.stream));
             n.forward(batch);
             MCHK(launch_loss_grad(n.Y, n.T, batch, n.cap, dout, n.E, n.dY, dl, (int)total, n.counter, n.stream));
             n.backward(batch);

@@ -171,21 +171,21 @@ hipError_t launch_gemm(const GemmArgs &g0, int ta, int tb, int members, hipStrea
 
 // grid (batch, members), block 64
 __global__ void gather_kernel(const float *Xall, const float *Tall, int din, int dout, const int *perm, long n_perm,
-                              const int *counter, int spe, int batch, int cap, long first, bf16 *X, float *T)
+                              const int *counter, int spe, int batch, int cap, bf16 *X, float *T)
 {
     const int b = blockIdx.x, e = blockIdx.y;
-    const long idx = perm ? perm[e * n_perm + (long)(*counter % spe) * batch + b] : first + b;
+    const long idx = perm ? perm[e * n_perm + (long)(*counter % spe) * batch + b] : b;
     const long row = (long)e * cap + b;
     for (int i = threadIdx.x; i < din; i += 64) X[row * din + i] = (bf16)Xall[idx * din + i];
     for (int i = threadIdx.x; i < dout; i += 64) T[row * dout + i] = Tall[idx * dout + i];
 }
 
 hipError_t launch_gather(const float *Xall, const float *Tall, int din, int dout, const int *perm, long n_perm,
-                         const int *counter, int spe, int batch, int cap, int members, long first, bf16 *X, float *T,
+                         const int *counter, int spe, int batch, int cap, int members, bf16 *X, float *T,
                          hipStream_t s)
 {
     hipLaunchKernelGGL(gather_kernel, dim3((unsigned)batch, (unsigned)members), dim3(64), 0, s, Xall, Tall, din, dout,
-                       perm, n_perm, counter, spe, batch, cap, first, X, T);
+                       perm, n_perm, counter, spe, batch, cap, X, T);
     return hipGetLastError();
 }
 

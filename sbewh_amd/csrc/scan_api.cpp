@@ -9,8 +9,12 @@
 // sum, fused stage kernel, error norm, observer), each kernel finding its
 // instance from a per-launch table of block offsets.  The host reads back one
 // error norm per instance per attempt.  Per instance, the arithmetic and the
-// step sequence are those of the single-instance path (same kernel bodies,
-// same controller), so a scan reproduces independent runs.
+// controller are those of the single-instance path, so a scan reproduces independent
+// runs to rounding.  Not to the bit in general: two-band chains run in registers by
+// themselves and on the general kernels here, 5 to 8 bands on at most 1024 k with one
+// k-point per wavefront by themselves and four here, which iterate a warm start
+// together, and layouts may be timed.  In a quiet interval, where the error norm is a
+// difference near rounding, the steps may part too, within the step tolerance.
 #include <array>
 #include <chrono>
 #include <functional>
