@@ -103,7 +103,9 @@ struct sbe_ctx {
     bool ucache_valid = false;
     bool resident_used = false;  // the last integration ran on the resident integrator
     double *err_partial = nullptr;
-    unsigned *err_ticket = nullptr;              // ticket of the fused attempt's last block (zero between launches)
+    // tickets of a launch's last block (zero between launches): of an attempt or an output,
+    // and of an observation on a caller's stream
+    unsigned *err_ticket = nullptr;
     unsigned long long *err_host = nullptr;      // pinned, mapped, fine-grained
     unsigned long long *err_host_dev = nullptr;  // its device address
     double *partial = nullptr;
@@ -819,8 +821,8 @@ inline void build(sbe_ctx *c, const sbe_model *m, const sbe_grid *g, const sbe_p
         c->y16 = dalloc<double>(SET_MAX * c->y1_stride);
     }
     c->err_partial = dalloc<double>(std::max(1024L, c->nk));  // one per stage block (>= 1 k-point each)
-    c->err_ticket = dalloc<unsigned>(1);
-    HIPCHK(hipMemset(c->err_ticket, 0, sizeof(unsigned)));
+    c->err_ticket = dalloc<unsigned>(2);
+    HIPCHK(hipMemset(c->err_ticket, 0, 2 * sizeof(unsigned)));
     // SBEWH_FUSE_BELOW overrides the stage-grid size under which an attempt's
     // stages share one launch (0: never, as for large grids)
     if (const char *env = std::getenv("SBEWH_FUSE_BELOW")) c->fuse_below_blocks = std::atol(env);

@@ -1,7 +1,7 @@
 // sbe_observe_device_noalloc: the current j(t) of a device state for callers
 // that cannot allocate device memory (code under HIP graph capture, tight
-// serving loops).  Same kernels and summation order as sbe_observe; the
-// per-k partial currents live in a file-scope device array instead of the
+// serving loops).  Same kernels and summation order as sbe_observe (two-band chains
+// included); the partial currents live in a file-scope device array instead of the
 // context's buffer, and the result goes to a caller-owned device buffer.
 #include <mutex>
 
@@ -49,6 +49,11 @@ extern "C" int sbe_observe_device_noalloc(sbe_ctx *ctx, const double *d_state, d
                  SCRATCH_DOUBLES / 3, c.nk);
         double *part = scratch_on(c.device);
         hipStream_t s = stream ? static_cast<hipStream_t>(stream) : c.stream;
+        if (c.chain()) {
+            // (a ticket of its own: the context's may be in use on the context's stream)
+            HIPCHK(launch_chain_output(c.chain_args(), d_state, d_j, part, nullptr, 0, c.err_ticket + 1, s));
+            return;
+        }
         StageInput in{};
         in.x = d_state;
         HIPCHK(launch_twiddles(c.geom, &in, 1, c.tw, s));

@@ -44,6 +44,19 @@ def test_noalloc_observe_equals_observe_twice_smaller_second():
         g.close()
 
 
+def test_noalloc_two_band_chain_equals_observe():
+    """identical bits for many states, one wavefront of k-points and several"""
+    for nk in (16, 256):
+        cfg = cases.chain(Nk=(nk, 1, 1))
+        g = SBEContext(cfg)
+        st = g.initial_state(g.fermi_level(cfg.occupied_bands))
+        for seed in range(12):
+            x = cases.perturbed_state(st, g.n, g.P, g.num_k, seed=seed, amp=0.1)
+            x[1] = 0
+            assert np.array_equal(noalloc_observe(g, x), g.observe(x)), (nk, seed)
+        g.close()
+
+
 def test_noalloc_rejects_grid_beyond_scratch():
     cfg = dataclasses.replace(cases.chain(), Nk=(262160, 1, 1))
     g = SBEContext(cfg)
