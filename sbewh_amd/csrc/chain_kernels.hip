@@ -12,8 +12,8 @@
 // stages, its error norm included, and an output time (current and fresh
 // derivative) is another.  Measured on 256 k, the general path first: an attempt
 // 49 us in two launches, now 11 us in one; an output time 24 us in six launches,
-// now 6 us; four right-hand sides 33.7 -> 14.9 us; a whole pulse with 1024 outputs
-// 149-162 -> 59-66 ms, half of it the host's round trips.  (With a lane per k-point
+// now 6 us; four right-hand sides 33.7 -> 14-17 us; a whole pulse with 1024 outputs
+// 144-164 -> 55-71 ms, half of it the host's round trips.  (With a lane per k-point
 // and its cells read through scalar loads an attempt takes 18 us.)
 #include <type_traits>
 
@@ -88,51 +88,119 @@ __device__ __forceinline__ void load_cells(const ChainArgs &c, const double *op,
     }
 }
 
-// e^{i 2 pi (frac + off)}, off of the vector potential A
-__device__ __forceinline__ cd phase_factor(const ChainArgs &c, double frac, double A)
+// (k + A) a_0 / 2 pi without k's own part: the phase offset of the vector potential A
+__device__ __forceinline__ double phase_offset(const ChainArgs &c, double A)
 {
-    const double off = ((c.kshift_au[0] + A) * c.a0[0] + c.kshift_au[1] * c.a0[1] + c.kshift_au[2] * c.a0[2]) / (2 * M_PI);
-    double s, co;
-    sincospi(2 * (frac + off), &s, &co);
-    return mk(co, s);
+    return ((c.kshift_au[0] + A) * c.a0[0] + c.kshift_au[1] * c.a0[1] + c.kshift_au[2] * c.a0[2]) / (2 * M_PI);
 }
 
-// sum_m z^m O_o(m), cells +m and -m sharing one power
-template <int MW, int NO>
-__device__ __forceinline__ void cell_sums(const ChainArgs &c, cd z, const Cells<MW> (&cell)[NO],
+// The powers z^m0 .. z^(m0 + 3) of a quad's phase factor z, for the highest m0 first and
+// then four lower at a time: each by its own argument, a lane one of them, rounded as the
+// twiddles of the general path are,
+struct DirectPowers {
+    double arg;
+    __device__ __forceinline__ void next(int m0, cd (&p)[4]) const
+    {
+        double s, co;
+        sincospi(2 * (arg * (double)(m0 + (int)(threadIdx.x & 3))), &s, &co);
+        const cd v = mk(co, s);
+        p[0] = quad_of<0>(v);
+        p[1] = quad_of<1>(v);
+        p[2] = quad_of<2>(v);
+        p[3] = quad_of<3>(v);
+    }
+    __device__ __forceinline__ void first(int m0, cd (&p)[4]) const { next(m0, p); }
+};
+// or, for an attempt's six stages, whose factors the lanes share out, as products
+// (z^-4 is z^4's conjugate).
+struct FactorPowers {
+    cd z, low[4];
+    __device__ __forceinline__ void first(int m0, cd (&p)[4])
+    {
+        low[0] = z;
+        low[1] = cmul(z, z);
+        low[2] = cmul(z, low[1]);
+        low[3] = cmul(low[1], low[1]);
+#pragma unroll
+        for (int j = 0; j < 4; j++) p[j] = low[j];
+        for (int m = 1; m < m0; m += 4)
+#pragma unroll
+            for (int j = 0; j < 4; j++) p[j] = cmul(p[j], low[3]);
+    }
+    __device__ __forceinline__ void next(int m0, cd (&p)[4]) const
+    {
+#pragma unroll
+        for (int j = 0; j < 4; j++) p[j] = m0 == 1 ? low[j] : cmul(p[j], cconj(low[3]));
+    }
+};
+// e^{i 2 pi (frac + off)}; what the sum's rounding loses (Knuth's two-sum) is put back to
+// first order, since the powers multiply it
+__device__ __forceinline__ cd phase_factor(const ChainArgs &c, double frac, double A)
+{
+    const double off = phase_offset(c, A), arg = frac + off, t = arg - frac;
+    const double lost = 2 * M_PI * ((frac - (arg - t)) + (off - t));
+    double s, co;
+    sincospi(2 * arg, &s, &co);
+    return mk(fma(-lost, s, co), fma(lost, co, s));
+}
+
+// sum_m z^m O_o(m), cells +m and -m sharing one power, from the far cells in: as a rule
+// the blocks decay, cell 0 by far the largest, and each sum rounds at its own size.  Right-
+// hand sides against long double, rms, the general path / cell 0 first / now: reach 4
+// 3.6e-16 / 3.3e-16 / 3.5e-16, reach 12 4.4e-16 / 4.8e-16 / 3.9e-16, reach 40 6.2e-16 /
+// 7.4e-16 / 4.5e-16.  In boxes read from memory four cells on each side are one trip:
+// four right-hand sides on 10000 k, reach 12, 31.7 -> 22.2 us, a propagation on 512 k,
+// reach 30, 4.87 -> 2.73 ms.
+template <int MW, int NO, class P>
+__device__ __forceinline__ void cell_sums(const ChainArgs &c, P pw, const Cells<MW> (&cell)[NO],
                                           const double *const (&op)[NO], int e, cd (&out)[NO])
 {
+    auto at = [&](int o, int r) {
+        const double2 t = reinterpret_cast<const double2 *>(op[o])[r * 4 + e];
+        return mk(t.x, t.y);
+    };
+    const int top = c.W - 1 + c.rmin, reach = MW > 0 ? MW : top > -c.rmin ? top : -c.rmin;
+    const int most = 1 + (reach - 1) / 4 * 4;
+    cd p[4];
+#pragma unroll
+    for (int o = 0; o < NO; o++) out[o] = mk(0, 0);
     if constexpr (MW > 0) {
+        pw.first(1, p);
 #pragma unroll
-        for (int o = 0; o < NO; o++) out[o] = cell[o].v[MW];
-        cd p[MW + 1];  // z^m by halves: fewer roundings and a shorter chain
-#pragma unroll
-        for (int m = 1; m <= MW; m++) {
-            p[m] = m == 1 ? z : cmul(p[m / 2], p[m - m / 2]);
+        for (int m = MW; m >= 1; m--)
 #pragma unroll
             for (int o = 0; o < NO; o++) {
-                out[o] = cfma(cell[o].v[MW + m], p[m], out[o]);
-                out[o] = cfma_jc(cell[o].v[MW - m], p[m], out[o]);
+                out[o] = cfma(cell[o].v[MW + m], p[m - 1], out[o]);
+                out[o] = cfma_jc(cell[o].v[MW - m], p[m - 1], out[o]);
             }
-        }
     } else {
-        auto at = [&](int o, int r) {
-            const double2 t = reinterpret_cast<const double2 *>(op[o])[r * 4 + e];
-            return mk(t.x, t.y);
-        };
+        for (int m0 = most; m0 >= 1; m0 -= 4) {
+            // a block's cells in one memory trip; outside the box cell 0, times 0
+            cd u[4][NO], d[4][NO];
 #pragma unroll
-        for (int o = 0; o < NO; o++) out[o] = at(o, -c.rmin);
-        const int top = c.W - 1 + c.rmin, mm = top > -c.rmin ? top : -c.rmin;
-        cd p = z;
-        for (int m = 1; m <= mm; m++) {
+            for (int j = 0; j < 4; j++)
 #pragma unroll
-            for (int o = 0; o < NO; o++) {
-                if (m <= top) out[o] = cfma(at(o, m - c.rmin), p, out[o]);
-                if (m <= -c.rmin) out[o] = cfma_jc(at(o, -m - c.rmin), p, out[o]);
+                for (int o = 0; o < NO; o++) {
+                    u[j][o] = at(o, (m0 + j <= top ? m0 + j : 0) - c.rmin);
+                    d[j][o] = at(o, (m0 + j <= -c.rmin ? -(m0 + j) : 0) - c.rmin);
+                }
+            if (m0 == most) pw.first(m0, p);
+            else pw.next(m0, p);
+#pragma unroll
+            for (int j = 3; j >= 0; j--) {
+                const cd pu = m0 + j <= top ? p[j] : mk(0, 0), pd = m0 + j <= -c.rmin ? p[j] : mk(0, 0);
+#pragma unroll
+                for (int o = 0; o < NO; o++) {
+                    out[o] = cfma(u[j][o], pu, out[o]);
+                    out[o] = cfma_jc(d[j][o], pd, out[o]);
+                }
             }
-            p = cmul(p, z);
         }
     }
+#pragma unroll
+    for (int o = 0; o < NO; o++)
+        if constexpr (MW > 0) out[o] = cadd(out[o], cell[o].v[MW]);
+        else out[o] = cadd(out[o], at(o, -c.rmin));
 }
 
 // entry of X Y - Y X: dX = X_00 - X_11 multiplies the off-diagonal of Y and the
@@ -222,7 +290,7 @@ __global__ __launch_bounds__(64) void chain_rhs_kernel(ChainArgs c, const double
     load_cells(c, c.Db, p.e, cell[1]);
     const cd rho = load_entry(x, p.at);
     cd o[2];
-    cell_sums(c, phase_factor(c, p.frac, x[0]), cell, op, p.e, o);
+    cell_sums(c, DirectPowers{p.frac + phase_offset(c, x[0])}, cell, op, p.e, o);
     store_entry(dxdt, p, c.P, chain_rate(c, p.e, o[0], o[1], E, rho), true);
 }
 
@@ -255,7 +323,7 @@ __global__ __launch_bounds__(64) void chain_output_kernel(ChainArgs c, const dou
     load_cells(c, c.dHb, p.e, cell[2]);
     const cd rho = load_entry(x, p.at);
     cd o[3];
-    cell_sums(c, phase_factor(c, p.frac, x[0]), cell, op, p.e, o);
+    cell_sums(c, DirectPowers{p.frac + phase_offset(c, x[0])}, cell, op, p.e, o);
     // -Im D_ab T_ba - Re dH_ab rho_ba, T = H0 rho - rho H0
     const cd T = quad<0, 2, 1, 3>(commutator(o[0], rho)), rt = quad<0, 2, 1, 3>(rho);
     double jk = -cmul(o[1], T).y - cmul(o[2], rt).x;
@@ -314,7 +382,7 @@ __global__ __launch_bounds__(64) void chain_attempt_kernel(ChainArgs c, ChainAtt
             in.y += s.c[q][j] * kd[kj].y;
         }
         cd o[2];
-        cell_sums(c, z[q], cell, op, e, o);
+        cell_sums(c, FactorPowers{z[q], {}}, cell, op, e, o);
         kd[q + 1] = chain_rate(c, e, o[0], o[1], s.E[q], in);
     }
     store_entry(s.xn, p, c.P, in, true);

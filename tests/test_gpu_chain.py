@@ -100,3 +100,38 @@ def test_chain_own_step_control_and_general_path(monkeypatch):
     for r, x in res[1:]:
         assert r["steps"] == res[0][0]["steps"] and r["rhs_calls"] == res[0][0]["rhs_calls"]
         assert np.abs(x - res[0][1]).max() < 1e-10
+
+
+@pytest.mark.parametrize("reach,nk,nf", [(2, 256, 16), (4, 256, 16), (12, 250, 25), (40, 243, 81)])
+def test_chain_rounding(reach, nk, nf, monkeypatch):
+    """right-hand sides are no further from long double than the general path's (5 % for
+    the spread of the mean over 16 states)"""
+    cfg = chain(reach, nk, nf, T2_fs=-1.0)
+    cfg.model.H[reach] += np.diag([-1.0, 1.0])
+    pi = np.longdouble("3.14159265358979323846264338327950288")
+    rms = []
+    for lr in ("1", None):
+        if lr:
+            monkeypatch.setenv("SBEWH_STAGE_LR", lr)
+        else:
+            monkeypatch.delenv("SBEWH_STAGE_LR")
+        g = SBEContext(cfg)
+        k = g.k_index_map()[:, 0].astype(np.longdouble) / nk
+        err = []
+        rng = np.random.default_rng(5)
+        for A in rng.uniform(-0.5, 0.5, 16):
+            x = np.zeros(g.state_size, complex)
+            x[0] = A
+            rho = cases.random_hermitian(rng, nk, 2, 0.3)
+            x[8:].reshape(nk, -1)[:, :4] = rho.reshape(nk, 4)
+            a = g.rho(g.rhs(x, 0.3))
+            arg = (k + np.longdouble(A) * np.longdouble(5.5) / (2 * pi))[:, None] * cfg.model.cells[:, 0]
+            arg = 2 * pi * (arg - np.round(arg))
+            op = (cfg.model.H + g.E(0.3)[0] * cfg.model.D[:, 0]).astype(np.clongdouble)
+            HE = np.einsum("kr,rab->kab", np.cos(arg) + 1j * np.sin(arg), op)
+            ref = -1j * (np.einsum("kab,kbc->kac", HE, rho) - np.einsum("kab,kbc->kac", rho, HE))
+            err.append(float(np.sqrt((np.abs(a - ref) ** 2).mean() / (np.abs(ref) ** 2).mean())))
+        rms.append(np.mean(err))
+        g.close()
+    print(f"[gpu] chain reach {reach}: general {rms[0]:.3e}, registers {rms[1]:.3e}", flush=True)
+    assert rms[1] <= 1.05 * rms[0]
