@@ -118,3 +118,33 @@ def test_resident_leaves_the_chain_path_alone():
         g.close()
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+# 64 k at four lanes per row; 6000 k, whose blocks at four lanes cannot all be resident, at one
+@pytest.mark.parametrize("n,nk", [(5, 64), (8, 64), (8, 6000)])
+def test_resident_5_to_8_bands(n, nk):
+    from sbewh_amd import model
+    from tests.test_gpu_stage_kernels import config
+    cfg = dataclasses.replace(config(n, (2, 0), (nk, 1), (5 if nk % 5 == 0 else 8, 1), sweeps=8, T2_fs=5.0, output_count=9), dim=1,
+                              Nk=(nk, 1, 1), Nf=(5 if nk % 5 == 0 else 8, 1, 1),
+                              pulses=model.elliptic_sin2(1.0, 0.0, 3000.0, 0.5))
+    say(f"[gpu] resident integrator: 1-D, {n} bands, {nk} k")
+    out = []
+    for device in (False, True):
+        g = SBEContext(dataclasses.replace(cfg, device_controller=device))
+        x = g.initial_state(0.0)
+        r = g.integrate(x, 9, log_capacity=0)
+        assert r["device_controller"] == device
+        out.append((r, x))
+        g.close()
+    (rh, xh), (rd, xd) = out
+    assert np.array_equal(rd["t"], rh["t"])
+    assert abs(rd["steps"] - rh["steps"]) <= 2
+    assert rel(rd["j"], rh["j"]) <= 1e-7
+    assert rel(xd, xh) <= 1e-7
+    if nk == 64:
+        o = Oracle(cfg)
+        xo = o.initial_state(0.0)
+        ro = o.integrate(xo, 9)
+        o.close()
+        assert rel(rd["j"], ro["j"]) <= 1e-7

@@ -105,6 +105,13 @@ def test_warm_start_steps(n, copies, monkeypatch):
     check_sequence(config(n, (2, 2), (6, 5), (6, 5), copies=copies), STEPS)
 
 
+@pytest.mark.parametrize("n", [13, 14, 15])
+def test_warm_start_steps_padded(n, monkeypatch):
+    """the same with the last bands of 16 as padding"""
+    monkeypatch.setenv("SBEWH_STAGE_LR", "4")
+    check_sequence(config(n, (2, 2), (6, 5), (6, 5)), STEPS)
+
+
 def test_warm_start_without_sweeps(monkeypatch):
     """no sweep allowed: a warm call keeps the previous eigenvectors in every layout"""
     cfg = config(16, (1, 1), (3, 4), (3, 4), sweeps=0)
