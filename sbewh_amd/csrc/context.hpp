@@ -140,8 +140,8 @@ struct sbe_ctx {
     // The layouts that refine a warm start by products (stage_device.hpp) are the
     // fastest on every grid timed once calls are warm: 8 bands at one / two / four
     // lanes per row 299 / 254 / 344 us per four right-hand sides on 150 x 150 k and
-    // 14.2 / 6.7 / 7.2 ms per propagation on 15 x 15 k (now 4.2 at two: small grids take
-    // a k-point per wavefront, stage_kernels.hip).  So only calls that
+    // 14.2 / 6.7 / 7.2 ms per propagation on 15 x 15 k (at two 1.6 times as fast again with
+    // a k-point per wavefront, which small grids take, stage_kernels.hip).  So only calls that
     // diagonalise from the identity each time, or not at all, or are bound to one
     // sweep, which is one of rotations, are timed: a new
     // state's first right-hand side then takes 0.35 instead of 1.9 ms on that

@@ -1446,7 +1446,8 @@ struct Frag8 {
 // place within the 16 lanes.  Four times the wavefronts of Frag8, each with a quarter
 // of the matrix instructions and of the arithmetic per entry: for grids that leave most
 // SIMDs idle, where the time is one wavefront's.  An attempt of six stages on 15 x 15 k:
-// 92.5 -> 48.7 us, a propagation of 56 attempts there 6.8 -> 4.2 ms.
+// 92.5 -> 48.7 us, a propagation there 7.1 -> 4.5 ms (other grids: ONE_K_MOST in
+// stage_kernels.hip).
 struct Acc1 {
     double r[1], i[1];
 };

@@ -126,8 +126,8 @@ int stage_variants(int N, int *lr_out, int cap)
 // Grids of 5 to 8 bands with a SIMD of its own for each k-point (256 CUs of four): a
 // k-point per wavefront (FragOne).  Above, four per wavefront (Frag8) run a
 // grid of up to 4096 k-points in one round, where the others take a second one.  Measured on a
-// propagation of 56 attempts, four per wavefront against one, by k-points: 225
-// 6.9 -> 4.6 ms, 900 8.3 -> 6.5 ms, 1296 8.4 -> 9.2 ms, 2025 9.5 -> 11.7 ms.
+// propagation of some 60 attempts, four per wavefront -> one, by k-points: 225
+// 7.1 -> 4.5 ms, 900 8.3 -> 6.4 ms, 1296 8.3 -> 9.4 ms, 2025 9.0 -> 11.0 ms.
 constexpr long ONE_K_MOST = 1024;
 
 // 16 bands at four lanes per row: a launch of decompositions that rotations make alone
